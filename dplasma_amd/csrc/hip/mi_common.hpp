@@ -100,7 +100,6 @@ enum WsId {
     WS_ADJ_SEGS,        //   segment table
     WS_POTRI,           // inverse: the seed / result image
     WS_DTD,             // task-insertion front-end: per-task diagonal-block inverses
-    WS_POTRF_REC,       // recursive diagonal factor: packed image of one tile's sub-tiles
     WS_BF16_PANEL,      // BF16-split FP32 factor: hi/lo images of one panel column
     WS_COUNT
 };
@@ -181,7 +180,7 @@ void noalloc_setup(int device);
 // reads; update: A(m, n) -= A(m, k) A(n, k)^T, SYRK when m == n.
 int task_prepare_fp64(int NB);
 int task_potrf_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int k, double *Winv);
-int task_trsm_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int k, const double *Winv);
+int task_trsm_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int k, double *Winv);
 int task_update_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int n, int k);
 size_t task_winv_elems(int NB);
 // R = B - A X for the symmetric A in lower tiles, FP64, enqueued on s

@@ -157,7 +157,7 @@ int mi_dtd_potrf(mi_dtd_t *d, int k)
 int mi_dtd_trsm(mi_dtd_t *d, int m, int k)
 {
     if (k < 0 || m <= k || m >= d->MT) return bad("TRSM tiles out of range");
-    const double *w = d->winv + (size_t)k * d->wsz;
+    double *w = d->winv + (size_t)k * d->wsz;
     return run_task(d, next_stream(d), {tile_id(d, k, k), winv_id(d, k)}, {tile_id(d, m, k)},
                     [&](hipStream_t s) { return task_trsm_fp64(d->c, s, d->dT, d->N, d->NB, m, k, w); });
 }

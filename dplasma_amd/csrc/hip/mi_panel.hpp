@@ -1,0 +1,442 @@
+// mi_panel.hpp -- the panel of the tile Cholesky (POTRF(k) and TRSM(m,k) of
+// src/zpotrf_L.jdf:91-343), factored in sub-columns of SB columns:
+//   k_diag_factor   one workgroup: the w x w diagonal block of sub-column j
+//   k_panel_solve   X = C L_jj^{-T} for every row below it, 16 rows a wave
+//   k_panel_update  the remaining columns of the tile column -= X X_k^T
+// (mi_potrf.hip launches them).  Everything works on 16 x 16 blocks held in
+// the accumulator layout of the 16x16x4 MFMA fed (B, A): element q of lane
+// l = 16 fk + fr is C(row fr, column row(q, fk)).  The same registers are,
+// element s for K slice s, the B operand of a product that contracts over
+// those columns (slice s then holds columns row(s, fk)), and likewise the A
+// operand X(fr, row(s, fk)); so a block passes from one product to the next
+// without leaving the registers, and blocks that other waves need travel as
+// [s][lane] images of 64 consecutive elements (no bank conflicts, whole
+// lines).
+#pragma once
+#include <utility>
+#include "mi_common.hpp"
+
+namespace mi {
+
+constexpr int SB = 128;               // columns of a sub-column
+constexpr int DB = 16;                // block side
+constexpr int DBN = SB / DB;          // blocks a side, at most
+// Operand images that k_diag_factor leaves for k_panel_solve, per 16-column
+// block b of a tile: W_b = L_bb^{-1}, then -L(b + i, b), i = 1 .. (blocks
+// left in its sub-column): DBN images of 256 elements, [lane][s] (16-byte
+// pieces per lane).
+constexpr int OPI = DB * DB;
+constexpr int OPB = DBN * OPI;
+
+// ------------------------------------------------------- cross-lane helpers
+// value of lane C of each row of 16 lanes
+template <int C> __device__ __forceinline__ double row_bcast(double v)
+{
+    return __longlong_as_double(
+        __builtin_amdgcn_update_dpp((long long)0, __double_as_longlong(v), 0x150 + C, 0xf, 0xf, true));
+}
+template <int C> __device__ __forceinline__ float row_bcast(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + C, 0xf, 0xf, true));
+}
+
+// a[C + i] -= row_bcast<C + i>(m) * f, i < K (K <= 8): one DPP FMA each (the
+// compiler does not fold a broadcast into the FP64 FMA).  The two wait
+// states that a DPP read needs after m was written are inside the block.
+#define MI_F(op, i) "v_fmac_" op "_dpp %[a" #i "], -%[m], %[f] row_newbcast:%[c" #i "] row_mask:0xf bank_mask:0xf\n\t"
+#define MI_A(i) [a##i] "+&v"(a[C + i])
+#define MI_C(i) [c##i] "n"(C + i)
+#define MI_FMAC(op, n)                                                        \
+    if constexpr (K == n)                                                     \
+    asm("s_nop 1\n\t" MI_F##n(op) : MI_A##n : [m] "v"(m), [f] "v"(f), MI_C##n)
+#define MI_F1(op) MI_F(op, 0)
+#define MI_F2(op) MI_F1(op) MI_F(op, 1)
+#define MI_F3(op) MI_F2(op) MI_F(op, 2)
+#define MI_F4(op) MI_F3(op) MI_F(op, 3)
+#define MI_F5(op) MI_F4(op) MI_F(op, 4)
+#define MI_F6(op) MI_F5(op) MI_F(op, 5)
+#define MI_F7(op) MI_F6(op) MI_F(op, 6)
+#define MI_F8(op) MI_F7(op) MI_F(op, 7)
+#define MI_A1 MI_A(0)
+#define MI_A2 MI_A1, MI_A(1)
+#define MI_A3 MI_A2, MI_A(2)
+#define MI_A4 MI_A3, MI_A(3)
+#define MI_A5 MI_A4, MI_A(4)
+#define MI_A6 MI_A5, MI_A(5)
+#define MI_A7 MI_A6, MI_A(6)
+#define MI_A8 MI_A7, MI_A(7)
+#define MI_C1 MI_C(0)
+#define MI_C2 MI_C1, MI_C(1)
+#define MI_C3 MI_C2, MI_C(2)
+#define MI_C4 MI_C3, MI_C(3)
+#define MI_C5 MI_C4, MI_C(4)
+#define MI_C6 MI_C5, MI_C(5)
+#define MI_C7 MI_C6, MI_C(6)
+#define MI_C8 MI_C7, MI_C(7)
+template <int C, int K> __device__ __forceinline__ void fmac_bcast(double *a, double m, double f)
+{
+    MI_FMAC("f64", 1); MI_FMAC("f64", 2); MI_FMAC("f64", 3); MI_FMAC("f64", 4);
+    MI_FMAC("f64", 5); MI_FMAC("f64", 6); MI_FMAC("f64", 7); MI_FMAC("f64", 8);
+}
+template <int C, int K> __device__ __forceinline__ void fmac_bcast(float *a, float m, float f)
+{
+    MI_FMAC("f32", 1); MI_FMAC("f32", 2); MI_FMAC("f32", 3); MI_FMAC("f32", 4);
+    MI_FMAC("f32", 5); MI_FMAC("f32", 6); MI_FMAC("f32", 7); MI_FMAC("f32", 8);
+}
+#undef MI_FMAC
+
+// a[c] -= row_bcast<c>(m) * f for C <= c < 16
+template <int C, class T> __device__ __forceinline__ void fmac_rest(T *a, T m, T f)
+{
+    if constexpr (C < DB) {
+        constexpr int K = DB - C < 8 ? DB - C : 8;
+        fmac_bcast<C, K>(a, m, f);
+        fmac_rest<C + K>(a, m, f);
+    }
+}
+
+// 1 / sqrt(x); NaN for x <= 0, NaN and infinity (and in FP32 for denormals,
+// which v_rsq_f32 takes for zero)
+__device__ __forceinline__ double rsq_refined(double x)
+{
+    // v_rsq_f64 is good to about 2^-26; one third-order step leaves rounding
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+__device__ __forceinline__ float rsq_refined(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float e = fmaf(-(x * y), y, 1.0f);
+    return fmaf(y * e, 0.5f, y);
+}
+
+// One column of the sweep over a 16 x 16 block, four copies of it side by
+// side in the rows of 16 lanes: lane fr holds row fr of D in v[] and row fr
+// of the identity in x[].  Column C: v[C] becomes L(fr, C), x[C] becomes
+// W(C, fr) (W = L^{-1}); both arrays lose the multiple of the column.
+// Entries above the diagonal hold arbitrary values throughout and never
+// reach another lane.  A lone wave issues one instruction every four
+// cycles, so the column costs its instruction count: the two FMA per later
+// column, and the pivot's chain.  Returns 1 / L(C, C).
+template <int C, class T> __device__ __forceinline__ T sweep_column(T *v, T *x)
+{
+    const T rd = rsq_refined(row_bcast<C>(v[C]));
+    const T m = v[C] * rd;
+    if constexpr (C + 1 < DB) fmac_bcast<C + 1, 1>(v, m, m);    // the next pivot first
+    x[C] = x[C] * rd;
+    fmac_rest<C + 2>(v, m, m);
+    fmac_rest<C + 1>(x, m, x[C]);
+    v[C] = m;
+    return rd;
+}
+// True when a pivot was not an ordinary positive number: its NaN reciprocal
+// root reaches every later column.
+template <class T, int... C>
+__device__ __forceinline__ bool sweep_fast(T *v, T *x, std::integer_sequence<int, C...>)
+{
+    T rd = T(0);
+    ((rd = sweep_column<C>(v, x)), ...);
+    return rd != rd;
+}
+
+// The same sweep with square root and division, for blocks with a pivot that
+// is not positive, infinite, NaN or denormal; the first non-positive (or
+// NaN) pivot's column goes to *fail (0: none) and counts as 1 from there on.
+template <int C, class T> __device__ __forceinline__ void sweep_column_exact(T *v, T *x, int fr, int *fail)
+{
+    T d0 = row_bcast<C>(v[C]);
+    const bool ok = d0 > T(0);
+    if (!ok && !*fail) *fail = C + 1;
+    d0 = ok ? d0 : T(1);
+    const T d = sqrt(d0), rd = T(1) / d;
+    const T m = v[C] * rd;
+    x[C] = x[C] * rd;
+    fmac_rest<C + 1>(v, m, m);
+    fmac_rest<C + 1>(x, m, x[C]);
+    v[C] = fr == C ? d : m;
+}
+template <class T, int... C>
+__device__ __forceinline__ void sweep_exact(T *v, T *x, int fr, int *fail, std::integer_sequence<int, C...>)
+{
+    (sweep_column_exact<C>(v, x, fr, fail), ...);
+}
+
+// ---------------------------------------------------------------------------
+// Cholesky factor of the n x n (n <= 128) diagonal block A (column-major,
+// ld), lower, in place: right-looking over 16-column blocks.  Eight waves;
+// the 16 x 16 blocks below the first diagonal block live in the registers of
+// waves 1..7 (dealt out column by column) from load to store.
+//   wave 0     factors D_p (sweep above), publishes W_p, forms X(p+1, p) =
+//              C W_p^T and the next diagonal block D_{p+1} -= X X^T itself,
+//   waves 1-7  meanwhile apply step p - 1 to their blocks, hand C(p+1, p)
+//              and D_{p+1} to wave 0 through LDS, and after W_p is there form
+//              the rest of block column p.
+// Two barriers a step.  Every block is updated in step order whatever the
+// timing.  Wave 7 stores what wave 0 leaves in LDS.  Bound by wave 0's chain: 16 dependent pivots (reciprocal square
+// root with one correction step, then a DPP FMA into the next pivot), then
+// eight MFMAs and the hand-offs.
+// op: the operand images for k_panel_solve (see OPB); info = info_base + j of
+// the first non-positive pivot j (1-based), as CORE_dpotrf reports it.
+//
+// Measured (n = 128): 20 us in FP64, 21 us in FP32 inside a factorization, of
+// which 2.5 us load the blocks; per 16 columns 3100-3900 cycles of sweep and
+// 1400 cycles of hand-off.  A whole-tile factor of 32-column blocks with
+// v_readlane broadcasts, W_jj on the chain and the tile in memory took 145 us
+// for 256 columns and 367 us (FP32) for 512.
+template <class T>
+__global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n, int ld, int info_base,
+                                                       int *__restrict__ d_info, T *__restrict__ op)
+{
+    typedef typename MF<T>::v4 V4;
+    constexpr int NW = 7;                                   // worker waves
+    constexpr int NBLK = DBN * (DBN + 1) / 2 - 1;           // blocks besides (0, 0)
+    constexpr int SLOTS = (NBLK + NW - 1) / NW;
+    __shared__ T Xl[DBN][OPI];                              // X(i, p) of the current step
+    constexpr int WP = DB + 2;                              // pitch of Wl: distinct banks for its writer
+    // W_p, image column t (64 s + 16 fk = 16 t) at t WP; two steps' worth, as
+    // is L_pp ([column][row]): a worker still stores the last step's
+    __shared__ __align__(16) T Wl[2][DB * WP];
+    __shared__ __align__(16) T Ll[2][DB][DB + 2];
+    __shared__ T Hc[OPI], Hd[OPI];                          // C(p+1, p) and D_{p+1} for wave 0
+    __shared__ __align__(16) T Dl[DB][DB + 2];              // D, [row][column]
+    __shared__ int s_fail;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4;
+    const int nb = (n + DB - 1) / DB;
+    if (tid == 0) s_fail = 0;
+
+    // element (r, c) of A; past n the identity, so that a ragged block
+    // factors like a whole one
+    auto elem = [&](int r, int c) -> T {
+        const T a = A[(int64_t)min(c, n - 1) * ld + min(r, n - 1)];
+        return r < n && c < n ? a : (r == c ? T(1) : T(0));
+    };
+    auto store = [&](int i, int j, const V4 &b) {           // block (i, j), below the diagonal
+        const int r = DB * i + fr;
+        if (r < n) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) A[(int64_t)(DB * j + MF<T>::row(q, fk)) * ld + r] = b[q];
+        }
+    };
+    auto put = [&](T *img, const V4 &b) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) img[64 * q + lane] = b[q];
+    };
+    auto put_op = [&](T *img, const V4 &b) { *(V4 *)(img + 4 * lane) = b; };
+    auto get = [&](const T *img) -> V4 {
+        V4 b;
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[q] = img[64 * q + lane];
+        return b;
+    };
+    auto get_w = [&](int p) -> V4 {
+        V4 b;
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[q] = Wl[p & 1][(4 * q + fk) * WP + fr];
+        return b;
+    };
+    // C - X_i X_j^T, both as [s][lane] images
+    auto prod = [&](V4 c, const V4 &xj, const V4 &xi) -> V4 {
+#pragma unroll
+        for (int s = 0; s < 4; s++) c = MF<T>::mfma(-xj[s], xi[s], c);
+        return c;
+    };
+    auto solve = [&](const V4 &w, const V4 &c) -> V4 {       // C W^T
+        V4 xx = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int s = 0; s < 4; s++) xx = MF<T>::mfma(w[s], c[s], xx);
+        return xx;
+    };
+
+    // Both roles run the same barriers: one before the loop's second half
+    // (W_p, C(p+1, p) and D_{p+1} are in LDS) and one after it (X(., p) is).
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);                      // it shares its SIMD with wave 4
+        T v[DB], x[DB];
+#pragma unroll
+        for (int c = 0; c < DB; c++) {
+            v[c] = elem(fr, c);
+            if (fk == 0) Dl[fr][c] = v[c];
+        }
+        for (int p = 0; p < nb; p++) {
+#pragma unroll
+            for (int c = 0; c < DB; c++) x[c] = fr == c ? T(1) : T(0);
+            if (__any(sweep_fast(v, x, std::make_integer_sequence<int, DB>()))) {
+                int fail = 0;
+#pragma unroll
+                for (int c = 0; c < DB; c++) {
+                    v[c] = Dl[fr][c];
+                    x[c] = fr == c ? T(1) : T(0);
+                }
+                sweep_exact(v, x, fr, &fail, std::make_integer_sequence<int, DB>());
+                if (fail && lane == 0) s_fail = DB * p + fail;
+            }
+            // W(c, fr) = x[c] as the A operand of W C^T: slice s, lane 16 fk +
+            // i holds W(i, row(s, fk)), so column fr is image column t
+            if (fk == 0) {
+                const int t = sizeof(T) == 8 ? fr : 4 * (fr & 3) + (fr >> 2);
+#pragma unroll
+                for (int c = 0; c < DB; c++) Wl[p & 1][t * WP + c] = x[c];
+            } else if (fk == 1) {
+#pragma unroll
+                for (int c = 0; c < DB; c++) Ll[p & 1][c][fr] = v[c];
+            }
+            __syncthreads();
+            if (s_fail) break;
+            if (p + 1 < nb) {
+                const V4 d0 = get(Hd);
+                const V4 xx = solve(get_w(p), get(Hc));
+                put(Xl[p + 1], xx);
+                const V4 d = prod(d0, xx, xx);
+#pragma unroll
+                for (int q = 0; q < 4; q++) Dl[fr][MF<T>::row(q, fk)] = d[q];
+            }
+            __syncthreads();
+            if (p + 1 < nb) {
+#pragma unroll
+                for (int c = 0; c < DB; c++) v[c] = Dl[fr][c];
+            }
+        }
+    } else {
+        // slot u: block t = wave + 7 u of the list (0,0) (1,0) .. (7,0) (1,1)
+        // (2,1) .. ; bi, bj are wave-uniform, bj = -1 where there is none
+        V4 blk[SLOTS];
+        int bi[SLOTS], bj[SLOTS];
+#pragma unroll
+        for (int u = 0; u < SLOTS; u++) {
+            int t = wave + NW * u, j = 0;
+            while (j < DBN && t >= DBN - j) { t -= DBN - j; j++; }
+            bj[u] = j < DBN && j + t < nb ? j : -1;
+            bi[u] = j + t;
+            if (bj[u] >= 0) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) blk[u][q] = elem(DB * bi[u] + fr, DB * j + MF<T>::row(q, fk));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SLOTS; u++)
+            if (bj[u] >= 0 && bi[u] == 1) put(bj[u] == 0 ? Hc : Hd, blk[u]);
+        for (int p = 0; p < nb; p++) {
+            if (p > 0) {
+                // step p - 1 on the blocks of columns >= p (wave 0 did (p, p));
+                // the two blocks that wave 0 needs next go to LDS
+#pragma unroll
+                for (int u = 0; u < SLOTS; u++)
+                    if (bj[u] >= p && bi[u] > p) {
+                        blk[u] = prod(blk[u], get(Xl[bj[u]]), get(Xl[bi[u]]));
+                        if (bi[u] == p + 1) put(bj[u] == p ? Hc : Hd, blk[u]);
+                    }
+            }
+            __syncthreads();
+            if (s_fail) break;
+            const V4 w = get_w(p);
+            T *opp = op + (int64_t)p * OPB;
+#pragma unroll
+            for (int u = 0; u < SLOTS; u++)
+                if (bj[u] == p && bi[u] > p + 1) {
+                    blk[u] = solve(w, blk[u]);
+                    put(Xl[bi[u]], blk[u]);
+                }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < SLOTS; u++)
+                if (bj[u] == p && bi[u] > p + 1) {
+                    store(bi[u], p, blk[u]);
+                    put_op(opp + (bi[u] - p) * OPI, -blk[u]);
+                }
+            // what wave 0 left: L_pp, W_p and X(p + 1, p)
+            if (wave == NW) {
+                put_op(opp, w);
+                if (p + 1 < nb) {
+                    const V4 xx = get(Xl[p + 1]);
+                    store(p + 1, p, xx);
+                    put_op(opp + OPI, -xx);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int c = 4 * u + fk;
+                    if (c <= fr && DB * p + fr < n) A[(int64_t)(DB * p + c) * ld + DB * p + fr] = Ll[p & 1][c][fr];
+                }
+            }
+        }
+    }
+    if (tid == 0 && s_fail) atomicCAS(d_info, 0, info_base + s_fail);
+}
+
+// ---------------------------------------------------------------------------
+// X = C L^{-T} for the rows below the diagonal block of a sub-column: columns
+// c0 .. c0 + w - 1 of tile column k, rows c0 + w.. of tile (k, k) (the first
+// g0 workgroups) and all rows of the tiles m0, m0 + 1, ... (gt workgroups a
+// tile).  A wave takes 16 rows with all w columns in registers (nbw =
+// ceil(w / 16) blocks): per 16-column block one product with W_b, then the
+// update of the later blocks; nothing passes between waves.  The operand
+// images of block column b + 1 are in flight while block column b is
+// multiplied; the four waves of a workgroup read the same images at about
+// the same time.  144 MFMAs a wave at w = 128; blocks past nbw multiply what
+// the unused images hold and are dropped.
+//
+// Bound by the latency of the first loads and of eight dependent products
+// (FP64, 13 us at 1000 rows; its 144 MFMAs of 64 cycles are 3.8 us).
+// Staging the images in LDS instead took 16-18 us a launch.
+template <class T>
+__global__ __launch_bounds__(256, 2) void k_panel_solve(T *__restrict__ Tt, int N, int NB, int MT, int k, int c0,
+                                                       int w, const T *__restrict__ op, int g0, int gt, int m0)
+{
+    typedef typename MF<T>::v4 V4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int fr = lane & 15, fk = lane >> 4;
+    const int g = blockIdx.x;
+    const int m = g < g0 ? k : m0 + (g - g0) / gt;
+    const int r0 = (g < g0 ? c0 + w + 64 * g : 64 * ((g - g0) % gt)) + 16 * wave;
+    const int rows = tile_rows(N, NB, MT, m);
+    if (r0 >= rows) return;
+    T *C = Tt + tile_index(MT, m, k) * (int64_t)NB * NB + (int64_t)c0 * NB;
+    const int nbw = (w + DB - 1) / DB;
+
+    V4 img[2][DBN];
+    auto load = [&](V4 *im, int b) {
+        const V4 *src = (const V4 *)(op + (int64_t)b * OPB) + lane;
+#pragma unroll
+        for (int i = 0; i < DBN; i++)
+            if (b + i < DBN) im[i] = src[64 * i];
+    };
+    load(img[0], 0);
+    const int r = r0 + fr, rc = min(r, rows - 1);
+    V4 acc[DBN];
+#pragma unroll
+    for (int b = 0; b < DBN; b++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int c = DB * b + MF<T>::row(q, fk);
+            const T a = C[(int64_t)min(c, w - 1) * NB + rc];
+            acc[b][q] = c < w ? a : T(0);
+        }
+#pragma unroll
+    for (int b = 0; b < DBN; b++) {
+        if (b < nbw) {
+            __builtin_amdgcn_sched_barrier(0);              // no image further ahead than this
+            if (b + 1 < nbw) load(img[(b + 1) & 1], b + 1);
+            const V4 *im = img[b & 1];
+            V4 xx = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int s = 0; s < 4; s++) xx = MF<T>::mfma(im[0][s], acc[b][s], xx);
+            acc[b] = xx;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int b2 = b + 1; b2 < DBN; b2++)
+                    acc[b2] = MF<T>::mfma(im[b2 - b][s], xx[s], acc[b2]);
+            if (r < rows) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = DB * b + MF<T>::row(q, fk);
+                    if (c < w) C[(int64_t)c * NB + r] = xx[q];
+                }
+            }
+        }
+    }
+}
+
+}  // namespace mi

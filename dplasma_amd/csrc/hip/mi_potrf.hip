@@ -1,28 +1,15 @@
 // mi_potrf.hip -- tile Cholesky (lower) on gfx950, tiles resident in HBM.
 //
-// The four task classes of src/zpotrf_L.jdf become three kernels launched
-// per step k:
-//   k_potrf_diag   POTRF(k)        :91-208   one workgroup factors the
-//                                            diagonal tile with a 32-wide
-//                                            right-looking blocking, the
-//                                            current panel held in LDS; it also
-//                                            writes the inverses of the 32x32
-//                                            diagonal blocks for the panel solve
-//                                            and records info = k*NB + j.
-//   k_trsm_panel   TRSM(m,k), m>k  :214-343  C <- C L_kk^{-T}; one workgroup per
-//                                            64-row strip of a panel tile,
-//                                            blocked by 32 columns, diagonal
-//                                            blocks applied through their
-//                                            inverses.
-//   k_update_mfma  SYRK(k,m) and   :349-633  C(m,n) -= A(m,k) A(n,k)^T for every
-//                  GEMM(m,n,k)               trailing tile in a column range, on
-//                                            v_mfma_f64_16x16x4_f64 with
-//                                            double-buffered LDS staging; SYRK
-//                                            is the m == n case restricted to
-//                                            the lower triangle.
-// The host loop runs the panel (POTRF+TRSM of step k+1) on a second stream
-// as soon as column k+1 has received its step-k update, so it overlaps the
-// rest of the step-k trailing update (one-panel look-ahead).
+// The four task classes of src/zpotrf_L.jdf become, per step k:
+//   the panel (mi_panel.hpp)  POTRF(k)       :91-208   and TRSM(m,k), m > k
+//                             :214-343: tile column k, 128 columns at a time
+//   k_update_*                SYRK(k,m) and   :349-633  C(m,n) -= A(m,k) A(n,k)^T
+//                             GEMM(m,n,k)               for every trailing tile
+//                             in a column range; SYRK is the m == n case
+//                             restricted to the lower triangle.
+// The host loop runs the panel of step k+1 on a second stream as soon as
+// column k+1 has received its step-k update, so it overlaps the rest of the
+// step-k trailing update (look-ahead).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -30,6 +17,7 @@
 #include <mutex>
 #include <type_traits>
 #include "mi_common.hpp"
+#include "mi_panel.hpp"
 #include "dplasma_mi.h"
 
 using namespace mi;
@@ -38,428 +26,6 @@ namespace {
 
 constexpr int PJB = 32;            // panel width inside the diagonal factorization
 constexpr int POTRF_THREADS = 512;
-
-// v = *p, kept where c holds and +0 elsewhere; p must be a valid address
-// whatever c is.  The load is unconditional, so that the compiler issues a
-// group of them together instead of branching around each and waiting for
-// it on its own.
-template <class T> __device__ __forceinline__ T load_if(const T *p, bool c)
-{
-    const T v = *p;
-    return c ? v : T(0);
-}
-
-// ---------------------------------------------------------------------------
-// One wave: acc[ct] += X[r0+i][0:K] * Y[c0+16ct+j][0:K]^T for the 16x16 output
-// tiles ct = 0, 1 (i, j < 16) on v_mfma_f64_16x16x4_f64, operands read straight
-// from column-major global memory (element (r, k) at X[k*ldx + r]); rows at or
-// beyond xr_lim / yr_lim read as zero.  K is a multiple of 32.  Operand lane
-// layout: A(i, k) and B(k, j) sit in lane 16k + i (resp. 16k + j); result
-// element q of lane l is D(4q + l/16, l%16).
-template <class T>
-__device__ inline void mfma_panel_2(const T *__restrict__ X, int ldx, int r0, int xr_lim,
-                                    const T *__restrict__ Y, int ldy, int c0, int yr_lim, int K,
-                                    typename MF<T>::v4 acc[2])
-{
-    typedef typename MF<T>::v4 V4;
-    const int lane = threadIdx.x & 63, fr = lane & 15, fk = lane >> 4;
-    const int xr = r0 + fr, y0 = c0 + fr, y1 = c0 + 16 + fr;
-    const bool xv = xr < xr_lim, yv0 = y0 < yr_lim, yv1 = y1 < yr_lim;
-    // rows past the limits read the last valid row (xr_lim, yr_lim >= 1)
-    const int xrc = min(xr, xr_lim - 1), y0c = min(y0, yr_lim - 1), y1c = min(y1, yr_lim - 1);
-    V4 e0 = {0, 0, 0, 0}, e1 = e0, o0 = e0, o1 = e0;
-    // 32 columns of K per pass, all 24 loads of a pass issued together; in
-    // FP32 the operands of pass p+1 are in flight while the 16 MFMAs of pass
-    // p run
-    T a[8], b0[8], b1[8];
-    auto load = [&](int k, T *pa, T *pb0, T *pb1) {
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            const int64_t kk = k + 4 * s + fk;
-            pa[s] = load_if(&X[kk * ldx + xrc], xv);
-            pb0[s] = load_if(&Y[kk * ldy + y0c], yv0);
-            pb1[s] = load_if(&Y[kk * ldy + y1c], yv1);
-        }
-    };
-    auto mul = [&]() {
-#pragma unroll
-        for (int s = 0; s < 8; s += 2) {
-            e0 = MF<T>::mfma(a[s], b0[s], e0);
-            e1 = MF<T>::mfma(a[s], b1[s], e1);
-            o0 = MF<T>::mfma(a[s + 1], b0[s + 1], o0);
-            o1 = MF<T>::mfma(a[s + 1], b1[s + 1], o1);
-        }
-    };
-    if constexpr (sizeof(T) == 8) {
-        // FP64: one chunk of 24 loads in flight (two would spill 45
-        // registers in k_trsm_tile)
-        for (int k = 0; k < K; k += 32) {
-            load(k, a, b0, b1);
-            mul();
-        }
-    } else {
-        if (K > 0) load(0, a, b0, b1);
-        for (int k = 0; k < K; k += 32) {
-            T na[8], nb0[8], nb1[8];
-            const bool more = k + 32 < K;
-            if (more) load(k + 32, na, nb0, nb1);
-            mul();
-            if (more) {
-#pragma unroll
-                for (int s = 0; s < 8; s++) { a[s] = na[s]; b0[s] = nb0[s]; b1[s] = nb1[s]; }
-            }
-        }
-    }
-    acc[0] += e0 + o0;
-    acc[1] += e1 + o1;
-}
-
-
-// C(r0:r0+32, c0:c0+32) -= X(r0:, 0:32) X(c0:, 0:32)^T on the lower triangle
-// of A (rows, columns < n), X held in LDS as P[k * RC + row]; one wave, 2 x 2
-// MFMA 16x16 tiles sharing their operands, K = 32.  The MFMA is fed (X_c, X_r)
-// so that it accumulates C^T: lane l then holds rows r0 + 16i + l % 16 of C,
-// and the loads and stores of the column-major C are 128-byte runs.
-template <class T>
-__device__ inline void syrk_unit32(T *__restrict__ A, int ld, int n, const T *__restrict__ P, int RC, int r0,
-                                   int c0, int fr, int fk, T *__restrict__ dsm = nullptr)
-{
-    typedef typename MF<T>::v4 V4;
-    V4 acc[2][2];                                    // acc[i][j]: rows r0+16i.., columns c0+16j..
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int r = r0 + 16 * i + fr, c = c0 + 16 * j + MF<T>::row(q, fk);
-                acc[i][j][q] = load_if(&A[(int64_t)min(c, n - 1) * ld + min(r, n - 1)], r < n && c < n && r >= c);
-            }
-    const int ra0 = min(r0 + fr, RC - 1), ra1 = min(r0 + 16 + fr, RC - 1);
-    const int cb0 = min(c0 + fr, RC - 1), cb1 = min(c0 + 16 + fr, RC - 1);
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int kk = (4 * s + fk) * RC;
-        const T x0 = -P[kk + ra0], x1 = -P[kk + ra1];
-        const T y0 = P[kk + cb0], y1 = P[kk + cb1];
-        acc[0][0] = MF<T>::mfma(y0, x0, acc[0][0]);
-        acc[0][1] = MF<T>::mfma(y1, x0, acc[0][1]);
-        acc[1][0] = MF<T>::mfma(y0, x1, acc[1][0]);
-        acc[1][1] = MF<T>::mfma(y1, x1, acc[1][1]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int r = r0 + 16 * i + fr, c = c0 + 16 * j + MF<T>::row(q, fk);
-                if (r < n && c < n && r >= c) A[(int64_t)c * ld + r] = acc[i][j][q];
-                // the unit also to LDS, column-major with stride 33 (its lower
-                // part is what the diagonal factor reads)
-                if (dsm) dsm[(c - c0) * 33 + (r - r0)] = acc[i][j][q];
-            }
-}
-
-// POTRF(k): right-looking by 32-column blocks in one workgroup of 8 waves,
-// with look-ahead inside the tile.  LDS holds the current block column X
-// (rows j0..n-1, 32 columns) as P[c * RC + row] (absolute rows), W_jj, and
-// the next diagonal block as its update left it (wave 0 updates that block
-// itself and reads it back from LDS rather than from the tile).
-// Per block j0:
-//   wave 0     L_jj = chol(D), W_jj = L_jj^{-1} in one register sweep over the
-//              32 columns (lanes 0..31: rows of L, lanes 32..63: columns of
-//              W, both by the FMA v[c2] -= m * L(c2, c) with L(c2, c)
-//              broadcast by v_readlane); columns past the tile edge get an
-//              identity diagonal
-//   waves 1-7  meanwhile: the trailing update of the previous block for
-//              columns >= j0 + 32 (A -= X X^T, 32x32 MFMA units from LDS)
-//   all        X = A(j0+32:n, j0:j0+32) W_jj^T on MFMA -> P and A;
-//              the next block column (j0+32 .. j0+63) updated first,
-//   wave 0     then loads the next diagonal block D while waves 1-7 go on
-//              with the rest of the trailing update.
-// Every element is updated in the same order as the right-looking loop, so
-// results do not depend on timing.  W_jj goes to Winv for the panel TRSM.
-// info = k*NB + j of the first non-positive pivot j (1-based), as
-// CORE_dpotrf reports it (src/zpotrf_L.jdf:200-202).
-template <class T>
-__device__ inline void potrf_tile_dev(T *__restrict__ A, int n, int ld, int RC, int info_base,
-                                      int *__restrict__ d_info, T *__restrict__ Winv)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    typedef typename MF<T>::v4 V4;
-    T *P = reinterpret_cast<T *>(smem_raw);          // 32 columns x RC rows (RC odd, >= n + 1)
-    T *Ws = P + 32 * RC;                             // W(i, j) at Ws[j*32 + i]
-    T *Dsm = Ws + 1024;                              // next diagonal block, column-major, stride 33
-    __shared__ int s_fail;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fk = lane >> 4;
-    const bool lrow = lane < 32;
-    if (tid == 0) s_fail = 0;
-
-    // v[c]: lanes < 32 hold D(lane, c) of the current diagonal block, lanes
-    // >= 32 the identity column that becomes W(:, lane - 32)
-    T v[32];
-    // from_lds: the block as the next-column update left it in Dsm (lower
-    // part; the strict upper part of v is never read)
-    auto load_diag = [&](int j0, bool from_lds) {
-        int j = lane - 32;
-        asm volatile("" : "+v"(j));                  // built per block: keeps the identity out of LICM
-        const int lr = min(lane, 31);
-#pragma unroll
-        for (int c = 0; c < 32; c++) {
-            const int r = j0 + lane, cc = j0 + c;
-            const T a = from_lds ? Dsm[c * 33 + lr]
-                                 : load_if(&A[(int64_t)min(cc, n - 1) * ld + min(r, n - 1)], r < n && cc < n);
-            v[c] = lrow ? ((r < n && cc < n) ? a : T(0)) : (c == j ? T(1) : T(0));
-        }
-    };
-    if (wave == 0) load_diag(0, false);
-    __syncthreads();
-
-    for (int j0 = 0; j0 < n; j0 += 32) {
-        const int jw = min(32, n - j0);
-        if (wave == 0) {
-            unsigned bad = 0;                        // non-positive pivots, bit c
-#pragma unroll
-            for (int c = 0; c < 32; c++) {
-                T d0 = readlane_t(v[c], c);
-                const bool ok = c < jw ? d0 > T(0) : true;
-                bad |= (ok ? 0u : 1u) << c;
-                d0 = ok && c < jw ? d0 : T(1);
-                const T d = sqrt(d0);
-                const T rd = T(1) / d;
-                const T sc = v[c] * rd;              // L(lane, c) below the diagonal / W(c, j)
-                const T m = (!lrow || lane > c) ? sc : T(0);
-                v[c] = lrow ? (lane == c ? d : (lane > c ? sc : v[c])) : sc;
-#pragma unroll
-                for (int c2 = c + 1; c2 < 32; c2++) v[c2] -= m * readlane_t(m, c2);
-            }
-            if (lrow) {
-#pragma unroll
-                for (int c = 0; c < 32; c++)
-                    if (c <= lane) P[c * RC + j0 + lane] = v[c];
-            } else {
-#pragma unroll
-                for (int c = 0; c < 32; c++) Ws[(lane - 32) * 32 + c] = v[c];
-            }
-            if (bad && lane == 0) s_fail = j0 + __builtin_ctz(bad) + 1;
-        } else if (j0 > 0) {
-            // trailing update of block j0-32 beyond the current block column
-            const int b0 = j0 + 32, nb = (n - b0 + 31) / 32;
-            for (int u = wave - 1; u < nb * (nb + 1) / 2; u += 7) {
-                int bi = 0, rem = u;                 // unit u -> (row block bi >= col block bj)
-                while (rem > bi) { rem -= bi + 1; bi++; }
-                syrk_unit32<T>(A, ld, n, P, RC, b0 + 32 * bi, b0 + 32 * rem, fr, fk);
-            }
-        }
-        __syncthreads();
-        if (s_fail) break;
-
-        // X = A(j0+32:n, j0:j0+32) W^T on MFMA (K = 32), accumulated as
-        // X^T = W P2^T so that lane l holds row rt + l % 16; rows to P and A
-        for (int rt = j0 + 32 + 16 * wave; rt < n; rt += 128) {
-            V4 e0 = {T(0), T(0), T(0), T(0)}, e1 = e0;
-            const int r = rt + fr;
-            const int rc = min(r, n - 1);
-#pragma unroll
-            for (int s4 = 0; s4 < 8; s4++) {
-                const int kk = 4 * s4 + fk;
-                const T a = load_if(&A[(int64_t)(j0 + min(kk, jw - 1)) * ld + rc], r < n && kk < jw);
-                e0 = MF<T>::mfma(Ws[kk * 32 + fr], a, e0);          // W(c, kk), c = fr
-                e1 = MF<T>::mfma(Ws[kk * 32 + 16 + fr], a, e1);     // c = 16 + fr
-            }
-            if (r < n) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int c = MF<T>::row(q, fk);
-                    P[c * RC + r] = e0[q];
-                    P[(16 + c) * RC + r] = e1[q];
-                    if (c < jw) A[(int64_t)(j0 + c) * ld + r] = e0[q];
-                    if (16 + c < jw) A[(int64_t)(j0 + 16 + c) * ld + r] = e1[q];
-                }
-            }
-        }
-        // L_jj to A, W_jj to Winv
-        for (int idx = tid; idx < 1024; idx += 512) {
-            const int c = idx >> 5, r = idx & 31;
-            if (r >= c && r < jw && c < jw) A[(int64_t)(j0 + c) * ld + j0 + r] = P[c * RC + j0 + r];
-            Winv[(j0 >> 5) * 1024 + idx] = Ws[idx];
-        }
-        __syncthreads();
-
-        // the next block column first (rows j0+32.., columns j0+32..j0+63)
-        const int b1 = j0 + 32;
-        if (b1 < n) {
-            for (int u = wave; u < (n - b1 + 31) / 32; u += 8)
-                syrk_unit32<T>(A, ld, n, P, RC, b1 + 32 * u, b1, fr, fk, u == 0 ? Dsm : nullptr);
-        }
-        __syncthreads();
-        if (wave == 0 && b1 < n) load_diag(b1, true);
-    }
-    if (tid == 0 && s_fail) atomicCAS(d_info, 0, info_base + s_fail);
-}
-
-template <class T>
-__global__ __launch_bounds__(512) void k_potrf_tile(T *__restrict__ A, int n, int ld, int RC,
-                                                   int info_base, int *__restrict__ d_info,
-                                                   T *__restrict__ Winv)
-{
-    potrf_tile_dev<T>(A, n, ld, RC, info_base, d_info, Winv);
-}
-
-// ---------------------------------------------------------------------------
-// TRSM(m,k) for m = k+1 .. MT-1: C <- C L^{-T}, one workgroup (4 waves) per
-// 64-row strip of a tile, 32 columns at a time:
-//   P = C[:, j0:j0+32] - X[:, 0:j0] L[j0:j0+32, 0:j0]^T   (MFMA, wave w: rows 16w..)
-//   X[:, j0:j0+32] = P W_jj^T                              (W from POTRF(k))
-constexpr int TS_ROWS = 64;
-template <class T>
-__global__ __launch_bounds__(256, 2) void k_trsm_tile(T *__restrict__ Tt, int N, int NB, int MT, int k,
-                                                  const T *__restrict__ Winv, int m0)
-{
-    __shared__ T P[32][TS_ROWS + 1];
-    __shared__ T Ws[1024];
-    typedef typename MF<T>::v4 V4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fk = lane >> 4;
-    const int strips = (NB + TS_ROWS - 1) / TS_ROWS;
-    const int m = m0 + blockIdx.x / strips;
-    const int r0 = (blockIdx.x % strips) * TS_ROWS;
-    const int rows_m = tile_rows(N, NB, MT, m);
-    if (r0 >= rows_m) return;
-    const int rv = min(TS_ROWS, rows_m - r0);
-    T *C = Tt + tile_index(MT, m, k) * (int64_t)NB * NB + r0;
-    const T *L = Tt + tile_index(MT, k, k) * (int64_t)NB * NB;
-
-    for (int j0 = 0; j0 < NB; j0 += 32) {
-        const int jw = min(32, NB - j0);
-        // this block's columns of C (written only by this step) and W_jj do
-        // not depend on the solve so far: in flight during the product
-        T cb[2][4], wv[4];
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int rr = wave * 16 + MF<T>::row(q, fk), c = ct * 16 + fr;
-                cb[ct][q] = load_if(&C[(int64_t)(j0 + min(c, jw - 1)) * NB + min(rr, rv - 1)], rr < rv && c < jw);
-            }
-#pragma unroll
-        for (int u = 0; u < 4; u++) wv[u] = Winv[(j0 >> 5) * 1024 + tid + 256 * u];
-        V4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-        if (j0 > 0) mfma_panel_2(C, NB, wave * 16, rv, L + j0, NB, 0, jw, j0, acc);
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int rr = wave * 16 + MF<T>::row(q, fk), c = ct * 16 + fr;
-                P[c][rr] = (rr < rv && c < jw) ? cb[ct][q] - acc[ct][q] : T(0);
-            }
-#pragma unroll
-        for (int u = 0; u < 4; u++) Ws[tid + 256 * u] = wv[u];
-        __syncthreads();
-        // X = P W_jj^T on MFMA (W_jj is zero above its diagonal), fed (W, P)
-        // so that element q of lane l holds row 16 w + l % 16 and column
-        // 16 ct + row(q, l / 16): the stores walk rows
-        {
-            V4 xo[2] = {{T(0), T(0), T(0), T(0)}, {T(0), T(0), T(0), T(0)}};
-#pragma unroll
-            for (int s4 = 0; s4 < 8; s4++) {
-                const int kk = 4 * s4 + fk;
-                const T a = P[kk][wave * 16 + fr];
-#pragma unroll
-                for (int ct = 0; ct < 2; ct++) xo[ct] = MF<T>::mfma(Ws[kk * 32 + ct * 16 + fr], a, xo[ct]);
-            }
-            const int rr = wave * 16 + fr;
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int c = ct * 16 + MF<T>::row(q, fk);
-                    if (rr < rv && c < jw) C[(int64_t)(j0 + c) * NB + rr] = xo[ct][q];
-                }
-        }
-        __syncthreads();
-    }
-}
-
-// TRSM(m,k) for few panel tiles (latency-bound steps): one workgroup per
-// 16-row strip; the left-looking product X[:, 0:j0] L[j0:j0+32, 0:j0]^T of
-// each 32-column block is split over the 4 waves by K (contiguous 32-column
-// slices, partial sums met in LDS), so the per-block chain is a quarter of
-// the 64-row kernel's; then P = C - sum and X = P W_jj^T on MFMA.  Bounded
-// to two workgroups per CU (256 registers a lane) without spills.
-constexpr int TSK_ROWS = 16;
-template <class T>
-__global__ __launch_bounds__(256, 2) void k_trsm_tile_ks(T *__restrict__ Tt, int N, int NB, int MT, int k,
-                                                     const T *__restrict__ Winv, int m0)
-{
-    __shared__ T red[4][32][TSK_ROWS + 1];       // partial products [wave][col][row]
-    __shared__ T P[32][TSK_ROWS + 1];
-    __shared__ T Ws[1024];
-    typedef typename MF<T>::v4 V4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fk = lane >> 4;
-    const int strips = (NB + TSK_ROWS - 1) / TSK_ROWS;
-    const int m = m0 + blockIdx.x / strips;
-    const int r0 = (blockIdx.x % strips) * TSK_ROWS;
-    const int rows_m = tile_rows(N, NB, MT, m);
-    if (r0 >= rows_m) return;
-    const int rv = min(TSK_ROWS, rows_m - r0);
-    T *C = Tt + tile_index(MT, m, k) * (int64_t)NB * NB + r0;
-    const T *L = Tt + tile_index(MT, k, k) * (int64_t)NB * NB;
-
-    for (int j0 = 0; j0 < NB; j0 += 32) {
-        const int jw = min(32, NB - j0);
-        // this block's columns of C (written only by this step) and W_jj do
-        // not depend on the solve so far: in flight during the product
-        T cb[2], wv[4];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int idx = tid + 256 * u, r = idx % TSK_ROWS, c = idx / TSK_ROWS;
-            cb[u] = load_if(&C[(int64_t)(j0 + min(c, jw - 1)) * NB + min(r, rv - 1)], r < rv && c < jw);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) wv[u] = Winv[(j0 >> 5) * 1024 + tid + 256 * u];
-        // this wave's K slice of the j0 solved columns
-        const int np = j0 / 32;
-        const int p0 = (np * wave) / 4, p1 = (np * (wave + 1)) / 4;
-        V4 acc[2] = {{T(0), T(0), T(0), T(0)}, {T(0), T(0), T(0), T(0)}};
-        if (p1 > p0)
-            mfma_panel_2(C + (int64_t)(32 * p0) * NB, NB, 0, rv, L + (int64_t)(32 * p0) * NB + j0, NB, 0, jw,
-                         32 * (p1 - p0), acc);
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) red[wave][ct * 16 + fr][MF<T>::row(q, fk)] = acc[ct][q];
-#pragma unroll
-        for (int u = 0; u < 4; u++) Ws[tid + 256 * u] = wv[u];
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int idx = tid + 256 * u, r = idx % TSK_ROWS, c = idx / TSK_ROWS;
-            const T sum = red[0][c][r] + red[1][c][r] + red[2][c][r] + red[3][c][r];
-            P[c][r] = (r < rv && c < jw) ? cb[u] - sum : T(0);
-        }
-        __syncthreads();
-        // X = P W_jj^T on MFMA (W_jj is zero above its diagonal): waves 0
-        // and 1 take 16 columns each, fed (W, P) so that the stores walk rows
-        if (wave < 2) {
-            V4 xo = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-            for (int s4 = 0; s4 < 8; s4++) {
-                const int kk = 4 * s4 + fk;
-                xo = MF<T>::mfma(Ws[kk * 32 + wave * 16 + fr], P[kk][fr], xo);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int c = wave * 16 + MF<T>::row(q, fk);
-                if (fr < rv && c < jw) C[(int64_t)(j0 + c) * NB + fr] = xo[q];
-            }
-        }
-        __syncthreads();
-    }
-}
 
 // ---------------------------------------------------------------------------
 // POTRF(k): factor the n x n diagonal tile A (ld) in place, lower.
@@ -700,16 +266,17 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
     *bn = s - (*bm) * nsub;
 }
 
-// The FP64 MFMA pipe of a gfx950 SIMD issues at full rate only with two
-// waves ready on it (one wave alone issues at half rate).  The workgroup's
-// waves form a WR x WC grid over its BMX x BMX block, each wave a
-// (BMX/WR) x (BMX/WC) sub-block of 16x16 MFMA tiles.  Two workgroups share
+// The workgroup's waves form a WR x WC grid over its BMX x BMX block, each
+// wave a (BMX/WR) x (BMX/WC) sub-block of 16x16 MFMA tiles.  Two workgroups share
 // each CU: WR x WC = 2 x 2 holds 256 registers per lane (two waves per
 // SIMD); 4 x 2 holds 128 (four waves per SIMD), so that a workgroup waiting
 // at a barrier or on memory still leaves two waves per SIMD issuing.
+// One block: C(r_base.., c_base..) -= A(r_base.., 0:K) B(c_base.., 0:K)^T, all
+// of them column-major with leading dimension NB; rows_m / cols_n bound the
+// rows of A and C / the rows of B and columns of C; diag: only row >= column.
 template <class T, int BMX, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__ Tt, int N, int NB, int MT, int k,
-                                                                int n_begin, int m_off, int nsub)
+__device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, int NB, int K, int rows_m, int cols_n,
+                                             int r_base, int c_base, bool diag)
 {
     // rows padded by 128 bytes: the four lane groups of a fragment read (k
     // rows 4s + l/16) then fall on alternating halves of the LDS banks
@@ -727,26 +294,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WC, wn = wave % WC;
 
-    // XCD-aware remap: consecutive workgroup ids land on different XCDs
-    // (round-robin), so give each XCD a contiguous range of blocks; the
-    // blocks of one tile then share their A/B panels in that XCD's L2.
-    const int G = gridDim.x, bid = blockIdx.x;
-    const int G8 = (G / 8) * 8;
-    const int L = (bid < G8) ? (bid % 8) * (G8 / 8) + bid / 8 : bid;
-
-    int m, n, bm, bn;
-    decode_block(L, nsub, n_begin, m_off, MT, &m, &n, &bm, &bn);
-    if (m == n && bm < bn) return;                 // strictly upper blocks of a diagonal tile
-
-    const int rows_m = tile_rows(N, NB, MT, m);
-    const int cols_n = tile_rows(N, NB, MT, n);
-    const int r_base = bm * BMX, c_base = bn * BMX;
-    if (r_base >= rows_m || c_base >= cols_n) return;
-    const bool full = (r_base + BMX <= rows_m) && (c_base + BMX <= cols_n) && (NB % BK == 0) && !(NB & 1);
-
-    const T *Ap = Tt + tile_index(MT, m, k) * (int64_t)NB * NB;
-    const T *Bp = Tt + tile_index(MT, n, k) * (int64_t)NB * NB;
-    T *Cp = Tt + tile_index(MT, m, n) * (int64_t)NB * NB;
+    const bool full = (r_base + BMX <= rows_m) && (c_base + BMX <= cols_n) && (K % BK == 0) && !(NB & 1);
 
     V4 acc[TR][TC];
 #pragma unroll
@@ -773,7 +321,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
                 const int kk = e / PR, r = (e % PR) * 2;
                 const int kg = k0 + kk;
                 T a0 = T(0), a1 = T(0), b0 = T(0), b1 = T(0);
-                if (kg < NB) {
+                if (kg < K) {
                     const T *ac = Ap + (int64_t)kg * NB;
                     const T *bc = Bp + (int64_t)kg * NB;
                     if (r_base + r < rows_m) a0 = ac[r_base + r];
@@ -802,7 +350,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
     // full off-diagonal blocks start from C (loaded with the first operands)
     // and end with a plain store; the others accumulate -A B^T from zero
     const int fr0 = lane & 15, fk0 = lane >> 4;
-    const bool pre = full && !((m == n) && (bm == bn));
+    const bool pre = full && !diag;
     if (pre) {
 #pragma unroll
         for (int p = 0; p < TR / 2; p++)
@@ -817,7 +365,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
                 }
             }
     }
-    const int nstage = (NB + BK - 1) / BK;
+    const int nstage = (K + BK - 1) / BK;
     gload(0);
     lstore(0);
     __syncthreads();
@@ -849,7 +397,6 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
     // epilogue: the MFMA was fed (B, A), so element q of lane l holds row
     // 2 (l % 16) + t (tile 2p + t) and column row(q, l / 16) of each 16x16
     // tile: a store walks row pairs
-    const bool diag = (m == n) && (bm == bn);
 #pragma unroll
     for (int p = 0; p < TR / 2; p++) {
         const int rr = r_base + wm * HR + 32 * p + 2 * fr;
@@ -869,6 +416,58 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__
                 }
             }
     }
+}
+
+// workgroup id -> position in the launch's list of blocks: consecutive ids
+// land on different XCDs (round-robin), so each XCD is given a contiguous
+// range of blocks; the blocks of one tile then share their A/B panels in
+// that XCD's L2
+__device__ __forceinline__ int xcd_block()
+{
+    const int G = gridDim.x, bid = blockIdx.x;
+    const int G8 = (G / 8) * 8;
+    return (bid < G8) ? (bid % 8) * (G8 / 8) + bid / 8 : bid;
+}
+
+template <class T, int BMX, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__ Tt, int N, int NB, int MT, int k,
+                                                                int n_begin, int m_off, int nsub)
+{
+    int m, n, bm, bn;
+    decode_block(xcd_block(), nsub, n_begin, m_off, MT, &m, &n, &bm, &bn);
+    if (m == n && bm < bn) return;                 // strictly upper blocks of a diagonal tile
+    const int rows_m = tile_rows(N, NB, MT, m);
+    const int cols_n = tile_rows(N, NB, MT, n);
+    const int r_base = bm * BMX, c_base = bn * BMX;
+    if (r_base >= rows_m || c_base >= cols_n) return;
+    const int64_t sz = (int64_t)NB * NB;
+    update_block<T, BMX, WR, WC>(Tt + tile_index(MT, m, k) * sz, Tt + tile_index(MT, n, k) * sz,
+                                 Tt + tile_index(MT, m, n) * sz, NB, NB, rows_m, cols_n, r_base, c_base,
+                                 m == n && bm == bn);
+}
+
+// Inside tile column k, after its columns c0 .. c0 + w - 1 are solved: the
+// columns from c0 + w on lose X X_k^T (K = w), X the solved rows of each tile
+// and X_k those of tile (k, k).  The first g0 block rows are those of tile
+// (k, k) below c0 + w (lower part), then gr block rows of each tile m0, m0 +
+// 1, ...; nc blocks a block row.
+template <class T, int BMX, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_panel_update(T *__restrict__ Tt, int N, int NB, int MT, int k,
+                                                                 int c0, int w, int g0, int gr, int nc, int m0)
+{
+    const int L = xcd_block();
+    const int rb = L / nc, bn = L - rb * nc;
+    const int c1 = c0 + w;
+    const int m = rb < g0 ? k : m0 + (rb - g0) / gr;
+    if (rb < g0 && rb < bn) return;
+    const int r_base = rb < g0 ? c1 + BMX * rb : BMX * ((rb - g0) % gr), c_base = c1 + BMX * bn;
+    const int rows_m = tile_rows(N, NB, MT, m);
+    const int cols_n = tile_rows(N, NB, MT, k);
+    if (r_base >= rows_m || c_base >= cols_n) return;
+    const int64_t sz = (int64_t)NB * NB;
+    T *Cp = Tt + tile_index(MT, m, k) * sz;
+    update_block<T, BMX, WR, WC>(Cp + (int64_t)c0 * NB, Tt + tile_index(MT, k, k) * sz + (int64_t)c0 * NB, Cp, NB, w,
+                                 rows_m, cols_n, r_base, c_base, rb == bn && rb < g0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1444,29 +1043,6 @@ __global__ __launch_bounds__(256) void k_update_valu(double *__restrict__ T, int
         }
 }
 
-// Recursive diagonal factor (hmb): the lower triangle of one n x n tile
-// (column-major, ld) <-> a packed lower image of hmb x hmb sub-tiles (the
-// layout of the whole matrix, one level down).  One thread per element of
-// the image; the strict upper part of the diagonal sub-tiles and padding
-// rows are copied out as zeros and never copied back.
-template <class T, bool TO_IMG>
-__global__ __launch_bounds__(256) void k_subtile_copy(T *__restrict__ tile, int n, int ld, int hmb, int MTs,
-                                                      T *__restrict__ img, int64_t nel)
-{
-    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (e >= nel) return;
-    const int64_t per = (int64_t)hmb * hmb;
-    int64_t t = e / per;
-    const int w = (int)(e - t * per), col = w / hmb, row = w - col * hmb;
-    int sn = 0;                                  // sub-tile column
-    while (t >= MTs - sn) { t -= MTs - sn; sn++; }
-    const int sm = sn + (int)t;
-    const int r = sm * hmb + row, cc = sn * hmb + col;
-    const bool in = r < n && cc < n && r >= cc;
-    if (TO_IMG) img[e] = in ? tile[(int64_t)cc * ld + r] : T(0);
-    else if (in) tile[(int64_t)cc * ld + r] = img[e];
-}
-
 __global__ void k_fill_int(int *p, int v, int n)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1499,12 +1075,14 @@ template <> struct KN<double> {
     static constexpr const char *trsm = "dpotrf_trsm_panel";
     static constexpr const char *update = "dpotrf_update";
     static constexpr const char *update_la = "dpotrf_update_la";
+    static constexpr const char *panel_update = "dpotrf_panel_update";
 };
 template <> struct KN<float> {
     static constexpr const char *potrf = "spotrf_potrf_diag";
     static constexpr const char *trsm = "spotrf_trsm_panel";
     static constexpr const char *update = "spotrf_update";
     static constexpr const char *update_la = "spotrf_update_la";
+    static constexpr const char *panel_update = "spotrf_panel_update";
     static constexpr const char *update_bf16 = "spotrf_update_bf16x3";
     static constexpr const char *update_bf16_la = "spotrf_update_bf16x3_la";
     static constexpr const char *split_panel = "spotrf_split_panel";
@@ -1512,68 +1090,97 @@ template <> struct KN<float> {
 
 template <class T> bool valu_panel() { return std::is_same<T, double>::value && g_panel_kernel == 0; }
 
-template <class T>
-int potrf_lds_bytes(int NB, int *RC)
-{
-    if (!valu_panel<T>()) {
-        *RC = ((NB + 15) & ~15) + 1;
-        return (32 * (*RC) + 1024 + 32 * 33) * (int)sizeof(T);
-    }
-    *RC = ((NB + 3) & ~3) + 4;
-    return (PJB * (*RC) + 1024) * (int)sizeof(double);
-}
+// Largest diagonal tile (or sub-tile, where hmb re-tiles it) that the entry
+// points take: what one workgroup's LDS held when a whole tile was factored
+// there.  The panel kernels need no such limit; larger tiles stay refused.
+template <class T> constexpr int diag_limit() { return sizeof(T) == 8 ? 560 : 1200; }
+constexpr int VALU_DIAG_LIMIT = 604;               // k_potrf_diag: the tile's block column in 160 KB of LDS
 
-// info_off: added to k*NB + j of a failing pivot (the offset of this tile
-// grid inside a larger matrix)
-template <class T>
-int launch_potrf(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k, T *Winv, int info_off = 0)
+template <class T> int check_diag(int n)
 {
-    // LDS and its row stride RC for the n rows of this tile (RC >= n + 1)
-    const int n = tile_rows(N, NB, MT, k);
-    int RC;
-    int lds = potrf_lds_bytes<T>(n, &RC);
-    T *A = dT + tile_index(MT, k, k) * (int64_t)NB * NB;
-    const double fl = (double)n * n * n / 3.0;
-    if (!valu_panel<T>()) {
-        MI_LAUNCH(c, s, KN<T>::potrf, fl, 2.0 * n * n * sizeof(T),
-                  k_potrf_tile<T><<<1, 512, lds, s>>>(A, n, NB, RC, info_off + k * NB, c->d_info, Winv));
-    } else {
-        MI_LAUNCH(c, s, KN<T>::potrf, fl, 2.0 * n * n * sizeof(T),
-                  k_potrf_diag<<<1, POTRF_THREADS, lds, s>>>((double *)A, n, NB, RC, info_off + k * NB,
-                                                              c->d_info, (double *)Winv));
+    if (n > (valu_panel<T>() ? VALU_DIAG_LIMIT : diag_limit<T>())) {
+        set_error("tile size %d exceeds the limit of the diagonal factorization (%d)", n,
+                  valu_panel<T>() ? VALU_DIAG_LIMIT : diag_limit<T>());
+        return -4;
     }
     return 0;
 }
 
-// TRSM(m, k) for the ntile tiles m = m0 .. m0 + ntile - 1 (by default every
-// m > k).
-template <class T>
-int launch_trsm(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k, const T *Winv, int m0 = -1,
-                int ntile = -1)
+// Panel engine 0 (FP64, tiles that fit its LDS): POTRF(k), then TRSM(m, k)
+// for the ntile tiles from m0, one launch each.
+int launch_panel_valu(Ctx *c, hipStream_t s, double *dT, int N, int NB, int MT, int k, double *Winv, bool diag, int m0,
+                      int ntile)
 {
-    if (m0 < 0) m0 = k + 1;
-    if (ntile < 0) ntile = MT - m0;
-    if (ntile <= 0) return 0;
-    double fl = 0.0;
-    for (int m = m0; m < m0 + ntile; m++) fl += (double)tile_rows(N, NB, MT, m) * NB * NB;
-    if (!valu_panel<T>()) {
-        // 64-row strips while there are many tiles; below ~50 tiles (FP64)
-        // or ~40 (FP32) of NB = 512 the 16-row K-split kernel is faster alone
-        const int strips = (NB + TS_ROWS - 1) / TS_ROWS;
-        if (ntile * strips >= (sizeof(T) == 8 ? 400 : 320)) {
-            MI_LAUNCH(c, s, KN<T>::trsm, fl, fl / NB * 2.0 * sizeof(T),
-                      k_trsm_tile<T><<<ntile * strips, 256, 0, s>>>(dT, N, NB, MT, k, Winv, m0));
-        } else {
-            // few tiles: 16-row strips with the K range split over the waves
-            const int ks = (NB + TSK_ROWS - 1) / TSK_ROWS;
-            MI_LAUNCH(c, s, KN<T>::trsm, fl, fl / NB * 2.0 * sizeof(T),
-                      k_trsm_tile_ks<T><<<ntile * ks, 256, 0, s>>>(dT, N, NB, MT, k, Winv, m0));
-        }
-    } else {
+    const int n = tile_rows(N, NB, MT, k);
+    if (diag) {
+        const int RC = ((n + 3) & ~3) + 4, lds = (PJB * RC + 1024) * (int)sizeof(double);
+        if (lds > 65536)
+            MI_CHECK(hipFuncSetAttribute((const void *)k_potrf_diag, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        double *A = dT + tile_index(MT, k, k) * (int64_t)NB * NB;
+        MI_LAUNCH(c, s, KN<double>::potrf, (double)n * n * n / 3.0, 16.0 * n * n,
+                  k_potrf_diag<<<1, POTRF_THREADS, lds, s>>>(A, n, NB, RC, k * NB, c->d_info, Winv));
+    }
+    if (ntile > 0) {
+        double fl = 0.0;
+        for (int m = m0; m < m0 + ntile; m++) fl += (double)tile_rows(N, NB, MT, m) * NB * NB;
         const int strips = (NB + TRSM_ROWS - 1) / TRSM_ROWS;
-        MI_LAUNCH(c, s, KN<T>::trsm, fl, fl / NB * 2.0 * sizeof(T),
-                  k_trsm_panel<<<ntile * strips, 256, 0, s>>>((double *)dT, N, NB, MT, k,
-                                                             (const double *)Winv, m0));
+        MI_LAUNCH(c, s, KN<double>::trsm, fl, fl / NB * 2.0 * sizeof(double),
+                  k_trsm_panel<<<ntile * strips, 256, 0, s>>>(dT, N, NB, MT, k, Winv, m0));
+    }
+    return 0;
+}
+
+// Panel of step k on s: POTRF(k) when diag, and TRSM(m, k) of the ntile tiles
+// m0, m0 + 1, ... (rows of the tile column), sub-column by sub-column of sb
+// columns (a multiple of 32, at most SB): factor its diagonal block, solve
+// the rows below, update the tile column's remaining columns.  ws: the
+// operand images, (NB / 16) OPB elements, written when diag and read again by
+// a call without it.
+//
+// Why sub-columns of 128: the diagonal block is one workgroup's chain of
+// pivots, everything else spreads over the chip, and a launch behind another
+// on one stream costs well under a microsecond.
+template <class T>
+int launch_panel(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k, T *ws, int sb, bool diag, int m0,
+                 int ntile)
+{
+    const int n = tile_rows(N, NB, MT, k);
+    if constexpr (std::is_same<T, double>::value)
+        if (valu_panel<T>() && n <= VALU_DIAG_LIMIT)
+            return launch_panel_valu(c, s, dT, N, NB, MT, k, ws, diag, m0, ntile);
+    double below = 0.0;                            // rows of the other tiles
+    for (int m = m0; m < m0 + ntile; m++) below += tile_rows(N, NB, MT, m);
+    T *A = dT + tile_index(MT, k, k) * (int64_t)NB * NB;
+    for (int c0 = 0; c0 < n; c0 += sb) {
+        const int w = std::min(sb, n - c0), c1 = c0 + w;
+        T *op = ws + (int64_t)(c0 / DB) * OPB;
+        if (diag)
+            MI_LAUNCH(c, s, KN<T>::potrf, (double)w * w * w / 3.0, 2.0 * w * w * sizeof(T),
+                      k_diag_factor<T><<<1, 512, 0, s>>>(A + (int64_t)c0 * NB + c0, w, NB, k * NB + c0, c->d_info, op));
+        const double rows = below + (diag ? n - c1 : 0);
+        const int g0 = diag ? (n - c1 + 63) / 64 : 0, gt = (NB + 63) / 64;
+        if (g0 + gt * ntile > 0)
+            MI_LAUNCH(c, s, KN<T>::trsm, rows * w * w, 2.0 * rows * w * sizeof(T),
+                      k_panel_solve<T><<<g0 + gt * ntile, 256, 0, s>>>(dT, N, NB, MT, k, c0, w, op, g0, gt, m0));
+        if (c1 >= n || (!diag && ntile <= 0)) continue;
+        // 128 x 128 blocks once they fill the chip twice over
+        auto grid = [&](int bm, int *b0, int *br, int *nc) {
+            *b0 = diag ? (n - c1 + bm - 1) / bm : 0;
+            *br = (NB + bm - 1) / bm;
+            *nc = (n - c1 + bm - 1) / bm;
+            return (*b0 + *br * ntile) * *nc;
+        };
+        int b0, br, nc;
+        const double fl = 2.0 * below * w * (n - c1) + (diag ? (double)w * (n - c1) * (n - c1 + 1.0) : 0.0);
+        const double by = (below + (diag ? 0.5 * (n - c1) : 0.0)) * (2.0 * (n - c1) + w) * sizeof(T);
+        if (grid(BM, &b0, &br, &nc) >= 512)
+            MI_LAUNCH(c, s, KN<T>::panel_update, fl, by,
+                      (k_panel_update<T, BM, 4, 2><<<grid(BM, &b0, &br, &nc), 512, 0, s>>>(dT, N, NB, MT, k, c0, w, b0,
+                                                                                          br, nc, m0)));
+        else
+            MI_LAUNCH(c, s, KN<T>::panel_update, fl, by,
+                      (k_panel_update<T, 64, 2, 2><<<grid(64, &b0, &br, &nc), 256, 0, s>>>(dT, N, NB, MT, k, c0, w, b0,
+                                                                                          br, nc, m0)));
     }
     return 0;
 }
@@ -1680,32 +1287,9 @@ int launch_split_panel(Ctx *c, hipStream_t s, const float *dT, int N, int NB, in
     return 0;
 }
 
-template <class T>
-int prepare_potrf(int NB)
-{
-    int RC;
-    int lds = potrf_lds_bytes<T>(NB, &RC);
-    int dev = 0;
-    MI_CHECK(hipGetDevice(&dev));
-    hipDeviceProp_t prop;
-    MI_CHECK(hipGetDeviceProperties(&prop, dev));
-    size_t limit = prop.sharedMemPerBlock;
-    if ((size_t)lds > limit) {
-        set_error("tile size NB=%d needs %d B of LDS for the diagonal factorization (limit %zu)",
-                  NB, lds, limit);
-        return -4;
-    }
-    if (lds > 65536) {
-        MI_CHECK(hipFuncSetAttribute(!valu_panel<T>() ? (const void *)k_potrf_tile<T> : (const void *)k_potrf_diag,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    }
-    return 0;
-}
-
-// Elements of the diagonal-block inverses handed from POTRF(k) to TRSM(k),
-// two steps in flight.
-constexpr size_t potrf_ws_elems(int NB) { return (size_t)2 * ((NB + 31) / 32) * 1024; }
-
+// Elements of the operand images handed from POTRF(k) to TRSM(k), two steps
+// in flight (the VALU panel's 32 x 32 inverses need a quarter of that).
+constexpr size_t potrf_ws_elems(int NB) { return (size_t)2 * ((NB + DB - 1) / DB) * OPB; }
 
 // Whole factorization of the packed lower tiles dT (N, NB), resident, with a
 // two-step look-ahead over two streams (src/zpotrf_L.jdf's priorities give
@@ -1724,53 +1308,16 @@ constexpr size_t potrf_ws_elems(int NB) { return (size_t)2 * ((NB + 31) / 32) * 
 // ring: cross-stream dependencies use the context's fixed ring of events
 // (created with the context) instead of its growing pool; every event is
 // waited on within three records of being recorded, far inside the ring.
-// POTRF(k) of an n x n diagonal tile (ld NB) as a tile Cholesky of its own
-// with hmb x hmb sub-tiles (src/zpotrf_L.jdf:168-192: the RECURSIVE body
-// re-tiles the task with smallnb when the tile is larger), enqueued on s:
-// the tile is copied into a packed image of sub-tiles, factored there by
-// the same POTRF / TRSM / update launches (many workgroups for the panel
-// solves and updates inside the tile), and the factor copied back.  hmb is
-// a multiple of 32, so the 32 x 32 diagonal-block inverses of sub-step j
-// land in Winv at block j * hmb / 32, where the panel TRSM of the enclosing
-// step reads them.  img: the packed image, (MTs (MTs + 1) / 2) hmb^2
-// elements.
-template <class T>
-int potrf_rec(Ctx *c, hipStream_t s, T *tile, int n, int NB, int hmb, T *Winv, int info_off, T *img)
-{
-    const int MTs = (n + hmb - 1) / hmb;
-    const int64_t nel = (int64_t)MTs * (MTs + 1) / 2 * hmb * hmb;
-    const unsigned grid = (unsigned)((nel + 255) / 256);
-    MI_LAUNCH(c, s, "potrf_rec_copy", 0.0, 16.0 * nel,
-              (k_subtile_copy<T, true><<<grid, 256, 0, s>>>(tile, n, NB, hmb, MTs, img, nel)));
-    int rc;
-    for (int j = 0; j < MTs; j++) {
-        T *w = Winv + (int64_t)(j * hmb / 32) * 1024;
-        if ((rc = launch_potrf<T>(c, s, img, n, hmb, MTs, j, w, info_off))) return rc;
-        if ((rc = launch_trsm<T>(c, s, img, n, hmb, MTs, j, w, -1, -1))) return rc;
-        if ((rc = launch_update<T>(c, s, img, n, hmb, MTs, j, j + 1, MTs, false, true))) return rc;
-    }
-    MI_LAUNCH(c, s, "potrf_rec_copy", 0.0, 16.0 * nel,
-              (k_subtile_copy<T, false><<<grid, 256, 0, s>>>(tile, n, NB, hmb, MTs, img, nel)));
-    return 0;
-}
-
-// hmb: recursive diagonal factor with sub-tiles of hmb (rounded down to a
-// multiple of 32, at least 32) for the diagonal tiles larger than that; 0:
-// one POTRF launch per step.  img_ext: the sub-tile image (nullptr: the
-// context's workspace).  rec_from: the first step whose diagonal tile is
-// factored recursively (the earlier ones take one POTRF launch).
-// Sub-tile size of the recursive diagonal factor used by default: two
-// sub-tiles of NB / 2 a side for NB >= 512 (a multiple of 64), none below
-// (the image then has 3 (NB / 2)^2 elements).  The FP64 factor uses it for
-// every step (N = 32768, NB = 512: 202.2 against 204.2 ms); the BF16-split
-// FP32 factor only from step MT / 2 on, where the panel chain is critical
-// (59.6 against 61.6-61.9 ms; from step 0 60.7 ms: in the first half the
-// extra panel launches compete with the bulk update).
+// hmb: the caller's sub-tile size of the diagonal factor (src/zpotrf_L.jdf:
+// 168-192 re-tiles POTRF(k) with smallnb); the panel's sub-columns are no
+// wider than that (rounded down to a multiple of 32, at least 32).  0: SB.
+// The entry points without one use NB / 2 for NB >= 512 (a multiple of 64),
+// which only matters for the tile sizes they take.
 constexpr int half_tile_hmb(int NB) { return (NB >= 512 && NB % 64 == 0) ? NB / 2 : 0; }
 
 template <class T>
 int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws, bool ring = false, int hmb = 0,
-                T *img_ext = nullptr, int rec_from = 0, bool wait = true)
+                bool wait = true)
 {
     *info = 0;
     if (N < 0 || NB <= 0) { set_error("bad sizes N=%d NB=%d", N, NB); return -2; }
@@ -1783,16 +1330,8 @@ int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws,
     size_t ring_next = 0;
     auto ev = [&]() -> hipEvent_t { return ring ? c->ev_ring[ring_next++ % c->ev_ring.size()] : next_event(c); };
     if (hmb > 0) hmb = std::max(32, hmb & ~31);
-    T *img = nullptr;
-    if (hmb > 0 && hmb < NB) {
-        const int MTs = (NB + hmb - 1) / hmb;
-        const size_t ib = (size_t)MTs * (MTs + 1) / 2 * hmb * hmb * sizeof(T);
-        if (!(img = img_ext ? img_ext : (T *)ws_get(c, WS_POTRF_REC, ib))) return -3;
-    }
-    // the largest diagonal block one POTRF launch factors: a sub-tile when
-    // the diagonal tiles are factored recursively (so NB may exceed what one
-    // launch's LDS holds), else a whole tile
-    if ((rc = prepare_potrf<T>(img ? hmb : NB))) return rc;
+    if ((rc = check_diag<T>(hmb > 0 ? std::min(hmb, NB) : NB))) return rc;
+    const int sb = hmb > 0 ? std::min(hmb, SB) : SB;
     // FP32 factor with BF16 updates: the main stream splits each panel
     // column once (tiles k+2.. of column k; its launches run in order, so one
     // image serves every step)
@@ -1801,13 +1340,8 @@ int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws,
         split = (__bf16 *)ws_get(c, WS_BF16_PANEL, (size_t)(MT - 2) * 2 * NB * NB * sizeof(__bf16));
         if (!split) return -3;
     }
-    auto diag = [&](int k) -> int {
-        T *w = ws + (k & 1) * wsz;
-        const int n = tile_rows(N, NB, MT, k);
-        if (img && n > hmb && k >= rec_from)
-            return potrf_rec<T>(c, c->s_panel, dT + tile_index(MT, k, k) * (int64_t)NB * NB, n, NB, hmb, w, k * NB,
-                                img);
-        return launch_potrf<T>(c, c->s_panel, dT, N, NB, MT, k, w);
+    auto panel = [&](int k) -> int {
+        return launch_panel<T>(c, c->s_panel, dT, N, NB, MT, k, ws + (k & 1) * wsz, sb, true, k + 1, MT - k - 1);
     };
 
     MI_CHECK(hipEventRecord(c->t0, c->s_main));
@@ -1817,8 +1351,7 @@ int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws,
     MI_CHECK(hipStreamWaitEvent(c->s_panel, start, 0));
 
     // panel 0
-    if ((rc = diag(0))) return rc;
-    if ((rc = launch_trsm<T>(c, c->s_panel, dT, N, NB, MT, 0, ws))) return rc;
+    if ((rc = panel(0))) return rc;
     hipEvent_t pk = ev();                          // TRSM(k) done
     MI_CHECK(hipEventRecord(pk, c->s_panel));
     hipEvent_t col_ready = nullptr;                // column k+1 updated by step k-1
@@ -1827,9 +1360,7 @@ int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws,
         // panel stream: column k+1 by step k, then the next panel
         if (col_ready) MI_CHECK(hipStreamWaitEvent(c->s_panel, col_ready, 0));
         if ((rc = launch_update<T>(c, c->s_panel, dT, N, NB, MT, k, k + 1, k + 2, bf16_split, true))) return rc;
-        T *w = ws + ((k + 1) & 1) * wsz;
-        if ((rc = diag(k + 1))) return rc;
-        if ((rc = launch_trsm<T>(c, c->s_panel, dT, N, NB, MT, k + 1, w))) return rc;
+        if ((rc = panel(k + 1))) return rc;
         hipEvent_t pk_next = ev();
         MI_CHECK(hipEventRecord(pk_next, c->s_panel));
         // main stream: the look-ahead column k+2, then the bulk of step k
@@ -1866,12 +1397,12 @@ int step_potrf(mi_ctx_t *c, int N, int NB, T *dT, int k, int *info)
 {
     if (N <= 0) { *info = 0; return 0; }
     const int MT = (N + NB - 1) / NB;
-    int rc = prepare_potrf<T>(NB);
+    int rc = check_diag<T>(NB);
     if (rc) return rc;
     T *ws = (T *)ws_get(c, WS_POTRF_WINV, potrf_ws_elems(NB) * sizeof(T));
     if (!ws) return -3;
     k_fill_int<<<1, 64, 0, c->s_main>>>(c->d_info, 0, 1);
-    if ((rc = launch_potrf<T>(c, c->s_main, dT, N, NB, MT, k, ws))) return rc;
+    if ((rc = launch_panel<T>(c, c->s_main, dT, N, NB, MT, k, ws, SB, true, k + 1, 0))) return rc;
     MI_CHECK(hipMemcpyAsync(info, c->d_info, sizeof(int), hipMemcpyDeviceToHost, c->s_main));
     return mi_synchronize(c);
 }
@@ -1879,14 +1410,14 @@ int step_potrf(mi_ctx_t *c, int N, int NB, T *dT, int k, int *info)
 template <class T>
 int step_trsm(mi_ctx_t *c, int N, int NB, T *dT, int k)
 {
-    // the diagonal-block inverses come from the POTRF launch of the same k
+    // the operand images come from the POTRF launch of the same k
     const int MT = (N + NB - 1) / NB;
-    const T *ws = (const T *)c->ws[WS_POTRF_WINV].p;
+    T *ws = (T *)c->ws[WS_POTRF_WINV].p;
     if (!ws || c->ws[WS_POTRF_WINV].bytes < potrf_ws_elems(NB) * sizeof(T)) {
         set_error("the panel solve of step k needs the POTRF launch of step k first");
         return -2;
     }
-    int rc = launch_trsm<T>(c, c->s_main, dT, N, NB, MT, k, ws);
+    int rc = launch_panel<T>(c, c->s_main, dT, N, NB, MT, k, ws, SB, false, k + 1, MT - k - 1);
     if (rc) return rc;
     return mi_synchronize(c);
 }
@@ -1907,14 +1438,14 @@ namespace mi {
 
 // Single tile tasks on the packed lower image, enqueued on s (the bodies of
 // the four task classes of src/zpotrf_L.jdf:91-633, one tile each).
-int task_prepare_fp64(int NB) { return prepare_potrf<double>(NB); }
+int task_prepare_fp64(int NB) { return check_diag<double>(NB); }
 int task_potrf_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int k, double *Winv)
 {
-    return launch_potrf<double>(c, s, dT, N, NB, (N + NB - 1) / NB, k, Winv);
+    return launch_panel<double>(c, s, dT, N, NB, (N + NB - 1) / NB, k, Winv, SB, true, k + 1, 0);
 }
-int task_trsm_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int k, const double *Winv)
+int task_trsm_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int k, double *Winv)
 {
-    return launch_trsm<double>(c, s, dT, N, NB, (N + NB - 1) / NB, k, Winv, m, 1);
+    return launch_panel<double>(c, s, dT, N, NB, (N + NB - 1) / NB, k, Winv, SB, false, m, 1);
 }
 // tile (m, n), m >= n > k: A(m, n) -= A(m, k) A(n, k)^T (SYRK when m == n)
 int task_update_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int n, int k)
@@ -1925,29 +1456,23 @@ size_t task_winv_elems(int NB) { return potrf_ws_elems(NB) / 2; }
 
 int spotrf_tiles_split(Ctx *c, int N, int NB, float *dT, int *info, bool bf16_split, bool wait)
 {
-    const int MT = NB > 0 ? (N + NB - 1) / NB : 0;
     return potrf_tiles<float>(c, N, NB, dT, info, bf16_split, nullptr, false, bf16_split ? half_tile_hmb(NB) : 0,
-                              nullptr, MT / 2, wait);
+                              wait);
 }
 }  // namespace mi
 
 // ---------------------------------------------------------------------------
 // Allocation-free FP64 factorization (mi_dpotrf_tiles_noalloc).  Its only
-// scratch memory, the 32 x 32 diagonal-block inverses that POTRF(k) hands to
-// TRSM(k) for two steps in flight and the sub-tile image of the recursive
-// diagonal factor (the same factor as mi_dpotrf_tiles), lives in this
-// file-scope device array instead of context workspaces: one copy per GPU,
-// held until the process ends, shared by every call on that GPU.  POTRF(k)
-// writes each 1024-element block whole before TRSM(k) reads it, and the
-// image is copied in from the tile before it is read, so nothing has to be
-// cleared between calls.  On the host the array's name is only a stand-in: host code uses
+// scratch memory, the operand images that a panel's diagonal factor hands to
+// its row solve, two steps in flight, lives in this file-scope device array
+// instead of context workspaces: one copy per GPU, held until the process
+// ends, shared by every call on that GPU.  Images are written before they
+// are read, so nothing has to be cleared between calls.  On the host the array's name is only a stand-in: host code uses
 // the device address that noalloc_setup reads once per device.
 namespace {
 constexpr int NOALLOC_MAX_NB = 1024;
 constexpr int NOALLOC_MAX_DEV = 64;
-constexpr size_t NOALLOC_WINV = potrf_ws_elems(NOALLOC_MAX_NB);                          // 512 KiB
-constexpr size_t NOALLOC_IMG = 3 * (size_t)(NOALLOC_MAX_NB / 2) * (NOALLOC_MAX_NB / 2);   // 6 MiB
-__device__ __align__(256) double scratch[NOALLOC_WINV + NOALLOC_IMG];
+__device__ __align__(256) double scratch[potrf_ws_elems(NOALLOC_MAX_NB)];                 // 2 MiB
 
 std::mutex g_noalloc_mu;
 bool g_noalloc_done[NOALLOC_MAX_DEV];
@@ -2071,8 +1596,7 @@ int mi_dpotrf_tiles_noalloc(mi_ctx_t *c, int N, int NB, double *dT, int *info)
     // this call
     const bool prof = c->prof;
     c->prof = false;
-    const int hmb = half_tile_hmb(NB);            // image: 3 (NB / 2)^2 <= NOALLOC_IMG elements
-    const int rc = potrf_tiles<double>(c, N, NB, dT, info, false, ptr, true, hmb, ptr + NOALLOC_WINV);
+    const int rc = potrf_tiles<double>(c, N, NB, dT, info, false, ptr, true, half_tile_hmb(NB));
     c->prof = prof;
     return rc;
 }

@@ -106,9 +106,9 @@ int mi_dspd_from_orth_tiles(mi_ctx_t *ctx, int N, int NB, const double *dQ, doub
 /* ------------------------------------------------------------ hot path */
 /* In-place tile Cholesky, lower: the POTRF/TRSM/SYRK/GEMM task classes of
  * src/zpotrf_L.jdf:91-633 as fused per-step launches with one-panel
- * look-ahead.  For NB >= 512 (a multiple of 64) the diagonal tiles are
- * factored recursively with sub-tiles of NB / 2 (as mi_dpotrf_tiles_rec
- * with hmb = NB / 2), which is faster there.  *info receives k*NB + iinfo of
+ * look-ahead.  Each tile column is factored in sub-columns of 128 columns.
+ * For NB >= 512 (a multiple of 64) this is mi_dpotrf_tiles_rec with hmb =
+ * NB / 2, otherwise with hmb = NB.  *info receives k*NB + iinfo of
  * the first non-positive pivot (src/zpotrf_L.jdf:200-202), 0 on success.
  * Blocking. */
 int mi_dpotrf_tiles(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
@@ -117,21 +117,20 @@ int mi_dpotrf_tiles(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
  * (v_mfma_f32_16x16x4_f32) trailing update, FP32 diagonal factor and panel
  * solve, same info rule.  Blocking. */
 int mi_spotrf_tiles(mi_ctx_t *ctx, int N, int NB, float *dT, int *info);
-/* mi_dpotrf_tiles with a recursive diagonal factor: POTRF(k) of every
- * diagonal tile larger than hmb runs as a tile Cholesky of that tile with
- * hmb x hmb sub-tiles (the RECURSIVE body of src/zpotrf_L.jdf:168-192 that
- * dplasma_zpotrf_setrecursive / dplasma_zpotrf_rec select,
- * src/zpotrf_wrapper.c:48-55,425-451).  hmb is rounded down to a multiple of
- * 32 (at least 32); hmb >= NB changes nothing.  Same info.  Blocking. */
+/* mi_dpotrf_tiles with the caller's re-tiling size of the diagonal factor:
+ * the sub-columns of the panel are min(hmb, 128) wide (the RECURSIVE body
+ * of src/zpotrf_L.jdf:168-192 that dplasma_zpotrf_setrecursive /
+ * dplasma_zpotrf_rec select, src/zpotrf_wrapper.c:48-55,425-451).  hmb is rounded down to a multiple of
+ * 32 (at least 32).  A diagonal tile of more than 560 rows needs hmb <= 560
+ * (else -4).  Same info.  Blocking. */
 int mi_dpotrf_tiles_rec(mi_ctx_t *ctx, int N, int NB, double *dT, int hmb, int *info);
 /* mi_dpotrf_tiles without any device allocation, for callers that cannot
  * allocate (code under stream capture, serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  Same arguments, results and
- * info as mi_dpotrf_tiles (bitwise the same factor, including its recursive
- * diagonal factor for NB >= 512).  Its scratch (the diagonal-block inverses
- * of two steps in flight and one diagonal tile's sub-tile image) is a fixed
- * 6.5 MiB device array, one per GPU, so NB <= 1024 (larger NB: -2 and an
- * error message).  Calls that overlap on one GPU race on that array,
+ * info as mi_dpotrf_tiles (bitwise the same factor).  Its scratch (the
+ * operand images that the panel's diagonal factor hands to its row solve, two
+ * steps in flight) is a fixed 2 MiB device array, one per GPU, so NB <= 1024
+ * (larger NB: -2 and an error message).  Calls that overlap on one GPU race on that array,
  * whichever context they use: serialize them.  The context's profiler is not
  * used by this call.  Blocking. */
 int mi_dpotrf_tiles_noalloc(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
@@ -192,8 +191,9 @@ int mi_dpotrf_step_potrf(mi_ctx_t *ctx, int N, int NB, double *dT, int k, int *i
  * MFMA 16x16x4 (default; two resident waves per SIMD keep it at full rate).
  * Process-wide. */
 int mi_set_update_engine(int which);
-/* Engine of POTRF(k) and the panel TRSM: 0 = VALU kernels, 1 = MFMA panel
- * updates with register/LDS diagonal blocks (default).  Process-wide. */
+/* Engine of POTRF(k) and the panel TRSM: 0 = VALU kernels (FP64, diagonal
+ * tiles of at most 604 rows), 1 = sub-columns of 16 x 16 blocks on MFMA
+ * (default).  Process-wide. */
 int mi_set_panel_engine(int which);
 int mi_dpotrf_step_trsm(mi_ctx_t *ctx, int N, int NB, double *dT, int k);
 int mi_dpotrf_step_update(mi_ctx_t *ctx, int N, int NB, double *dT, int k, int n_begin, int n_end);
