@@ -18,6 +18,7 @@
 #include <type_traits>
 #include "mi_common.hpp"
 #include "mi_panel.hpp"
+#include "mi_update.hpp"
 #include "dplasma_mi.h"
 
 using namespace mi;
@@ -244,8 +245,7 @@ __global__ __launch_bounds__(256) void k_trsm_panel(double *__restrict__ T, int 
 // ---------------------------------------------------------------------------
 // Trailing update on MFMA: C(m,n) -= A(m,k) A(n,k)^T for tile columns n in
 // [n_begin, n_end), rows m in [n, MT).  One workgroup = one BMX x BMX block of
-// one tile (BMX = 128, or 64 for launches too small to fill the chip); four
-// waves, each a BMX/2 quadrant as (BMX/32)^2 MFMA 16x16 tiles.
+// one tile.
 constexpr int BM = 128, BK = 16;
 
 // workgroup L of an update launch -> tile (m, n) and its 128x128 block
@@ -267,10 +267,7 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
 }
 
 // The workgroup's waves form a WR x WC grid over its BMX x BMX block, each
-// wave a (BMX/WR) x (BMX/WC) sub-block of 16x16 MFMA tiles.  Two workgroups share
-// each CU: WR x WC = 2 x 2 holds 256 registers per lane (two waves per
-// SIMD); 4 x 2 holds 128 (four waves per SIMD), so that a workgroup waiting
-// at a barrier or on memory still leaves two waves per SIMD issuing.
+// wave a (BMX/WR) x (BMX/WC) sub-block of 16x16 MFMA tiles.
 // One block: C(r_base.., c_base..) -= A(r_base.., 0:K) B(c_base.., 0:K)^T, all
 // of them column-major with leading dimension NB; rows_m / cols_n bound the
 // rows of A and C / the rows of B and columns of C; diag: only row >= column.
@@ -429,46 +426,89 @@ __device__ __forceinline__ int xcd_block()
     return (bid < G8) ? (bid % 8) * (G8 / 8) + bid / 8 : bid;
 }
 
-template <class T, int BMX, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__ Tt, int N, int NB, int MT, int k,
-                                                                int n_begin, int m_off, int nsub)
-{
-    int m, n, bm, bn;
-    decode_block(xcd_block(), nsub, n_begin, m_off, MT, &m, &n, &bm, &bn);
-    if (m == n && bm < bn) return;                 // strictly upper blocks of a diagonal tile
-    const int rows_m = tile_rows(N, NB, MT, m);
-    const int cols_n = tile_rows(N, NB, MT, n);
-    const int r_base = bm * BMX, c_base = bn * BMX;
-    if (r_base >= rows_m || c_base >= cols_n) return;
-    const int64_t sz = (int64_t)NB * NB;
-    update_block<T, BMX, WR, WC>(Tt + tile_index(MT, m, k) * sz, Tt + tile_index(MT, n, k) * sz,
-                                 Tt + tile_index(MT, m, n) * sz, NB, NB, rows_m, cols_n, r_base, c_base,
-                                 m == n && bm == bn);
-}
-
-// Inside tile column k, after its columns c0 .. c0 + w - 1 are solved: the
-// columns from c0 + w on lose X X_k^T (K = w), X the solved rows of each tile
-// and X_k those of tile (k, k).  The first g0 block rows are those of tile
-// (k, k) below c0 + w (lower part), then gr block rows of each tile m0, m0 +
-// 1, ...; nc blocks a block row.
-template <class T, int BMX, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC, 2) void k_panel_update(T *__restrict__ Tt, int N, int NB, int MT, int k,
-                                                                 int c0, int w, int g0, int gr, int nc, int m0)
+// The whole tiles' update, and inside tile column k, after its columns c0 ..
+// c0 + w - 1 are solved, that of the columns from c0 + w on (K = w): X the
+// solved rows of each tile, X_k those of tile (k, k).  Of the latter's blocks
+// the first g0 block rows are those of tile (k, k) below c0 + w (lower part),
+// then gr block rows of each tile m0, m0 + 1, ...; nc blocks a block row.
+struct UpdArgs {
+    int N, NB, MT, k;
+    int n_begin, m_off, nsub;                      // whole tiles
+    int c0, w, g0, gr, nc, m0;                     // panel (w > 0)
+};
+// Workgroup -> block; false: nothing to do.
+__device__ __forceinline__ bool update_decode(const UpdArgs &u, int BMX, int *m, int *n, int *r_base, int *c_base,
+                                              int *rows_m, int *cols_n, bool *diag)
 {
     const int L = xcd_block();
-    const int rb = L / nc, bn = L - rb * nc;
-    const int c1 = c0 + w;
-    const int m = rb < g0 ? k : m0 + (rb - g0) / gr;
-    if (rb < g0 && rb < bn) return;
-    const int r_base = rb < g0 ? c1 + BMX * rb : BMX * ((rb - g0) % gr), c_base = c1 + BMX * bn;
-    const int rows_m = tile_rows(N, NB, MT, m);
-    const int cols_n = tile_rows(N, NB, MT, k);
-    if (r_base >= rows_m || c_base >= cols_n) return;
-    const int64_t sz = (int64_t)NB * NB;
-    T *Cp = Tt + tile_index(MT, m, k) * sz;
-    update_block<T, BMX, WR, WC>(Cp + (int64_t)c0 * NB, Tt + tile_index(MT, k, k) * sz + (int64_t)c0 * NB, Cp, NB, w,
-                                 rows_m, cols_n, r_base, c_base, rb == bn && rb < g0);
+    if (u.w > 0) {
+        const int rb = L / u.nc, bn = L - rb * u.nc;
+        const bool own = rb < u.g0;
+        if (own && rb < bn) return false;
+        *m = own ? u.k : u.m0 + (rb - u.g0) / u.gr;
+        *n = u.k;
+        *r_base = own ? u.c0 + u.w + BMX * rb : BMX * ((rb - u.g0) % u.gr);
+        *c_base = u.c0 + u.w + BMX * bn;
+        *diag = own && rb == bn;
+    } else {
+        int bm, bn;
+        decode_block(L, u.nsub, u.n_begin, u.m_off, u.MT, m, n, &bm, &bn);
+        if (*m == *n && bm < bn) return false;     // strictly upper blocks of a diagonal tile
+        *r_base = bm * BMX;
+        *c_base = bn * BMX;
+        *diag = *m == *n && bm == bn;
+    }
+    *rows_m = tile_rows(u.N, u.NB, u.MT, *m);
+    *cols_n = tile_rows(u.N, u.NB, u.MT, *n);
+    return *r_base < *rows_m && *c_base < *cols_n;
 }
+
+// operands staged through registers: any leading dimension and alignment
+template <class T, int BMX, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__ Tt, UpdArgs u)
+{
+    int m, n, r_base, c_base, rows_m, cols_n;
+    bool diag;
+    if (!update_decode(u, BMX, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
+    const int64_t sz = (int64_t)u.NB * u.NB, off = (int64_t)u.c0 * u.NB;
+    update_block<T, BMX, WR, WC>(Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
+                                 Tt + tile_index(u.MT, m, n) * sz, u.NB, u.w > 0 ? u.w : u.NB, rows_m, cols_n, r_base,
+                                 c_base, diag);
+}
+
+// operands straight into LDS (mi_update.hpp)
+template <class S, class T, int OCC>
+__global__ __launch_bounds__(S::NT, OCC) void k_update_lds(T *__restrict__ Tt, UpdArgs u)
+{
+    __shared__ __align__(1024) unsigned char lds[S::LDS];
+    int m, n, r_base, c_base, rows_m, cols_n;
+    bool diag;
+    if (!update_decode(u, S::BM, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
+    const int64_t sz = (int64_t)u.NB * u.NB, off = (int64_t)u.c0 * u.NB;
+    update_block_lds<S, T>(lds, Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
+                           Tt + tile_index(u.MT, m, n) * sz, u.NB, u.w > 0 ? u.w : u.NB, rows_m, cols_n, r_base,
+                           c_base, diag);
+}
+// Shapes, by the step-0 update of N = 32768, NB = 512 (1953 tiles) alone, all
+// with the C vectors taken in late (register-staged before: FP64 64.8 TF, FP32
+// 121 TF; a library product of 16384 reaches 74 and 153 TF):
+//   FP64  2 x 4 waves, BK 16 x 2: 69.7 TF; BK 8 x 4: 68.1; 2 x 2 waves, BK 8
+//         x 4: 68.2
+//   FP32  2 x 2 waves, BK 16 x 4: 130 TF; x 3 and three workgroups a CU: 123;
+//         BK 16 x 2 and four: 120; BK 32 x 2: 126
+// and of N = 4096, NB = 256 (64 x 64 blocks, 37.3 / 58.5 TF before): BK 16 x
+// 3: 41.3 / 62.6 TF, x 4: 39.6 / 61.2, BK 8 x 8: 38.3 / 60.9.
+template <class T> struct UpdShapes;
+template <> struct UpdShapes<double> {
+    typedef UpdShape<double, 128, 2, 4, 16, 2, 2, 2> big;
+    typedef UpdShape<double, 64, 2, 2, 16, 3, 2, 1> small;
+    static constexpr int occ = 4;
+};
+template <> struct UpdShapes<float> {
+    typedef UpdShape<float, 128, 2, 2, 16, 4, 4, 4> big;
+    typedef UpdShape<float, 64, 2, 2, 16, 3, 2, 1> small;
+    static constexpr int occ = 2;
+};
 
 // ---------------------------------------------------------------------------
 // FP32 trailing update on BF16 MFMA with a two-term split of both operands
@@ -1054,9 +1094,6 @@ __global__ void k_fill_int(int *p, int v, int n)
 int g_panel_kernel = 1;
 // trailing-update engine: 0 = FP64 VALU, 1 = MFMA (default)
 int g_update_kernel = -1;
-// waves per workgroup of the 128x128 MFMA update: 4 (2 x 2) or 8 (4 x 2);
-// 0 = not yet read from the environment (DPLASMA_MI_UPDATE_WAVES)
-int g_update_waves = 0;
 // FP32 trailing update of mi_spotrf_tiles and the FP32 step launches: 0 =
 // FP32 MFMA (default), 1 = BF16 MFMA, two-term split (the mixed solve passes
 // its choice as an argument instead)
@@ -1089,6 +1126,33 @@ template <> struct KN<float> {
 };
 
 template <class T> bool valu_panel() { return std::is_same<T, double>::value && g_panel_kernel == 0; }
+
+// Launch the update blocks of u (K contraction columns) with the block side
+// that suits the launch; grid(bm) sets u for blocks of bm and returns their
+// number.
+template <class T, class G>
+int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, double by, T *dT, UpdArgs &u, int K,
+                         const G &grid)
+{
+    typedef typename UpdShapes<T>::big Big;
+    typedef typename UpdShapes<T>::small Small;
+    constexpr int occ = UpdShapes<T>::occ;
+    // a launch of fewer than two 128 x 128 blocks per CU leaves the chip
+    // idle: 64 x 64 blocks give four times the workgroups at a quarter of
+    // the chain
+    int64_t g = grid(Big::BM);
+    const bool big = g >= 512 && update_lds_ok<Big>(dT, u.NB, K);
+    if (!big) g = grid(Small::BM);
+    if (g > 0x7fffffff) { set_error("update grid too large"); return -3; }
+    if (g <= 0) return 0;
+    if (big)
+        MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Big, T, occ><<<(unsigned)g, Big::NT, 0, s>>>(dT, u)));
+    else if (update_lds_ok<Small>(dT, u.NB, K))
+        MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Small, T, 2><<<(unsigned)g, Small::NT, 0, s>>>(dT, u)));
+    else
+        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, 64, 2, 2><<<(unsigned)g, 256, 0, s>>>(dT, u)));
+    return 0;
+}
 
 // Largest diagonal tile (or sub-tile, where hmb re-tiles it) that the entry
 // points take: what one workgroup's LDS held when a whole tile was factored
@@ -1163,24 +1227,17 @@ int launch_panel(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k, T *
             MI_LAUNCH(c, s, KN<T>::trsm, rows * w * w, 2.0 * rows * w * sizeof(T),
                       k_panel_solve<T><<<g0 + gt * ntile, 256, 0, s>>>(dT, N, NB, MT, k, c0, w, op, g0, gt, m0));
         if (c1 >= n || (!diag && ntile <= 0)) continue;
-        // 128 x 128 blocks once they fill the chip twice over
-        auto grid = [&](int bm, int *b0, int *br, int *nc) {
-            *b0 = diag ? (n - c1 + bm - 1) / bm : 0;
-            *br = (NB + bm - 1) / bm;
-            *nc = (n - c1 + bm - 1) / bm;
-            return (*b0 + *br * ntile) * *nc;
-        };
-        int b0, br, nc;
         const double fl = 2.0 * below * w * (n - c1) + (diag ? (double)w * (n - c1) * (n - c1 + 1.0) : 0.0);
         const double by = (below + (diag ? 0.5 * (n - c1) : 0.0)) * (2.0 * (n - c1) + w) * sizeof(T);
-        if (grid(BM, &b0, &br, &nc) >= 512)
-            MI_LAUNCH(c, s, KN<T>::panel_update, fl, by,
-                      (k_panel_update<T, BM, 4, 2><<<grid(BM, &b0, &br, &nc), 512, 0, s>>>(dT, N, NB, MT, k, c0, w, b0,
-                                                                                          br, nc, m0)));
-        else
-            MI_LAUNCH(c, s, KN<T>::panel_update, fl, by,
-                      (k_panel_update<T, 64, 2, 2><<<grid(64, &b0, &br, &nc), 256, 0, s>>>(dT, N, NB, MT, k, c0, w, b0,
-                                                                                          br, nc, m0)));
+        UpdArgs u{N, NB, MT, k, 0, 0, 0, c0, w, 0, 0, 0, m0};
+        auto grid = [&](int bm) -> int64_t {
+            u.g0 = diag ? (n - c1 + bm - 1) / bm : 0;
+            u.gr = (NB + bm - 1) / bm;
+            u.nc = (n - c1 + bm - 1) / bm;
+            return ((int64_t)u.g0 + (int64_t)u.gr * ntile) * u.nc;
+        };
+        int rc = launch_update_blocks<T>(c, s, KN<T>::panel_update, fl, by, dT, u, w, grid);
+        if (rc) return rc;
     }
     return 0;
 }
@@ -1200,23 +1257,12 @@ int launch_update_run(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k
     if (ntiles <= 0) return 0;
     int nsub = (NB + BM - 1) / BM;
     int64_t grid = ntiles * nsub * nsub;
-    // a launch of fewer than two 128x128 blocks per CU is latency-bound:
-    // 64x64 blocks give four times the workgroups at a quarter of the chain
     if (g_update_kernel < 0) {
         const char *e = getenv("DPLASMA_MI_UPDATE");
         g_update_kernel = (e && !strcmp(e, "valu")) ? 0 : 1;
     }
-    if (!g_update_waves) {
-        const char *e = getenv("DPLASMA_MI_UPDATE_WAVES");
-        g_update_waves = (e && atoi(e) == 4) ? 4 : 8;
-    }
     const bool valu = std::is_same<T, double>::value && g_update_kernel == 0;
     const bool bf16 = std::is_same<T, float>::value && bf16_split;
-    const bool small = grid < 512 && !valu && !bf16;
-    if (small) {
-        nsub = (NB + 63) / 64;
-        grid = ntiles * nsub * nsub;
-    }
     if (grid > 0x7fffffff) { set_error("update grid too large"); return -3; }
     // algorithmic flops / bytes of the covered tiles: each C tile read and
     // written once, each panel tile (m, k) the launch needs read once
@@ -1249,18 +1295,13 @@ int launch_update_run(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k
         MI_LAUNCH(c, s, la ? KN<float>::update_bf16_la : KN<float>::update_bf16, fl, by,
                   k_update_bf16x3<<<(unsigned)grid, 256, 0, s>>>((float *)dT, N, NB, MT, k, n_begin, m_off,
                                                                  nsub));
-    else if (small)
-        MI_LAUNCH(c, s, la ? KN<T>::update_la : KN<T>::update, fl, by,
-                  k_update_mfma<T, 64, 2, 2><<<(unsigned)grid, 256, 0, s>>>(dT, N, NB, MT, k, n_begin, m_off,
-                                                                            nsub));
-    else if (g_update_waves == 8)
-        MI_LAUNCH(c, s, la ? KN<T>::update_la : KN<T>::update, fl, by,
-                  k_update_mfma<T, BM, 4, 2><<<(unsigned)grid, 512, 0, s>>>(dT, N, NB, MT, k, n_begin, m_off,
-                                                                            nsub));
-    else
-        MI_LAUNCH(c, s, la ? KN<T>::update_la : KN<T>::update, fl, by,
-                  k_update_mfma<T, BM, 2, 2><<<(unsigned)grid, 256, 0, s>>>(dT, N, NB, MT, k, n_begin, m_off,
-                                                                            nsub));
+    else {
+        UpdArgs u{N, NB, MT, k, n_begin, m_off, 0, 0, 0, 0, 0, 0, 0};
+        return launch_update_blocks<T>(c, s, la ? KN<T>::update_la : KN<T>::update, fl, by, dT, u, NB, [&](int bm) {
+            u.nsub = (NB + bm - 1) / bm;
+            return ntiles * u.nsub * u.nsub;
+        });
+    }
     return 0;
 }
 
