@@ -162,6 +162,19 @@ __device__ __forceinline__ void sweep_exact(T *v, T *x, int fr, int *fail, std::
     (sweep_column_exact<C>(v, x, fr, fail), ...);
 }
 
+// x := W = L^{-1} by rows as in the sweep: v holds L (lane fr: row fr), rd the
+// reciprocal of L(fr, fr), x the identity on entry.
+template <int C, class T> __device__ __forceinline__ void invert_column(T *v, T *x, T rd)
+{
+    x[C] = x[C] * row_bcast<C>(rd);
+    fmac_rest<C + 1>(x, v[C], x[C]);
+}
+template <class T, int... C>
+__device__ __forceinline__ void invert_rows(T *v, T *x, T rd, std::integer_sequence<int, C...>)
+{
+    (invert_column<C>(v, x, rd), ...);
+}
+
 // ---------------------------------------------------------------------------
 // Cholesky factor of the n x n (n <= 128) diagonal block A (column-major,
 // ld), lower, in place: right-looking over 16-column blocks.  Eight waves;

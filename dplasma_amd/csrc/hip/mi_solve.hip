@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "mi_common.hpp"
+#include "mi_panel.hpp"
 #include "dplasma_mi.h"
 
 using namespace mi;
@@ -452,9 +453,9 @@ __global__ __launch_bounds__(256) void k_gemv_bwd(const T *__restrict__ Tt, int 
 // Forward it subtracts L(rows, block h) X(block h) for every block h < g - 1
 // as X(block h) appears; the L operands of the next block are loaded while
 // the wave waits.  Then z = W_g y with W_g the inverse of the 128 x 128
-// diagonal triangle (k_inv128, staged in LDS at the start), and, once the
+// diagonal triangle (k_wave_prep, staged in LDS at the start), and, once the
 // last block appears, x_g = z - M_g X(block g - 1) with the link matrix
-// M_g = W_g L(g, g - 1) (k_wave_link), so the chain between two workgroups
+// M_g = W_g L(g, g - 1) (k_wave_prep), so the chain between two workgroups
 // is one 128 x 128 x 16 product.  Backward mirrors it from the last block
 // with L^T, W_g^T and M_g = W_g^T L(g + 1, g)^T.  Each L element is read
 // once per sweep.  Every workgroup waits only on lower logical indices, so
@@ -510,103 +511,186 @@ __device__ inline void wv_store(T *p, T v)
     __hip_atomic_store(q, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Inverse of each 128 x 128 diagonal triangle of L (column-major, 128 x 128
-// per block g, at W128 + g * 16384) from the 32 x 32 inverses W32 of
-// k_inv_diag_blocks by doubling: W21 = -W22 L21 W11, for 32 then 64 rows.
-// Rows beyond N act as identity.  One workgroup per block.
-template <class T>
-__global__ __launch_bounds__(256) void k_inv128(const T *__restrict__ Tt, int N, int NB, int MT,
-                                               const T *__restrict__ W32, T *__restrict__ W128)
+// What the wavefront solve needs of block g of 128 rows, in one launch (one
+// workgroup of eight waves per block), on 16 x 16 blocks in the layouts of
+// mi_panel.hpp:
+//   W_g   the inverse of the diagonal triangle, column-major at W128 + g *
+//         16384: wave w inverts the diagonal block w in registers, then
+//         forms block row w of W_g^T = I L_gg^{-T} by the substitution of
+//         k_panel_solve;
+//   Mf_g  = W_g L(g, g - 1), column-major, for the forward sweep;
+//   Mb_g  = W_g^T L(g + 1, g)^T, row-major, for the backward sweep.
+// Rows and columns beyond N act as identity in L_gg and as zero elsewhere.
+// unit: the diagonal of L counts as ones.
+//
+// Bound by its chains on one CU per block: 58 us at N = 32768 in FP64, 28 us
+// at 3200 in FP32 (560 and 380 us with 32 x 32 inverses, doubling and link
+// products on the VALU in four launches).
+constexpr int PREP_NT = 512;
+constexpr int PREP_BP = DB + 2;                     // column pitch of a block of W in LDS
+template <class T> constexpr size_t prep_lds()
 {
-    __shared__ T tmp[64 * 65];
-    const int g = blockIdx.x, tid = threadIdx.x;
-    const int r0 = g * WV_RB, nblk = NB / 32;
-    T *Wg = W128 + (int64_t)g * 16384;
-    auto L = [&](int i, int j) -> T {       // L(r0 + i, r0 + j), i > j, 0 beyond N
-        return (r0 + i < N) ? *sym_elem(Tt, MT, NB, r0 + i, r0 + j) : T(0);
-    };
-    for (int e = tid; e < 16384; e += 256) {
-        const int i = e & 127, j = e >> 7;
-        const int bi = i >> 5, bj = j >> 5;
-        T v = T(0);
-        if (bi == bj) {
-            const int rc = r0 + 32 * bi;
-            if (rc < N) {
-                const int tk = rc / NB, cb = (rc - tk * NB) / 32;
-                v = W32[((int64_t)tk * nblk + cb) * 1024 + (j & 31) * 32 + (i & 31)];
-            } else {
-                v = (i == j) ? T(1) : T(0);
+    return (36 * DB * PREP_BP + 28 * OPI) * sizeof(T);
+}
+template <class T>
+__global__ __launch_bounds__(PREP_NT, 2) void k_wave_prep(const T *__restrict__ Tt, int N, int NB, int MT, int unit,
+                                                         T *__restrict__ W128, T *__restrict__ Mf, T *__restrict__ Mb)
+{
+    typedef typename MF<T>::v4 V4;
+    extern __shared__ __align__(16) unsigned char prep_smem[];
+    T *Wb = reinterpret_cast<T *>(prep_smem);       // W(i, j) blocks, i >= j: element (r, c) at [c][r]
+    T *Li = Wb + 36 * DB * PREP_BP;                 // -L(i, j), i > j, as [s][lane] operand images
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4;
+    const int g = blockIdx.x, nwg = gridDim.x, r0 = g * WV_RB;
+    auto wblk = [&](int i, int j) { return Wb + (i * (i + 1) / 2 + j) * DB * PREP_BP; };
+    auto limg = [&](int i, int j) { return Li + (i * (i - 1) / 2 + j) * OPI; };
+    // element (r, c) of the rows below or in block row g, clamped; 16-row
+    // blocks lie in one tile
+    auto base = [&](int row, int col) { return sym_elem(Tt, MT, NB, row, col); };
+
+    // the blocks below the diagonal: 28, dealt to the waves
+    for (int t = wave; t < 28; t += 8) {
+        int i = 1, rem = t;
+        while (rem >= i) { rem -= i; i++; }
+        const int row = r0 + DB * i, col = r0 + DB * rem;
+        if (row < N) {
+            const T *L = base(row, col);
+            const int rr = min(fr, N - 1 - row);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const T a = L[(int64_t)MF<T>::row(s, fk) * NB + rr];
+                limg(i, rem)[64 * s + lane] = row + fr < N ? -a : T(0);
             }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) limg(i, rem)[64 * s + lane] = T(0);
         }
-        Wg[j * 128 + i] = v;
+    }
+    // inverse of diagonal block `wave`: lane fr holds row fr of L in v, row
+    // fr of the identity in x, which becomes W(., fr)
+    {
+        const int row = r0 + DB * wave;
+        T v[DB], x[DB];
+        const T *L = base(min(row, (N - 1) & ~15), min(row, (N - 1) & ~15));
+#pragma unroll
+        for (int c = 0; c < DB; c++) {
+            const int rc = max(0, min(fr, N - 1 - row)), cc = max(0, min(c, N - 1 - row));
+            const T a = L[(int64_t)cc * NB + rc];
+            v[c] = row + fr < N && row + c < N && fr >= c ? a : (fr == c ? T(1) : T(0));
+            x[c] = fr == c ? T(1) : T(0);
+        }
+        T rd = T(1);
+        if (!unit) {
+            T d = T(1);
+#pragma unroll
+            for (int c = 0; c < DB; c++) d = fr == c ? v[c] : d;
+            rd = T(1) / d;
+        }
+        invert_rows(v, x, rd, std::make_integer_sequence<int, DB>());
+        // column fr of the block: x[c] = W(c, fr); upper part exact zeros
+        if (fk == 0) {
+#pragma unroll
+            for (int c = 0; c < DB; c++) wblk(wave, wave)[fr * PREP_BP + c] = x[c];
+        }
     }
     __syncthreads();
-    for (int h = 32; h < 128; h *= 2) {
-        for (int p = 0; p < 128; p += 2 * h) {
-            const int q = p + h;
-            // tmp = L(q.., p..) W(p.., p..)   (h x h)
-            for (int e = tid; e < h * h; e += 256) {
-                const int i = e % h, j = e / h;
-                T a = T(0);
-                for (int k = j; k < h; k++) a += L(q + i, p + k) * Wg[(p + j) * 128 + p + k];
-                tmp[j * 65 + i] = a;
-            }
-            __syncthreads();
-            // W(q.., p..) = -W(q.., q..) tmp
-            for (int e = tid; e < h * h; e += 256) {
-                const int i = e % h, j = e / h;
-                T a = T(0);
-                for (int k = 0; k <= i; k++) a += Wg[(q + k) * 128 + q + i] * tmp[j * 65 + k];
-                Wg[(p + j) * 128 + q + i] = -a;
-            }
-            __syncthreads();
-        }
-    }
-}
 
-// Link matrices M_g = op(W_g) op(L)(g, h), h the block solved just before g
-// (g - 1 forward, g + 1 backward): 128 x 128 at M + g * 16384, column-major
-// forward and row-major backward (the order in which the solve reads it).
-// op(L)(g, h)(j, k) = L(128 g + j, 128 h + k) forward, L(128 h + k, 128 g + j)
-// backward; rows beyond N are zero.  One workgroup per block; thread (k =
-// tid % 128) accumulates rows i = tid / 128 + 2 e of column k.
-template <class T, bool TRANS>
-__global__ __launch_bounds__(256) void k_wave_link(const T *__restrict__ Tt, int N, int NB, int MT,
-                                                  const T *__restrict__ W128, T *__restrict__ M)
-{
-    __shared__ T sw[128][33];     // op(W_g)(i, j0 + jj)
-    __shared__ T sl[32][129];     // op(L)(j0 + jj, k)
-    const int g = blockIdx.x, nwg = gridDim.x, tid = threadIdx.x;
-    if (TRANS ? g + 1 >= nwg : g == 0) return;
-    const int h = TRANS ? g + 1 : g - 1;
-    const T *Wg = W128 + (int64_t)g * 16384;
-    const int k = tid & 127, i0 = tid >> 7;
-    T acc[64];
+    // block row j = wave of X = W_g^T: X(j, b) = W(b, j)^T, b >= j
+    {
+        const int j = wave;
+        V4 acc[8];
 #pragma unroll
-    for (int e = 0; e < 64; e++) acc[e] = T(0);
-    for (int j0 = 0; j0 < 128; j0 += 32) {
-        for (int e = tid; e < 128 * 32; e += 256) {
-            const int i = e & 127, jj = e >> 7;
-            sw[i][jj] = TRANS ? Wg[i * 128 + j0 + jj] : Wg[(j0 + jj) * 128 + i];
-        }
-        for (int e = tid; e < 32 * 128; e += 256) {
-            const int jj = e & 31, kk = e >> 5;
-            const int row = TRANS ? 128 * h + kk : 128 * g + j0 + jj;
-            const int col = TRANS ? 128 * g + j0 + jj : 128 * h + kk;
-            sl[jj][kk] = row < N ? *sym_elem(Tt, MT, NB, row, col) : T(0);
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int jj = 0; jj < 32; jj++) {
-            const T l = sl[jj][k];
+        for (int b = 0; b < 8; b++)
 #pragma unroll
-            for (int e = 0; e < 64; e++) acc[e] += sw[i0 + 2 * e][jj] * l;
+            for (int q = 0; q < 4; q++) acc[b][q] = b == j && fr == MF<T>::row(q, fk) ? T(1) : T(0);
+        T *Wg = W128 + (int64_t)g * 16384 + (int64_t)(DB * j + fr) * 128;
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            V4 xx = {T(0), T(0), T(0), T(0)};
+            if (b >= j) {
+                // A operand W_bb(i = fr, k = row(s, fk))
+                const T *w = wblk(b, b);
+#pragma unroll
+                for (int s = 0; s < 4; s++) xx = MF<T>::mfma(w[MF<T>::row(s, fk) * PREP_BP + fr], acc[b][s], xx);
+#pragma unroll
+                for (int b2 = b + 1; b2 < 8; b2++) {
+                    const T *l = limg(b2, b) + lane;
+#pragma unroll
+                    for (int s = 0; s < 4; s++) acc[b2] = MF<T>::mfma(l[64 * s], xx[s], acc[b2]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int c = MF<T>::row(q, fk);
+                Wg[DB * b + c] = xx[q];
+                if (b > j) wblk(b, j)[fr * PREP_BP + c] = xx[q];
+            }
         }
-        __syncthreads();
     }
-    T *Mg = M + (int64_t)g * 16384;            // column-major forward, row-major backward
+    __syncthreads();
+
+    // Forward link: Mf(c, hc) = sum_r W(c, r) L(g r, h hc), h = g - 1, as
+    // D(i = hc, j = c): A(hc, r) = L(r, hc), four consecutive r a lane (slice s
+    // contracts over r = 4 fk + s), B(r, c) = W(c, r).  Wave w: columns hc of
+    // block w, all block rows of c.
+    if (g > 0) {
+        const int hc = r0 - WV_RB + DB * wave + fr;
+        T *out = Mf + (int64_t)g * 16384;
+        V4 la[8];
 #pragma unroll
-    for (int e = 0; e < 64; e++) Mg[TRANS ? (i0 + 2 * e) * 128 + k : k * 128 + i0 + 2 * e] = acc[e];
+        for (int p = 0; p < 8; p++) {
+            const int row = r0 + DB * p, rb = min(row, (N - 1) & ~15);
+            const T *L = base(rb, hc);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const T a = L[min(4 * fk + s, N - 1 - rb)];
+                la[p][s] = row + 4 * fk + s < N ? a : T(0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            V4 d = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int p = 0; p <= i; p++) {
+                const T *w = wblk(i, p) + 4 * fk * PREP_BP + fr;
+#pragma unroll
+                for (int s = 0; s < 4; s++) d = MF<T>::mfma(la[p][s], w[s * PREP_BP], d);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) out[(DB * wave + MF<T>::row(q, fk)) * 128 + DB * i + fr] = d[q];
+        }
+    }
+    // Backward link: Mb(r, kk) = sum_i W(i, r) L(h kk, g i), h = g + 1, as
+    // D(i = r, j = kk): A(r, i) = W(i, r), B(i, kk) = L(kk, i).  Wave w:
+    // columns kk of block w, all block rows of r.
+    if (g + 1 < nwg) {
+        const int kk = r0 + WV_RB + DB * wave + fr;
+        T *out = Mb + (int64_t)g * 16384;
+        V4 lb[8];
+#pragma unroll
+        for (int p = 0; p < 8; p++) {
+            const T *L = base(min(kk, N - 1), r0 + DB * p);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const T a = L[(int64_t)MF<T>::row(s, fk) * NB];
+                lb[p][s] = kk < N ? a : T(0);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            V4 d = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int p = j; p < 8; p++) {
+                const T *w = wblk(p, j) + fr * PREP_BP;
+#pragma unroll
+                for (int s = 0; s < 4; s++) d = MF<T>::mfma(w[MF<T>::row(s, fk)], lb[p][s], d);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) out[(DB * j + MF<T>::row(q, fk)) * 128 + DB * wave + fr] = d[q];
+        }
+    }
 }
 
 // Index mappings of the wavefront solve.  The NW waves of a workgroup own
@@ -1179,19 +1263,17 @@ int trsm_prepare(Ctx *c, hipStream_t s, int unit, int N, int NB, const T *dT, T 
 {
     const int MT = (N + NB - 1) / NB;
     const int nblk = (NB + 31) / 32;
-    MI_LAUNCH(c, s, SN<T>::inv, (double)MT * NB * 32 * 32 / 3.0, (double)MT * NB * 32 * 2.0 * sizeof(T),
-              k_inv_diag_blocks<T><<<MT * nblk, 32, 0, s>>>(dT, N, NB, MT, unit, W));
     if (NB % 32 == 0 && g_wave_solve) {
         const int nwg = (N + WV_RB - 1) / WV_RB;
         T *W128 = W + (size_t)MT * nblk * 1024;
-        MI_LAUNCH(c, s, SN<T>::inv, (double)nwg * 128 * 128 * 128 / 3.0, (double)nwg * 16384 * 2.0 * sizeof(T),
-                  k_inv128<T><<<nwg, 256, 0, s>>>(dT, N, NB, MT, W, W128));
         T *Mf = W128 + (size_t)nwg * 16384, *Mb = Mf + (size_t)nwg * 16384;
-        MI_LAUNCH(c, s, SN<T>::link, (double)nwg * 128 * 128 * 128, (double)nwg * 16384 * 3.0 * sizeof(T),
-                  k_wave_link<T, false><<<nwg, 256, 0, s>>>(dT, N, NB, MT, W128, Mf));
-        MI_LAUNCH(c, s, SN<T>::link, (double)nwg * 128 * 128 * 128, (double)nwg * 16384 * 3.0 * sizeof(T),
-                  k_wave_link<T, true><<<nwg, 256, 0, s>>>(dT, N, NB, MT, W128, Mb));
+        if (int rc = set_lds((const void *)k_wave_prep<T>, prep_lds<T>())) return rc;
+        MI_LAUNCH(c, s, SN<T>::link, (double)nwg * 128 * 128 * 128 * (2.0 + 1.0 / 3.0), (double)nwg * 16384 * 5.5 * sizeof(T),
+                  k_wave_prep<T><<<nwg, PREP_NT, prep_lds<T>(), s>>>(dT, N, NB, MT, unit, W128, Mf, Mb));
+        return 0;
     }
+    MI_LAUNCH(c, s, SN<T>::inv, (double)MT * NB * 32 * 32 / 3.0, (double)MT * NB * 32 * 2.0 * sizeof(T),
+              k_inv_diag_blocks<T><<<MT * nblk, 32, 0, s>>>(dT, N, NB, MT, unit, W));
     return 0;
 }
 

@@ -137,3 +137,43 @@ def test_update_shapes(dev, po, N, NB, shift, dtype):
             assert (np.abs(g[:tm, :tn] - exp) <= tol)[low].all()
             assert np.array_equal(g[:tm, :tn][~low], C[:tm, :tn][~low])
             assert np.array_equal(g[tm:], C[tm:])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("unit", [False, True])
+@pytest.mark.parametrize("trans", [111, 112])
+@pytest.mark.parametrize("N,NB", [(1, 32), (15, 32), (17, 32), (127, 128), (129, 96), (145, 160), (257, 64),
+                                  (400, 160), (529, 512)])
+def test_wavefront_inverses_at_block_edges(dev, po, N, NB, trans, unit, dtype):
+    """The 128-row inverses and link matrices of the wavefront solve, ragged
+    in every way; the strict upper triangles and padding hold NaN.  With
+    |off-diagonal| <= 1 / N and a diagonal in [1, 2] the inverse's entries
+    stay below 2, so x is within a few N eps of the exact one."""
+    print(f"wave N={N} NB={NB} {trans} {unit} {dtype.__name__}", flush=True)
+    rng = np.random.default_rng(N + NB)
+    A = rng.uniform(-1.0, 1.0, (N, N)) / N
+    A[np.diag_indices(N)] = 1.0 + rng.uniform(0.0, 1.0, N)
+    L = np.tril(A).astype(dtype).astype(np.float64)
+    T = po.full_to_symtiles(L, NB).astype(dtype)
+    MT = (N + NB - 1) // NB
+    for n in range(MT):
+        for m in range(n, MT):
+            i = n * MT - n * (n - 1) // 2 + (m - n)
+            t = T[i * NB * NB:(i + 1) * NB * NB].reshape((NB, NB), order="F")
+            tm, tn = min(NB, N - m * NB), min(NB, N - n * NB)
+            t[tm:, :] = np.nan
+            t[:, tn:] = np.nan
+            if m == n:
+                t[np.triu_indices(tm, 1)] = np.nan
+    B = rng.uniform(-1.0, 1.0, (N, 3)).astype(dtype)
+    dT, dB = dev.upload(T), dev.upload(np.asfortranarray(B).reshape(-1, order="F"))
+    fn = dev.M.mi_dtrsm_LL if dtype == np.float64 else dev.M.mi_strsm_LL
+    dev.check(fn(dev.h, trans, 132 if unit else 131, 1.0, N, NB, dT, 3, dB, N), "trsm")
+    x = dev.download(dB, (N * 3,), dtype).reshape((N, 3), order="F").astype(np.float64)
+    dev.free(dT)
+    dev.free(dB)
+    if unit:
+        L[np.diag_indices(N)] = 1.0
+    ref = np.linalg.solve(L.T if trans == 112 else L, B.astype(np.float64))
+    eps = 2.0 ** -53 if dtype == np.float64 else EPS32
+    assert np.abs(x - ref).max() <= 16 * (N + 16) * eps * max(1.0, np.abs(ref).max())
