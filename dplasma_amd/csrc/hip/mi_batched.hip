@@ -1,5 +1,5 @@
 // mi_batched.hip -- many independent SPD systems of uneven sizes, factored
-// and solved in one persistent launch (captured in a hipGraph for replay).
+// and solved in persistent launches (captured in a hipGraph for replay).
 //
 // No counterpart in the reference (its batching growth path: each matrix
 // is dplasma_dposv, src/zposv_wrapper.c:63-113, on one tile; the per-matrix
@@ -11,440 +11,479 @@
 // sum_{j<i} n_j^2 of one buffer; its right-hand side (NRHS = 1) at offset
 // sum_{j<i} n_j of another.  n_i <= 1024.
 //
-// Kernel: gridDim = (workgroups per CU) x CUs workgroups of 4 waves; each
-// takes matrices from a queue (one atomic counter) in decreasing size order
-// (longest first, which bounds the imbalance by the last small matrices) and
-// factors one matrix with all its waves, left-looking over 32-column panels:
-//   1. panel update C -= L(j:n, 0:j) L(j:j+32, 0:j)^T on MFMA, strips of SH
-//      rows staged through LDS in K chunks of 32;
-//   2. the 32x32 diagonal block factored and inverted (W = L_jj^-1) by wave
-//      0 in one register sweep (one v_readlane broadcast per column);
-//   3. the rows below: X = C W^T on MFMA;
-// then the two triangular solves, 32 rows at a time (partial sums by all
-// waves, the 32-row substitution by wave 0).
-// Two strip heights are compiled (SH = 64 and 128): matrices with
-// n <= nsplit take SH = 64.  nsplit and the workgroups per CU are the tile
-// shape the autotuner picks (mi_batch_autotune).
+// A workgroup takes matrices from a queue (one atomic counter) in decreasing
+// size order (longest first, which bounds the imbalance by the last small
+// matrices) and factors one matrix with all its NW waves, left-looking over
+// panels of 16 NW columns, on 16 x 16 blocks in the accumulator layout of
+// mi_panel.hpp:
+//   1. the panel's diagonal block rows (one a wave) lose the products with
+//      every column to the left, then diag_factor factors the block and leaves
+//      the images of -L and W in LDS;
+//   2. the other block rows, RT a wave at a time, do the same product and are
+//      solved against these images, in registers from load to store.
+// In these products a wave's own rows are MFMA operands straight from memory;
+// the panel's rows are staged through LDS for all waves.
+// The right-hand side is carried along like one more row below the matrix (y,
+// kept in LDS), so the forward solve comes with the factorization; the
+// backward solve then goes through the panels from the last.
+// Three instances: matrices above 128 (panels of 128), those of at most 128
+// and of at most 64 (one panel, and more workgroups per CU).
+//
+// Measured (512 matrices of one order with solve, FP64 / FP32 ms; in brackets
+// 64- or 128-wide panels of 32-column blocks from memory, factored by
+// v_readlane broadcasts, and a separate solve): n = 1024 5.16 / 2.55 (9.11 /
+// 4.69), 512 0.96 / 0.47 (2.02 / 1.02), 256 0.25 / 0.12 (0.53 / 0.31), 128
+// 0.084 / 0.045 (0.150 / 0.116), 32 0.028 / 0.023 (0.042 / 0.038); 4096 of
+// 32..1024 14.2 / 6.8 (26.0 / 13.7).  Bound at n = 1024 by the products to the
+// left (4.2 us a stage of a full pass, 3.4 us of it MFMA; half-empty last
+// passes), below 256 by the chain of pivots (diag_factor).
 #include <algorithm>
 #include <numeric>
 #include <vector>
 
 #include "mi_common.hpp"
+#include "mi_panel.hpp"
 #include "dplasma_mi.h"
 
 using namespace mi;
 
 namespace {
 
-constexpr int BW = 32;            // diagonal block / panel-solve width
-// width of the panel the long update covers: 64 in FP64 (two workgroups of
-// 76 KB LDS per CU), 128 in FP32 (42 -> 50 KB; in FP64 the 92 KB it needs
-// would leave one workgroup per CU: 36.3 against 28.8 ms for the batch)
-template <class T> constexpr int panel_width() { return sizeof(T) == 8 ? 64 : 128; }
 constexpr int BMAX = 1024;        // largest matrix order of a batch
+constexpr int BKC = 16;           // columns to the left per stage
 
-// A[i] where c holds, +0 elsewhere; ic is i clamped into the matrix.  In
-// FP64 the load reads ic, a valid address, whatever c is: the compiler then
-// issues the loads of a whole staging group together instead of branching
-// around each one and waiting for it on its own (batch 28.7 -> 21.3 ms).  In
-// FP32 that raises the register spills (0 -> 186) and costs more than it
-// gains (19.1 -> 26.1 ms), so there the load stays conditional on c.
-template <class T> __device__ __forceinline__ T mload(const T *A, int ic, int i, bool c)
-{
-    if constexpr (sizeof(T) == 8) {
-        const T v = A[ic];                        // read whatever c is
-        return c ? v : T(0);
-    } else {
-        return c ? A[i] : T(0);
-    }
-}
-
-template <class T, int SH, int BWC>
-struct BLds {
-    static constexpr int LPA = SH + 128 / (int)sizeof(T);
-    static constexpr int LPB = BWC + 128 / (int)sizeof(T);
-};
-
-template <class T>
-struct BShared {
-    T sa[BW * (128 + 128 / sizeof(T))];   // -L rows of the strip, [kk][row]
-    T sb[BW * (panel_width<T>() + 128 / sizeof(T))];   // L rows of the panel's columns, [kk][col]
-    T ws[BW][BW + 1];                     // its inverse
-    T ys[BMAX];                           // solve vector
-    T red[8][BW];
+template <class T, int NW, bool MULTI> struct BShared {
+    static constexpr int PW = DB * NW;                   // panel columns
+    static constexpr int WP = DIAG_WP;
+    T img[NW * (NW - 1) / 2][OPI];                       // -L(i, j), i > j, of the current panel
+    T w[NW][DB * WP];                                    // W_p, image column t at t WP
+    DiagLds<T> ds;
+    T bs[MULTI ? 2 : 1][MULTI ? BKC : 1][PW + 128 / sizeof(T)];   // staged rows of the panel, [k][row]
+    T ys[MULTI ? BMAX : PW];                             // y, then x
+    T ts[PW];                                            // right-hand side of a panel's solve
+    T red[4][MULTI ? PW : 1];                            // partial sums
     int idx;
-    int fail;
 };
 
-// 1. C(0:M, 0:jb) -= L(j0:n, k0:k1) L(j0:j0+jb, k0:k1)^T, C = A(j0:n, j0:j0+jb),
-// jb <= BWC (k0, k1 multiples of 32): the long update of a panel of BWC
-// columns over every column left of it (k0 = 0, k1 = j0), or the update of
-// the second half of a 64-wide panel by its first half
-template <class T, int SH, int BWC>
-__device__ void panel_update(T *__restrict__ A, int n, int j0, int jb, int k0, int k1, BShared<T> &sh)
+// v summed over each row of 16 lanes, in every lane of the row
+template <class T> __device__ __forceinline__ T row_sum(T v)
 {
-    typedef typename MF<T>::v4 V4;
-    constexpr int LPA = BLds<T, SH, BWC>::LPA, LPB = BLds<T, SH, BWC>::LPB;
-    constexpr int TC = BWC / 16;                // 16-column MFMA tiles
-    constexpr int NB_ = BWC * BW / 256;         // staged B elements per thread
-    constexpr int TW = SH / 64;                 // 16-row MFMA tiles per wave
-    constexpr int NA = SH * BW / 256;           // staged A elements per thread
-    // opaque per call: offsets derived from tid are recomputed here instead
-    // of being held live across the caller's loops
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fk = lane >> 4;
-    const int M = n - j0;
-    const int lda = n;   // n <= 1024: 32-bit offsets
-    for (int s = 0; s < M; s += SH) {
-        V4 acc[TW][TC];
-#pragma unroll
-        for (int i = 0; i < TW; i++)
-#pragma unroll
-            for (int jj = 0; jj < TC; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int row = s + wave * (SH / 4) + i * 16 + fr;
-                    const int col = jj * 16 + MF<T>::row(q, fk);
-                    acc[i][jj][q] = mload(A, (j0 + min(col, jb - 1)) * lda + j0 + min(row, M - 1),
-                                          (j0 + col) * lda + j0 + row, row < M && col < jb && row >= col);
-                }
-        T ra[NA], rb[NB_];
-        auto gload = [&](int kc) {
-#pragma unroll
-            for (int p = 0; p < NA; p++) {
-                const int e = tid + 256 * p, kk = e / SH, r = e - kk * SH;
-                ra[p] = -mload(A, (kc + kk) * lda + j0 + min(s + r, M - 1), (kc + kk) * lda + j0 + s + r, s + r < M);
-            }
-#pragma unroll
-            for (int p = 0; p < NB_; p++) {
-                const int e = tid + 256 * p, kk = e / BWC, c = e - kk * BWC;
-                rb[p] = mload(A, (kc + kk) * lda + j0 + min(c, jb - 1), (kc + kk) * lda + j0 + c, c < jb);
-            }
-        };
-        auto lstore = [&]() {
-#pragma unroll
-            for (int p = 0; p < NA; p++) {
-                const int e = tid + 256 * p, kk = e / SH, r = e - kk * SH;
-                sh.sa[kk * LPA + r] = ra[p];
-            }
-#pragma unroll
-            for (int p = 0; p < NB_; p++) {
-                const int e = tid + 256 * p, kk = e / BWC, c = e - kk * BWC;
-                sh.sb[kk * LPB + c] = rb[p];
-            }
-        };
-        if (k0 < k1) gload(k0);
-        for (int kc = k0; kc < k1; kc += BW) {
-            __syncthreads();                    // previous chunk consumed
-            lstore();
-            __syncthreads();
-            if (kc + BW < k1) gload(kc + BW);
-#pragma unroll
-            for (int kq = 0; kq < BW / 4; kq++) {
-                const int kk = kq * 4 + fk;
-                T a[TW], b[TC];
-#pragma unroll
-                for (int i = 0; i < TW; i++) a[i] = sh.sa[kk * LPA + wave * (SH / 4) + i * 16 + fr];
-#pragma unroll
-                for (int jj = 0; jj < TC; jj++) b[jj] = sh.sb[kk * LPB + jj * 16 + fr];
-#pragma unroll
-                for (int i = 0; i < TW; i++)
-#pragma unroll
-                    for (int jj = 0; jj < TC; jj++) acc[i][jj] = MF<T>::mfma(b[jj], a[i], acc[i][jj]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < TW; i++)
-#pragma unroll
-            for (int jj = 0; jj < TC; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int row = s + wave * (SH / 4) + i * 16 + fr;
-                    const int col = jj * 16 + MF<T>::row(q, fk);
-                    if (row < M && col < jb && row >= col) A[(j0 + col) * lda + j0 + row] = acc[i][jj][q];
-                }
-    }
+    v += row_rotate<8>(v);
+    v += row_rotate<4>(v);
+    v += row_rotate<2>(v);
+    v += row_rotate<1>(v);
+    return v;
 }
 
-// 2. factor the diagonal block and invert it in one register sweep of wave
-// 0: lanes 0-31 hold rows of the block and become L_jj, lanes 32-63 hold
-// the rows of the identity and become the columns of W = L_jj^-1 (the same
-// eliminations applied to [L | I]).  Returns the 1-based column of the first
-// non-positive pivot within the block, or 0.
-template <class T>
-__device__ __forceinline__ int diag_block(T *__restrict__ A, int n, int j0, int jb, BShared<T> &sh)
-{
-    const int tid = threadIdx.x;
-    const int lda = n;   // n <= 1024: 32-bit offsets
-    if (tid < 64) {
-        int fail = 0;
-        int r = tid;
-        // opaque to the optimizer: keeps the 32 identity tests below from
-        // being hoisted out of the caller's panel loop into live registers
-        asm volatile("" : "+v"(r));
-        const bool lrow = r < BW;
-        const int jw = r - BW;
-        T v[BW];
-        const int rc = min(r, jb - 1);
+template <class T, int NW, int RT, bool MULTI> struct Batch {
+    typedef typename MF<T>::v4 V4;
+    typedef BShared<T, NW, MULTI> SH;
+    static constexpr int PW = SH::PW;
+    SH &sh;
+    int lane, wave, fr, fk;
+
+    __device__ __forceinline__ explicit Batch(SH &s) : sh(s) { refresh(); }
+    // The lane's coordinates, opaque to the compiler from here on: what it
+    // derives from them (addresses, conditions per block) is computed where it
+    // is used instead of being held across the caller's loops.
+    __device__ __forceinline__ void refresh()
+    {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        lane = tid & 63;
+        wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        asm volatile("" : "+s"(wave));
+        fr = lane & 15;
+        fk = lane >> 4;
+    }
+    __device__ __forceinline__ T *limg(int i, int j) { return sh.img[i * (i - 1) / 2 + j]; }
+    __device__ __forceinline__ V4 get_w(int p)
+    {
+        V4 w;
 #pragma unroll
-        for (int c = 0; c < BW; c++) {
-            const bool ld = lrow && r < jb && c < jb && c <= r;
-            const T a = mload(A, (j0 + min(c, jb - 1)) * lda + j0 + rc, (j0 + c) * lda + j0 + r, ld);
-            const T id = lrow ? ((r == c) ? T(1) : T(0)) : ((c == jw) ? T(1) : T(0));
-            v[c] = ld ? a : id;
+        for (int q = 0; q < 4; q++) w[q] = sh.w[p][(4 * q + fk) * SH::WP + fr];
+        return w;
+    }
+    // x[c] = W(c, fr) of block p, in the lanes of the first row
+    __device__ __forceinline__ void put_w(int p, const T *x)
+    {
+        const int t = sizeof(T) == 8 ? fr : 4 * (fr & 3) + (fr >> 2);
+        if (fk == 0) {
+#pragma unroll
+            for (int c = 0; c < DB; c++) sh.w[p][t * SH::WP + c] = x[c];
         }
+    }
+    __device__ __forceinline__ static V4 mul(const V4 &a, const V4 &b, V4 c)
+    {
 #pragma unroll
-        for (int c = 0; c < BW; c++) {
-            const T piv = readlane_t(v[c], c);
-            if (!(piv > T(0)) && fail == 0) fail = c + 1;
-            const T d = sqrt(piv > T(0) ? piv : T(1));
-            const T rd = T(1) / d;
-            const T sc = v[c] * rd;
-            const T m = (!lrow || r > c) ? sc : T(0);
-            v[c] = lrow ? (r == c ? d : (r > c ? sc : v[c])) : sc;
+        for (int s = 0; s < 4; s++) c = MF<T>::mfma(a[s], b[s], c);
+        return c;
+    }
+    __device__ __forceinline__ V4 get(const T *img)
+    {
+        V4 v;
 #pragma unroll
-            for (int c2 = c + 1; c2 < BW; c2++) {
-                v[c2] -= m * readlane_t(m, c2);
-                // at most four broadcasts in flight: keeps the scalar
-                // registers they land in from piling up (fewer spills)
-                if ((c2 & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < 4; q++) v[q] = img[64 * q + lane];
+        return v;
+    }
+    // X = C L^{-T} for one block row, against the panel's images; put(b, X_b)
+    template <int BI, class PUT> __device__ __forceinline__ void solve_strip(V4 (&acc)[NW], int nbc, PUT &&put)
+    {
+        if constexpr (BI < NW) {
+            if (BI < nbc) {
+                __builtin_amdgcn_sched_barrier(0);
+                acc[BI] = mul(get_w(BI), acc[BI], V4{T(0), T(0), T(0), T(0)});
+#pragma unroll
+                for (int b2 = BI + 1; b2 < NW; b2++) acc[b2] = mul(get(limg(b2, BI)), acc[BI], acc[b2]);
+                put(BI, acc[BI]);
+                solve_strip<BI + 1>(acc, nbc, put);
             }
         }
-        if (r == 0) sh.fail = (fail > 0 && fail <= jb) ? fail : 0;   // wave-uniform
-        if (lrow) {
-            if (r < jb) {
+    }
+
+    // One pass over the block rows base, base + 1, .. (NW RA of them, below
+    // nrb) of the panel at p0: load, update by the columns to the left (UPD),
+    // solve against the panel's images (SOLVE), store.  The pass over the
+    // diagonal block's rows (no solve) stores their lower part, and updates
+    // the right-hand side's row into sh.ts when b.
+    template <int RA, bool UPD, bool SOLVE>
+    __device__ __forceinline__ void pass(T *__restrict__ A, int n, const T *__restrict__ b, int p0, int base, int nrb)
+    {
+        const int lda = n;                                   // n <= 1024: 32-bit offsets
+        const int ncol = min(PW, n - p0), nbc = (ncol + DB - 1) / DB;
+        refresh();
+        V4 acc[RA][NW];
+        const T *src[RA];                                    // this lane's row, clamped
 #pragma unroll
-                for (int c = 0; c < BW; c++)
-                    if (c <= r && c < jb) A[(j0 + c) * lda + j0 + r] = v[c];
+        for (int t = 0; t < RA; t++) {
+            src[t] = A + min(p0 + DB * (base + NW * t + wave) + fr, n - 1);
+#pragma unroll
+            for (int j = 0; j < NW; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) acc[t][j][q] = src[t][min(p0 + DB * j + MF<T>::row(q, fk), n - 1) * lda];
+        }
+        if constexpr (UPD) left_update<RA, !SOLVE>(A, lda, n, p0, base + wave < nrb, acc, src, b);
+        auto put = [&](int rb, int j, const V4 &v) {
+            const int r = p0 + DB * rb + fr;
+            if (r < n) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = p0 + DB * j + MF<T>::row(q, fk);
+                    if (c < n && (SOLVE || r >= c)) A[c * lda + r] = v[q];
+                }
+            }
+        };
+        if constexpr (!SOLVE) {
+            if (wave < nrb) {
+#pragma unroll
+                for (int j = 0; j < NW; j++)
+                    if (j <= wave) put(wave, j, acc[0][j]);
             }
         } else {
 #pragma unroll
-            for (int c = 0; c < BW; c++) sh.ws[c][jw] = v[c];      // W(c, jw)
-        }
-    }
-    __syncthreads();
-    const int f = sh.fail;
-    __syncthreads();
-    return f;
-}
-
-// 3. rows below the diagonal block: X = C W^T, in place
-template <class T, int SH>
-__device__ void panel_solve(T *__restrict__ A, int n, int j0, int jb, BShared<T> &sh)
-{
-    typedef typename MF<T>::v4 V4;
-    constexpr int TW = SH / 64;
-    // opaque per call: offsets derived from tid are recomputed here instead
-    // of being held live across the caller's loops
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fk = lane >> 4;
-    const int lda = n;   // n <= 1024: 32-bit offsets
-    for (int s = j0 + jb; s < n; s += SH) {
-        T a[TW][BW / 4];
-#pragma unroll
-        for (int i = 0; i < TW; i++)
-#pragma unroll
-            for (int kq = 0; kq < BW / 4; kq++) {
-                const int row = s + wave * (SH / 4) + i * 16 + fr, k = kq * 4 + fk;
-                a[i][kq] = mload(A, (j0 + min(k, jb - 1)) * lda + min(row, n - 1), (j0 + k) * lda + row, row < n && k < jb);
+            for (int t = 0; t < RA; t++) {
+                const int rb = base + NW * t + wave;
+                if (rb < nrb) solve_strip<0>(acc[t], nbc, [&](int j, const V4 &v) { put(rb, j, v); });
             }
-        V4 acc[TW][2];
-#pragma unroll
-        for (int i = 0; i < TW; i++)
-#pragma unroll
-            for (int jj = 0; jj < 2; jj++) acc[i][jj] = V4{T(0), T(0), T(0), T(0)};
-#pragma unroll
-        for (int kq = 0; kq < BW / 4; kq++) {
-            T b[2];
-#pragma unroll
-            for (int jj = 0; jj < 2; jj++) b[jj] = sh.ws[jj * 16 + fr][kq * 4 + fk];   // W^T(k, c) = W(c, k)
-#pragma unroll
-            for (int i = 0; i < TW; i++)
-#pragma unroll
-                for (int jj = 0; jj < 2; jj++) acc[i][jj] = MF<T>::mfma(b[jj], a[i][kq], acc[i][jj]);
         }
-#pragma unroll
-        for (int i = 0; i < TW; i++)
-#pragma unroll
-            for (int jj = 0; jj < 2; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int row = s + wave * (SH / 4) + i * 16 + fr;
-                    const int col = jj * 16 + MF<T>::row(q, fk);
-                    if (row < n && col < jb) A[(j0 + col) * lda + row] = acc[i][jj][q];
-                }
     }
-}
 
-// Left-looking over panels of PW = 64 (FP64) or 128 (FP32) columns: one long
-// update of the whole panel by every column left of it (the strip of L to
-// the left is streamed once per PW columns instead of once per 32), then
-// the panel's blocks of BW = 32: the update by the panel's earlier blocks,
-// diagonal block, and the rows below it.
-template <class T>
-__device__ int factor_one(T *__restrict__ A, int n, bool narrow, BShared<T> &sh)
-{
-    constexpr int PW = panel_width<T>();
-    for (int p0 = 0; p0 < n; p0 += PW) {
-        const int pb = min(PW, n - p0);
-        if (narrow) panel_update<T, 64, PW>(A, n, p0, pb, 0, p0, sh);
-        else panel_update<T, 128, PW>(A, n, p0, pb, 0, p0, sh);
+    // y(p0 ..) = (b - L(p0.., 0:p0) y) L^{-T}: the right-hand side's row against
+    // the panel's images, by the calling wave; t: its values so far
+    __device__ __forceinline__ void solve_row(const T *t, int n, int p0)
+    {
+        const int ncol = min(PW, n - p0), nbc = (ncol + DB - 1) / DB;
+        V4 acc[NW];
+#pragma unroll
+        for (int j = 0; j < NW; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                // columns past n count as zero
+                const int c = DB * j + MF<T>::row(q, fk);
+                acc[j][q] = c < ncol ? t[min(c, ncol - 1)] : T(0);
+            }
+        solve_strip<0>(acc, nbc, [&](int j, const V4 &v) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int c = p0 + DB * j + MF<T>::row(q, fk);
+                if (fr == 0 && c < n) sh.ys[c] = v[q];
+            }
+        });
+    }
+
+    // factor; y = L^{-1} b into sh.ys when b; 0 or the first bad column
+    __device__ __forceinline__ int factor(T *__restrict__ A, int n, const T *__restrict__ b)
+    {
+        for (int p0 = 0; p0 < n; p0 += PW) {
+            const int nrb = (n - p0 + DB - 1) / DB;          // block rows
+            if constexpr (MULTI) {
+                if (p0 > 0) {
+                    pass<1, true, false>(A, n, b, p0, 0, nrb);
+                    __syncthreads();
+                }
+            }
+            const int f = diag_factor<T, NW, NW>(
+                A + (int64_t)p0 * n + p0, min(PW, n - p0), n, sh.ds, [&](int i, int j) { return limg(i, j); },
+                [&](int p) { return sh.w[p]; }, [](int, const V4 &) {}, [](int, int, const V4 &) {});
+            if (f) return p0 + f;
+            if constexpr (MULTI) {
+                int base = NW;
+                if (p0 == 0) {
+                    for (; base < nrb; base += NW) pass<1, false, true>(A, n, b, p0, base, nrb);
+                } else {
+                    for (; base + NW < nrb; base += NW * RT) pass<RT, true, true>(A, n, b, p0, base, nrb);
+                    if (base < nrb) pass<1, true, true>(A, n, b, p0, base, nrb);
+                }
+            }
+            // (the wave that has the fewest rows in the last pass)
+            if (b && wave == NW - 1) solve_row(p0 > 0 ? sh.ts : b + p0, n, p0);
+            __syncthreads();
+        }
+        return 0;
+    }
+
+    // acc -= L(rows, 0:p0) L(p0.., 0:p0)^T; on: this wave has rows.  ROW: also
+    // sh.ts = b(p0..) - L(p0.., 0:p0) y, from the staged rows.
+    // One step ahead: the loads of the next stage are in flight while a stage
+    // is multiplied; in FP64 with one block row a wave (half the products, and
+    // one workgroup a CU) two.
+    template <int RA, bool ROW>
+    __device__ __forceinline__ void left_update(const T *__restrict__ A, int lda, int n, int p0, bool on,
+                                                V4 (&acc)[RA][NW], const T *const (&src)[RA], const T *__restrict__ b)
+    {
+        constexpr int EPT = PW * BKC / (64 * NW);            // staged elements of a thread
+        constexpr int KS = 64 * NW / PW;                     // columns staged at a time
+        constexpr int D = RA == 1 && sizeof(T) == 8 ? 2 : 1; // stages ahead
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));                        // offsets recomputed here, not held by the caller
+        const int sc = tid % PW, sk = tid / PW;              // row of the panel, first column
+        const T *bp = A + min(p0 + sc, n - 1);
+        const int nst = p0 / BKC;                            // a multiple of PW / BKC
+        T rb[D][EPT], a[D + 1][RA][4], dot = T(0);
+        auto load_b = [&](int st, T *x) {
+#pragma unroll
+            for (int e = 0; e < EPT; e++) x[e] = bp[(st * BKC + sk + e * KS) * lda];
+        };
+        auto store_b = [&](int buf, const T *x) {
+#pragma unroll
+            for (int e = 0; e < EPT; e++) sh.bs[buf][sk + e * KS][sc] = x[e];
+        };
+        auto load_a = [&](int st, T (*x)[4]) {
+#pragma unroll
+            for (int t = 0; t < RA; t++)
+#pragma unroll
+                for (int s = 0; s < 4; s++) x[t][s] = src[t][(st * BKC + 4 * s + fk) * lda];
+        };
+        load_b(0, rb[0]);
+        load_a(0, a[0]);
+        if constexpr (D > 1) {
+            if (nst > 1) load_a(1, a[1]);
+        }
+        store_b(0, rb[0]);
+        if constexpr (D > 1) {
+            if (nst > 1) load_b(1, rb[1]);
+        }
         __syncthreads();
-        for (int j0 = p0; j0 < p0 + pb; j0 += BW) {
-            const int jb = min(BW, n - j0);
-            if (j0 > p0) {
-                if (narrow) panel_update<T, 64, BW>(A, n, j0, jb, p0, j0, sh);
-                else panel_update<T, 128, BW>(A, n, j0, jb, p0, j0, sh);
+        // stage st from LDS half st % 2 and operand set st % (D + 1); stage
+        // st + D is loaded meanwhile
+        auto stage = [&](int st, auto ub, auto ua) {
+            constexpr int buf = decltype(ub)::value, set = decltype(ua)::value;
+            if (st + D < nst) {
+                load_b(st + D, rb[(buf + D) % D]);
+                if (on) load_a(st + D, a[(set + D) % (D + 1)]);
+            }
+            if (on) {
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    T bf[NW];
+#pragma unroll
+                    for (int j = 0; j < NW; j++) bf[j] = sh.bs[buf][4 * s + fk][DB * j + fr];
+#pragma unroll
+                    for (int j = 0; j < NW; j++)
+#pragma unroll
+                        for (int t = 0; t < RA; t++) acc[t][j] = MF<T>::mfma(bf[j], -a[set][t][s], acc[t][j]);
+                }
+            }
+            if (ROW && b) {
+#pragma unroll
+                for (int e = 0; e < EPT; e++)
+                    dot += sh.bs[buf][sk + e * KS][sc] * sh.ys[st * BKC + sk + e * KS];
+            }
+            if (st + 1 < nst) store_b(buf ^ 1, rb[(buf + 1) % D]);
+            __syncthreads();
+        };
+        typedef std::integral_constant<int, 0> I0;
+        typedef std::integral_constant<int, 1> I1;
+        typedef std::integral_constant<int, 2> I2;
+        if constexpr (D == 1) {
+            for (int st = 0; st < nst; st += 2) {
+                stage(st, I0(), I0());
+                stage(st + 1, I1(), I1());
+            }
+        } else {
+            for (int st = 0; st < nst;) {
+                stage(st++, I0(), I0());
+                stage(st++, I1(), I1());
+                if (st >= nst) break;
+                stage(st++, I0(), I2());
+                stage(st++, I1(), I0());
+                if (st >= nst) break;
+                stage(st++, I0(), I1());
+                stage(st++, I1(), I2());
+            }
+        }
+        if (ROW && b) {
+            sh.red[sk][sc] = dot;
+            __syncthreads();
+            if (sk == 0) {
+                T t = p0 + sc < n ? b[p0 + sc] : T(0);
+#pragma unroll
+                for (int e = 0; e < KS; e++) t -= sh.red[e][sc];
+                sh.ts[sc] = t;
+            }
+        }
+    }
+
+    // images of -L and W of the panel at p0 (ncol == PW), from memory
+    __device__ __forceinline__ void load_images(const T *__restrict__ A, int lda, int p0)
+    {
+        for (int u = wave; u < NW * (NW - 1) / 2; u += NW) {
+            int i = 1, j = u;
+            while (j >= i) { j -= i; i++; }
+            T *img = limg(i, j);
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                img[64 * s + lane] = -A[(p0 + DB * j + MF<T>::row(s, fk)) * lda + p0 + DB * i + fr];
+        }
+        T v[DB], x[DB];
+        T d = T(1);
+        const int c0 = p0 + DB * wave;
+#pragma unroll
+        for (int c = 0; c < DB; c++) {
+            v[c] = A[(c0 + c) * lda + c0 + fr];
+            x[c] = fr == c ? T(1) : T(0);
+            d = fr == c ? v[c] : d;
+        }
+        invert_rows(v, x, T(1) / d, std::make_integer_sequence<int, DB>());
+        put_w(wave, x);
+    }
+
+    // x = L^{-T} y, y and x in sh.ys; the last panel's images are in LDS
+    __device__ __forceinline__ void backward(const T *__restrict__ A, int n)
+    {
+        const int lda = n, last = (n - 1) / PW * PW;
+        for (int p0 = last; p0 >= 0; p0 -= PW) {
+            refresh();
+            const int ncol = min(PW, n - p0), nbc = (ncol + DB - 1) / DB;
+            if (MULTI && p0 < last) {
+                load_images(A, lda, p0);
+                // t = y - L(p0 + PW.., panel)^T x: wave w the columns of block w
+                const T *Lc = A + (int64_t)(p0 + DB * wave) * lda;
+                T s[DB];
+#pragma unroll
+                for (int c = 0; c < DB; c++) s[c] = T(0);
+                for (int r = p0 + PW; r < n; r += 64) {
+                    const int rr = min(r + lane, n - 1);
+                    const T xr = r + lane < n ? sh.ys[rr] : T(0);
+                    T l[DB];
+#pragma unroll
+                    for (int c = 0; c < DB; c++) l[c] = Lc[c * lda + rr];
+#pragma unroll
+                    for (int c = 0; c < DB; c++) s[c] += l[c] * xr;
+                }
+                T mine = T(0);
+#pragma unroll
+                for (int c = 0; c < DB; c++) {
+                    T t = row_sum(s[c]);
+                    t += __shfl_xor(t, 16);
+                    t += __shfl_xor(t, 32);
+                    mine = fr == c ? t : mine;
+                }
+                if (fk == 0) sh.ts[DB * wave + fr] = sh.ys[p0 + DB * wave + fr] - mine;
                 __syncthreads();
             }
-            const int f = diag_block<T>(A, n, j0, jb, sh);
-            if (f) return j0 + f;
-            if (narrow) panel_solve<T, 64>(A, n, j0, jb, sh);
-            else panel_solve<T, 128>(A, n, j0, jb, sh);
+            const T *t0 = MULTI && p0 < last ? sh.ts : sh.ys + p0;
+            if (wave == 0) {
+                // x_p = W_p^T (t_p - sum_{i > p} L(i, p)^T x_i): lane (fr, fk)
+                // holds element fr of a block in every fk
+                T xb[NW];
+#pragma unroll
+                for (int i = 0; i < NW; i++) xb[i] = T(0);
+#pragma unroll
+                for (int p = NW - 1; p >= 0; p--) {
+                    if (p >= nbc) continue;
+                    asm volatile("" : "+v"(lane), "+v"(fr), "+v"(fk));
+                    T s[4] = {T(0), T(0), T(0), T(0)};       // column row(q, fk)
+#pragma unroll
+                    for (int i = p + 1; i < NW; i++)
+                        if (i < nbc) {
+                            const V4 l = get(limg(i, p));
+#pragma unroll
+                            for (int q = 0; q < 4; q++) s[q] += l[q] * xb[i];
+                        }
+                    const V4 w = get_w(p);                   // W(fr, row(q, fk))
+                    T tv = T(0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        s[q] = row_sum(s[q]);
+                        // column fr of the block from the lanes that hold it
+                        const T o = __shfl(s[q], MF<T>::lane_of(fr));
+                        tv = MF<T>::slice_of(fr) == q ? o : tv;
+                    }
+                    tv += DB * p + fr < ncol ? t0[DB * p + fr] : T(0);
+                    T xv = T(0);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const T o = __shfl(row_sum(w[q] * tv), MF<T>::lane_of(fr));
+                        xv = MF<T>::slice_of(fr) == q ? o : xv;
+                    }
+                    xb[p] = xv;
+                    if (fk == 0 && DB * p + fr < ncol) sh.ys[p0 + DB * p + fr] = xv;
+                }
+            }
             __syncthreads();
         }
     }
-    return 0;
-}
+};
 
-// L L^T x = b in place (NRHS = 1)
-template <class T>
-__device__ void solve_one(const T *__restrict__ A, int n, T *__restrict__ b, BShared<T> &sh)
+template <class T, int NW, int RT, bool MULTI, int OCC>
+__global__ __launch_bounds__(64 * NW, OCC) void k_posv_batched(int count, const int *__restrict__ order,
+                                                              const int *__restrict__ nsz,
+                                                              const int64_t *__restrict__ aoff,
+                                                              const int64_t *__restrict__ boff, T *__restrict__ A,
+                                                              T *__restrict__ B, int *__restrict__ info,
+                                                              int *__restrict__ counter)
 {
-    const int tid = threadIdx.x;
-    const int lda = n;   // n <= 1024: 32-bit offsets
-    const int nblk = (n + BW - 1) / BW;
-    for (int i = tid; i < n; i += 256) sh.ys[i] = b[i];
-    __syncthreads();
-    // forward: y = L^-1 b
-    for (int bj = 0; bj < nblk; bj++) {
-        const int j0 = bj * BW, jb = min(BW, n - j0);
-        {
-            const int r = tid & 31, sl = tid >> 5;
-            T acc = T(0);
-            if (r < jb) {
-                // eight independent loads in flight per step
-                int k = sl;
-                for (; k + 56 < j0; k += 64) {
-                    T a[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) a[u] = A[(k + 8 * u) * lda + j0 + r];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) acc += a[u] * sh.ys[k + 8 * u];
-                }
-                for (; k < j0; k += 8) acc += A[k * lda + j0 + r] * sh.ys[k];
-            }
-            sh.red[sl][r] = acc;
-        }
-        __syncthreads();
-        if (tid < 64) {
-            const int r = tid;
-            T t = T(0), dg = T(1);
-            if (r < jb) {
-                t = sh.ys[j0 + r];
-                for (int sl = 0; sl < 8; sl++) t -= sh.red[sl][r];
-                dg = A[(j0 + r) * lda + j0 + r];
-            }
-            // the block's row r, loaded before the sequential substitution
-            T Lr[BW];
-#pragma unroll
-            for (int c = 0; c < BW; c++)
-                Lr[c] = mload(A, (j0 + min(c, jb - 1)) * lda + j0 + min(r, jb - 1), (j0 + c) * lda + j0 + r, r < jb && c < r);
-            const T idg = T(1) / dg;
-#pragma unroll
-            for (int c = 0; c < BW; c++) {
-                if (c < jb) {
-                    const T yc = readlane_t(t * idg, c);
-                    if (r == c) t = yc;
-                    else if (r > c) t -= Lr[c] * yc;
-                }
-            }
-            if (r < jb) sh.ys[j0 + r] = t;
-        }
-        __syncthreads();
-    }
-    // backward: x = L^-T y
-    for (int bj = nblk - 1; bj >= 0; bj--) {
-        const int j0 = bj * BW, jb = min(BW, n - j0);
-        {
-            const int r = tid >> 3, sl = tid & 7;
-            T acc = T(0);
-            if (r < jb) {
-                int k = j0 + jb + sl;
-                for (; k + 56 < n; k += 64) {
-                    T a[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) a[u] = A[(j0 + r) * lda + k + 8 * u];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) acc += a[u] * sh.ys[k + 8 * u];
-                }
-                for (; k < n; k += 8) acc += A[(j0 + r) * lda + k] * sh.ys[k];
-            }
-            sh.red[sl][r] = acc;
-        }
-        __syncthreads();
-        if (tid < 64) {
-            const int r = tid;
-            T t = T(0), dg = T(1);
-            if (r < jb) {
-                t = sh.ys[j0 + r];
-                for (int sl = 0; sl < 8; sl++) t -= sh.red[sl][r];
-                dg = A[(j0 + r) * lda + j0 + r];
-            }
-            // the block's column r (L(c, r), c > r), loaded before the substitution
-            T Lc[BW];
-#pragma unroll
-            for (int c = 0; c < BW; c++)
-                Lc[c] = mload(A, (j0 + min(r, jb - 1)) * lda + j0 + min(c, jb - 1), (j0 + r) * lda + j0 + c,
-                              r < jb && c > r && c < jb);
-            const T idg = T(1) / dg;
-#pragma unroll
-            for (int c = BW - 1; c >= 0; c--) {
-                if (c < jb) {
-                    const T xc = readlane_t(t * idg, c);
-                    if (r == c) t = xc;
-                    else if (r < c) t -= Lc[c] * xc;
-                }
-            }
-            if (r < jb) sh.ys[j0 + r] = t;
-        }
-        __syncthreads();
-    }
-    for (int i = tid; i < n; i += 256) b[i] = sh.ys[i];
-}
-
-template <class T>
-__global__ __launch_bounds__(256, 2) void k_posv_batched(int count, const int *__restrict__ order,
-                                                        const int *__restrict__ nsz,
-                                                        const int64_t *__restrict__ aoff,
-                                                        const int64_t *__restrict__ boff, T *__restrict__ A,
-                                                        T *__restrict__ B, int *__restrict__ info,
-                                                        int *__restrict__ counter, int nsplit)
-{
-    __shared__ BShared<T> sh;
+    __shared__ __align__(16) BShared<T, NW, MULTI> sh;
+    Batch<T, NW, RT, MULTI> bt(sh);
     for (;;) {
-        if (threadIdx.x == 0) sh.idx = atomicAdd(counter, 1);
+        if (threadIdx.x == 0) {
+            sh.idx = atomicAdd(counter, 1);
+            sh.ds.fail = 0;
+        }
         __syncthreads();
         const int q = sh.idx;
-        __syncthreads();
         if (q >= count) break;
         const int m = order[q];
         const int n = nsz[m];
         T *Am = A + aoff[m];
-        const int f = factor_one<T>(Am, n, n <= nsplit, sh);
+        T *b = B ? B + boff[m] : nullptr;
+        const int f = bt.factor(Am, n, b);
         if (threadIdx.x == 0) info[m] = f;
-        if (f == 0 && B) solve_one<T>(Am, n, B + boff[m], sh);
+        if (f == 0 && b) {
+            bt.backward(Am, n);
+            for (int i = threadIdx.x; i < n; i += 64 * NW) b[i] = sh.ys[i];
+        }
         __syncthreads();
     }
 }
 
+// Size classes of the queue (largest first): above 128, at most 128, at most 64.
+constexpr int BATCH_CLASSES = 3;
+
 __global__ void k_batch_reset(int *counter)
 {
-    if (threadIdx.x == 0) counter[threadIdx.x] = 0;
+    if (threadIdx.x < BATCH_CLASSES) counter[threadIdx.x] = 0;
 }
 
 }  // namespace
@@ -457,12 +496,13 @@ struct mi_batch_s {
     int64_t a_elems = 0, b_elems = 0;
     int *d_n = nullptr, *d_order = nullptr, *d_info = nullptr, *d_counter = nullptr;
     int64_t *d_aoff = nullptr, *d_boff = nullptr;
-    int nsplit = 128, wg_per_cu = 2, cus = 0;
-    // captured graph of the last (A, B, type, shape) it ran on
+    int first[BATCH_CLASSES + 1] = {0, 0, 0, 0};   // queue positions where the classes begin
+    int nsplit = 128, wg_per_cu = 2, cus = 0;      // (nsplit: kept for mi_batch_get_shape only)
+    // captured graph of the last (A, B, type, grid) it ran on
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     const void *g_a = nullptr, *g_b = nullptr;
-    int g_type = -1, g_nsplit = -1, g_wg = -1;
+    int g_type = -1, g_wg = -1;
     double last_ms = 0.0;
 };
 
@@ -476,13 +516,34 @@ void batch_drop_graph(mi_batch_t *p)
     p->graph = nullptr;
 }
 
+// One class: count matrices from queue position q0, at most `wgs` workgroups.
+template <class T>
+void batch_launch(mi_batch_t *p, int cls, int q0, int count, int wgs, T *dA, T *dB, int *counter, hipStream_t s)
+{
+    if (count <= 0) return;
+    const unsigned grid = (unsigned)std::max(1, std::min(count, wgs));
+    const int *order = p->d_order + q0;
+    constexpr bool f64 = sizeof(T) == 8;
+    if (cls == 0)
+        k_posv_batched<T, 8, 2, true, f64 ? 2 : 4><<<grid, 512, 0, s>>>(count, order, p->d_n, p->d_aoff, p->d_boff, dA,
+                                                                        dB, p->d_info, counter);
+    else if (cls == 1)
+        k_posv_batched<T, 8, 1, false, f64 ? 2 : 4><<<grid, 512, 0, s>>>(count, order, p->d_n, p->d_aoff, p->d_boff, dA, dB,
+                                                               p->d_info, counter);
+    else
+        k_posv_batched<T, 4, 1, false, f64 ? 3 : 4><<<grid, 256, 0, s>>>(count, order, p->d_n, p->d_aoff, p->d_boff, dA, dB,
+                                                               p->d_info, counter);
+}
+
+int batch_class(int n) { return n > 128 ? 0 : n > 64 ? 1 : 2; }
+
 template <class T>
 int batch_enqueue(mi_batch_t *p, T *dA, T *dB, hipStream_t s)
 {
-    k_batch_reset<<<1, 1, 0, s>>>(p->d_counter);
-    const unsigned grid = (unsigned)std::max(1, std::min(p->count, p->wg_per_cu * p->cus));
-    k_posv_batched<T><<<grid, 256, 0, s>>>(p->count, p->d_order, p->d_n, p->d_aoff, p->d_boff, dA, dB, p->d_info,
-                                          p->d_counter, p->nsplit);
+    k_batch_reset<<<1, 64, 0, s>>>(p->d_counter);
+    for (int cls = 0; cls < BATCH_CLASSES; cls++)
+        batch_launch<T>(p, cls, p->first[cls], p->first[cls + 1] - p->first[cls],
+                        (cls == 2 ? 2 : 1) * p->wg_per_cu * p->cus, dA, dB, p->d_counter + cls, s);
     MI_CHECK(hipGetLastError());
     return 0;
 }
@@ -497,9 +558,9 @@ int batch_run_loop(mi_batch_t *p, T *dA, T *dB)
     if (p->count == 0) return 0;
     MI_CHECK(hipEventRecord(c->t0, s));
     for (int q = 0; q < p->count; q++) {
-        k_batch_reset<<<1, 1, 0, s>>>(p->d_counter);
-        k_posv_batched<T><<<1, 256, 0, s>>>(1, p->d_order + q, p->d_n, p->d_aoff, p->d_boff, dA, dB, p->d_info,
-                                           p->d_counter, p->nsplit);
+        k_batch_reset<<<1, 64, 0, s>>>(p->d_counter);
+        const int cls = q < p->first[1] ? 0 : q < p->first[2] ? 1 : 2;
+        batch_launch<T>(p, cls, q, 1, 1, dA, dB, p->d_counter, s);
     }
     MI_CHECK(hipGetLastError());
     MI_CHECK(hipEventRecord(c->t1, s));
@@ -521,8 +582,7 @@ int batch_run(mi_batch_t *p, T *dA, T *dB, int use_graph)
     int rc;
     if (p->count == 0) return 0;
     if (use_graph) {
-        if (!p->exec || p->g_a != dA || p->g_b != dB || p->g_type != type || p->g_nsplit != p->nsplit ||
-            p->g_wg != p->wg_per_cu) {
+        if (!p->exec || p->g_a != dA || p->g_b != dB || p->g_type != type || p->g_wg != p->wg_per_cu) {
             batch_drop_graph(p);
             MI_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             rc = batch_enqueue<T>(p, dA, dB, s);
@@ -535,7 +595,6 @@ int batch_run(mi_batch_t *p, T *dA, T *dB, int use_graph)
             p->g_a = dA;
             p->g_b = dB;
             p->g_type = type;
-            p->g_nsplit = p->nsplit;
             p->g_wg = p->wg_per_cu;
         }
         MI_CHECK(hipEventRecord(c->t0, s));
@@ -558,26 +617,20 @@ template <class T>
 int batch_autotune(mi_batch_t *p, const T *dA0, const T *dB0, T *dA, T *dB, int *choice)
 {
     mi_ctx_t *c = p->ctx;
-    static const int splits[] = {0, 256, 512, BMAX};
-    static const int wgs[] = {1, 2};
     double best = 1e300;
-    int bs = p->nsplit, bw = p->wg_per_cu, k = 0, bk = 0;
-    for (int w : wgs)
-        for (int sp : splits) {
-            p->nsplit = sp;
-            p->wg_per_cu = w;
-            double t = 0.0;
-            for (int rep = 0; rep < 2; rep++) {     // the first run warms up
-                MI_CHECK(hipMemcpyAsync(dA, dA0, (size_t)p->a_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
-                if (dB) MI_CHECK(hipMemcpyAsync(dB, dB0, (size_t)p->b_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
-                int rc = batch_run<T>(p, dA, dB, 0);
-                if (rc) return rc;
-                t = p->last_ms;
-            }
-            if (t < best) { best = t; bs = sp; bw = w; bk = k; }
-            k++;
+    int bw = p->wg_per_cu, bk = 0;
+    for (int w = 1; w <= 2; w++) {
+        p->wg_per_cu = w;
+        double t = 0.0;
+        for (int rep = 0; rep < 2; rep++) {         // the first run warms up
+            MI_CHECK(hipMemcpyAsync(dA, dA0, (size_t)p->a_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
+            if (dB) MI_CHECK(hipMemcpyAsync(dB, dB0, (size_t)p->b_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
+            int rc = batch_run<T>(p, dA, dB, 0);
+            if (rc) return rc;
+            t = p->last_ms;
         }
-    p->nsplit = bs;
+        if (t < best) { best = t; bw = w; bk = w - 1; }
+    }
     p->wg_per_cu = bw;
     if (choice) *choice = bk;
     return 0;
@@ -623,6 +676,11 @@ int mi_batch_create(mi_ctx_t *c, int count, const int *n, mi_batch_t **plan)
     std::vector<int> order(count);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return n[a] > n[b]; });
+    for (int cls = 1; cls <= BATCH_CLASSES; cls++) {
+        int q = p->first[cls - 1];
+        while (q < count && batch_class(n[order[q]]) < cls) q++;
+        p->first[cls] = q;
+    }
     int dev = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -632,7 +690,7 @@ int mi_batch_create(mi_ctx_t *c, int count, const int *n, mi_batch_t **plan)
     if (e == hipSuccess) e = hipMalloc(&p->d_n, m * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&p->d_order, m * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&p->d_info, m * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&p->d_counter, sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&p->d_counter, BATCH_CLASSES * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&p->d_aoff, m * sizeof(int64_t));
     if (e == hipSuccess) e = hipMalloc(&p->d_boff, m * sizeof(int64_t));
     if (e == hipSuccess && count) e = hipMemcpy(p->d_n, n, count * sizeof(int), hipMemcpyHostToDevice);

@@ -42,6 +42,9 @@ template <> struct MF<double> {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
     __device__ static inline int row(int q, int fk) { return 4 * q + fk; }
+    // the element and a lane (of the group's first) with row(element, lane / 16) == r
+    __device__ static inline int slice_of(int r) { return r >> 2; }
+    __device__ static inline int lane_of(int r) { return 16 * (r & 3); }
 };
 template <> struct MF<float> {
     typedef fx4 v4;
@@ -51,6 +54,8 @@ template <> struct MF<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     __device__ static inline int row(int q, int fk) { return 4 * fk + q; }
+    __device__ static inline int slice_of(int r) { return r & 3; }
+    __device__ static inline int lane_of(int r) { return 16 * (r >> 2); }
 };
 
 // Wave-uniform copy of a value held by one lane (v_readlane_b32; two for a double).

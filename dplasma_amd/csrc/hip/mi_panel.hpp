@@ -40,6 +40,19 @@ template <int C> __device__ __forceinline__ float row_bcast(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + C, 0xf, 0xf, true));
 }
 
+// value rotated by C lanes within each row of 16 (row_ror)
+template <int C> __device__ __forceinline__ float row_rotate(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + C, 0xf, 0xf, true));
+}
+template <int C> __device__ __forceinline__ double row_rotate(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + C, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + C, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // a[C + i] -= row_bcast<C + i>(m) * f, i < K (K <= 8): one DPP FMA each (the
 // compiler does not fold a broadcast into the FP64 FMA).  The two wait
 // states that a DPP read needs after m was written are inside the block.
@@ -176,49 +189,47 @@ __device__ __forceinline__ void invert_rows(T *v, T *x, T rd, std::integer_seque
 }
 
 // ---------------------------------------------------------------------------
-// Cholesky factor of the n x n (n <= 128) diagonal block A (column-major,
-// ld), lower, in place: right-looking over 16-column blocks.  Eight waves;
-// the 16 x 16 blocks below the first diagonal block live in the registers of
-// waves 1..7 (dealt out column by column) from load to store.
-//   wave 0     factors D_p (sweep above), publishes W_p, forms X(p+1, p) =
-//              C W_p^T and the next diagonal block D_{p+1} -= X X^T itself,
-//   waves 1-7  meanwhile apply step p - 1 to their blocks, hand C(p+1, p)
-//              and D_{p+1} to wave 0 through LDS, and after W_p is there form
-//              the rest of block column p.
+// Cholesky factor of the n x n (n <= 16 NBK) block A (column-major, ld),
+// lower, in place: right-looking over 16-column blocks, by the NW waves of a
+// workgroup; the 16 x 16 blocks below the first diagonal block live in the
+// registers of waves 1.. (dealt out column by column) from load to store.
+//   wave 0   factors D_p (sweep above), publishes W_p, forms X(p+1, p) =
+//            C W_p^T and the next diagonal block D_{p+1} -= X X^T itself,
+//   others   meanwhile apply step p - 1 to their blocks, hand C(p+1, p)
+//            and D_{p+1} to wave 0 through LDS, and after W_p is there form
+//            the rest of block column p.
 // Two barriers a step.  Every block is updated in step order whatever the
-// timing.  Wave 7 stores what wave 0 leaves in LDS.  Bound by wave 0's chain: 16 dependent pivots (reciprocal square
-// root with one correction step, then a DPP FMA into the next pivot), then
-// eight MFMAs and the hand-offs.
-// op: the operand images for k_panel_solve (see OPB); info = info_base + j of
-// the first non-positive pivot j (1-based), as CORE_dpotrf reports it.
-//
-// Measured (n = 128): 20 us in FP64, 21 us in FP32 inside a factorization, of
-// which 2.5 us load the blocks; per 16 columns 3100-3900 cycles of sweep and
-// 1400 cycles of hand-off.  A whole-tile factor of 32-column blocks with
-// v_readlane broadcasts, W_jj on the chain and the tile in memory took 145 us
-// for 256 columns and 367 us (FP32) for 512.
-template <class T>
-__global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n, int ld, int info_base,
-                                                       int *__restrict__ d_info, T *__restrict__ op)
+// timing.  The last wave stores what wave 0 leaves in LDS.  Bound by wave
+// 0's chain: 16 dependent pivots (reciprocal square root with one correction
+// step, then a DPP FMA into the next pivot), then eight MFMAs and the
+// hand-offs.
+// xl(i, p): LDS image ([s][lane]) of -X(i, p), valid until step p + 1 is
+// over; wl(p): W_p in LDS, image column t at t DIAG_WP, valid as long (both
+// may keep all steps); out_w(p, W_p), out_x(i, p, -X(i, p)): called by the
+// wave that has the block.  Returns the 1-based column of the first pivot
+// that is not positive, or 0, to every wave (ds.fail is 0 on entry and
+// ordered before this by a barrier).
+constexpr int DIAG_WP = DB + 2;                             // distinct banks for the writer of W
+template <class T> struct DiagLds {
+    T hc[OPI], hd[OPI];                                     // C(p+1, p) and D_{p+1} for wave 0
+    __align__(16) T ll[2][DB][DIAG_WP];                     // L_pp, [column][row]
+    __align__(16) T dl[DB][DIAG_WP];                        // D, [row][column]
+    int fail;
+};
+template <class T, int NW, int NBK, class XL, class WL, class OW, class OX>
+__device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, DiagLds<T> &ds, XL &&xl, WL &&wl, OW &&out_w,
+                                           OX &&out_x)
 {
     typedef typename MF<T>::v4 V4;
-    constexpr int NW = 7;                                   // worker waves
-    constexpr int NBLK = DBN * (DBN + 1) / 2 - 1;           // blocks besides (0, 0)
-    constexpr int SLOTS = (NBLK + NW - 1) / NW;
-    __shared__ T Xl[DBN][OPI];                              // X(i, p) of the current step
-    constexpr int WP = DB + 2;                              // pitch of Wl: distinct banks for its writer
-    // W_p, image column t (64 s + 16 fk = 16 t) at t WP; two steps' worth, as
-    // is L_pp ([column][row]): a worker still stores the last step's
-    __shared__ __align__(16) T Wl[2][DB * WP];
-    __shared__ __align__(16) T Ll[2][DB][DB + 2];
-    __shared__ T Hc[OPI], Hd[OPI];                          // C(p+1, p) and D_{p+1} for wave 0
-    __shared__ __align__(16) T Dl[DB][DB + 2];              // D, [row][column]
-    __shared__ int s_fail;
-    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int NK = NW - 1;                              // worker waves
+    constexpr int NBLK = NBK * (NBK + 1) / 2 - 1;           // blocks besides (0, 0)
+    constexpr int SLOTS = (NBLK + NK - 1) / NK;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, fk = lane >> 4;
     const int nb = (n + DB - 1) / DB;
-    if (tid == 0) s_fail = 0;
 
     // element (r, c) of A; past n the identity, so that a ragged block
     // factors like a whole one
@@ -237,7 +248,6 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
 #pragma unroll
         for (int q = 0; q < 4; q++) img[64 * q + lane] = b[q];
     };
-    auto put_op = [&](T *img, const V4 &b) { *(V4 *)(img + 4 * lane) = b; };
     auto get = [&](const T *img) -> V4 {
         V4 b;
 #pragma unroll
@@ -245,15 +255,16 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
         return b;
     };
     auto get_w = [&](int p) -> V4 {
+        const T *w = wl(p);
         V4 b;
 #pragma unroll
-        for (int q = 0; q < 4; q++) b[q] = Wl[p & 1][(4 * q + fk) * WP + fr];
+        for (int q = 0; q < 4; q++) b[q] = w[(4 * q + fk) * DIAG_WP + fr];
         return b;
     };
-    // C - X_i X_j^T, both as [s][lane] images
-    auto prod = [&](V4 c, const V4 &xj, const V4 &xi) -> V4 {
+    // C + M_j X_i^T, M_j = -X_j; both as operand images
+    auto prod = [&](V4 c, const V4 &mj, const V4 &xi) -> V4 {
 #pragma unroll
-        for (int s = 0; s < 4; s++) c = MF<T>::mfma(-xj[s], xi[s], c);
+        for (int s = 0; s < 4; s++) c = MF<T>::mfma(mj[s], xi[s], c);
         return c;
     };
     auto solve = [&](const V4 &w, const V4 &c) -> V4 {       // C W^T
@@ -266,12 +277,12 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
     // Both roles run the same barriers: one before the loop's second half
     // (W_p, C(p+1, p) and D_{p+1} are in LDS) and one after it (X(., p) is).
     if (wave == 0) {
-        __builtin_amdgcn_s_setprio(3);                      // it shares its SIMD with wave 4
+        __builtin_amdgcn_s_setprio(3);                      // it shares its SIMD with other waves
         T v[DB], x[DB];
 #pragma unroll
         for (int c = 0; c < DB; c++) {
             v[c] = elem(fr, c);
-            if (fk == 0) Dl[fr][c] = v[c];
+            if (fk == 0) ds.dl[fr][c] = v[c];
         }
         for (int p = 0; p < nb; p++) {
 #pragma unroll
@@ -280,48 +291,49 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
                 int fail = 0;
 #pragma unroll
                 for (int c = 0; c < DB; c++) {
-                    v[c] = Dl[fr][c];
+                    v[c] = ds.dl[fr][c];
                     x[c] = fr == c ? T(1) : T(0);
                 }
                 sweep_exact(v, x, fr, &fail, std::make_integer_sequence<int, DB>());
-                if (fail && lane == 0) s_fail = DB * p + fail;
+                if (fail && lane == 0) ds.fail = DB * p + fail;
             }
             // W(c, fr) = x[c] as the A operand of W C^T: slice s, lane 16 fk +
             // i holds W(i, row(s, fk)), so column fr is image column t
             if (fk == 0) {
-                const int t = sizeof(T) == 8 ? fr : 4 * (fr & 3) + (fr >> 2);
+                T *w = wl(p) + (sizeof(T) == 8 ? fr : 4 * (fr & 3) + (fr >> 2)) * DIAG_WP;
 #pragma unroll
-                for (int c = 0; c < DB; c++) Wl[p & 1][t * WP + c] = x[c];
+                for (int c = 0; c < DB; c++) w[c] = x[c];
             } else if (fk == 1) {
 #pragma unroll
-                for (int c = 0; c < DB; c++) Ll[p & 1][c][fr] = v[c];
+                for (int c = 0; c < DB; c++) ds.ll[p & 1][c][fr] = v[c];
             }
             __syncthreads();
-            if (s_fail) break;
+            if (ds.fail) break;
             if (p + 1 < nb) {
-                const V4 d0 = get(Hd);
-                const V4 xx = solve(get_w(p), get(Hc));
-                put(Xl[p + 1], xx);
-                const V4 d = prod(d0, xx, xx);
+                const V4 d0 = get(ds.hd);
+                const V4 xx = solve(get_w(p), get(ds.hc));
+                put(xl(p + 1, p), -xx);
+                const V4 d = prod(d0, -xx, xx);
 #pragma unroll
-                for (int q = 0; q < 4; q++) Dl[fr][MF<T>::row(q, fk)] = d[q];
+                for (int q = 0; q < 4; q++) ds.dl[fr][MF<T>::row(q, fk)] = d[q];
             }
             __syncthreads();
             if (p + 1 < nb) {
 #pragma unroll
-                for (int c = 0; c < DB; c++) v[c] = Dl[fr][c];
+                for (int c = 0; c < DB; c++) v[c] = ds.dl[fr][c];
             }
         }
+        __builtin_amdgcn_s_setprio(0);
     } else {
-        // slot u: block t = wave + 7 u of the list (0,0) (1,0) .. (7,0) (1,1)
-        // (2,1) .. ; bi, bj are wave-uniform, bj = -1 where there is none
+        // slot u: block t = wave + NK u of the list (0,0) (1,0) .. (NBK-1,0)
+        // (1,1) (2,1) .. ; bi, bj are wave-uniform, bj = -1 where there is none
         V4 blk[SLOTS];
         int bi[SLOTS], bj[SLOTS];
 #pragma unroll
         for (int u = 0; u < SLOTS; u++) {
-            int t = wave + NW * u, j = 0;
-            while (j < DBN && t >= DBN - j) { t -= DBN - j; j++; }
-            bj[u] = j < DBN && j + t < nb ? j : -1;
+            int t = wave + NK * u, j = 0;
+            while (j < NBK && t >= NBK - j) { t -= NBK - j; j++; }
+            bj[u] = j < NBK && j + t < nb ? j : -1;
             bi[u] = j + t;
             if (bj[u] >= 0) {
 #pragma unroll
@@ -330,7 +342,7 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
         }
 #pragma unroll
         for (int u = 0; u < SLOTS; u++)
-            if (bj[u] >= 0 && bi[u] == 1) put(bj[u] == 0 ? Hc : Hd, blk[u]);
+            if (bj[u] >= 0 && bi[u] == 1) put(bj[u] == 0 ? ds.hc : ds.hd, blk[u]);
         for (int p = 0; p < nb; p++) {
             if (p > 0) {
                 // step p - 1 on the blocks of columns >= p (wave 0 did (p, p));
@@ -338,44 +350,69 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
 #pragma unroll
                 for (int u = 0; u < SLOTS; u++)
                     if (bj[u] >= p && bi[u] > p) {
-                        blk[u] = prod(blk[u], get(Xl[bj[u]]), get(Xl[bi[u]]));
-                        if (bi[u] == p + 1) put(bj[u] == p ? Hc : Hd, blk[u]);
+                        blk[u] = prod(blk[u], get(xl(bj[u], p - 1)), -get(xl(bi[u], p - 1)));
+                        if (bi[u] == p + 1) put(bj[u] == p ? ds.hc : ds.hd, blk[u]);
                     }
             }
             __syncthreads();
-            if (s_fail) break;
+            if (ds.fail) break;
             const V4 w = get_w(p);
-            T *opp = op + (int64_t)p * OPB;
 #pragma unroll
             for (int u = 0; u < SLOTS; u++)
                 if (bj[u] == p && bi[u] > p + 1) {
                     blk[u] = solve(w, blk[u]);
-                    put(Xl[bi[u]], blk[u]);
+                    put(xl(bi[u], p), -blk[u]);
                 }
             __syncthreads();
 #pragma unroll
             for (int u = 0; u < SLOTS; u++)
                 if (bj[u] == p && bi[u] > p + 1) {
                     store(bi[u], p, blk[u]);
-                    put_op(opp + (bi[u] - p) * OPI, -blk[u]);
+                    out_x(bi[u], p, -blk[u]);
                 }
             // what wave 0 left: L_pp, W_p and X(p + 1, p)
-            if (wave == NW) {
-                put_op(opp, w);
+            if (wave == NK) {
+                out_w(p, w);
                 if (p + 1 < nb) {
-                    const V4 xx = get(Xl[p + 1]);
-                    store(p + 1, p, xx);
-                    put_op(opp + OPI, -xx);
+                    const V4 mx = get(xl(p + 1, p));
+                    store(p + 1, p, -mx);
+                    out_x(p + 1, p, mx);
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int c = 4 * u + fk;
-                    if (c <= fr && DB * p + fr < n) A[(int64_t)(DB * p + c) * ld + DB * p + fr] = Ll[p & 1][c][fr];
+                    if (c <= fr && DB * p + fr < n) A[(int64_t)(DB * p + c) * ld + DB * p + fr] = ds.ll[p & 1][c][fr];
                 }
             }
         }
     }
-    if (tid == 0 && s_fail) atomicCAS(d_info, 0, info_base + s_fail);
+    return __builtin_amdgcn_readfirstlane(ds.fail);
+}
+
+// The diagonal block of a sub-column: n <= 128, one workgroup of eight waves.
+// op: the operand images for k_panel_solve (see OPB); info = info_base + j of
+// the first non-positive pivot j (1-based), as CORE_dpotrf reports it.
+//
+// Measured (n = 128): 20 us in FP64, 21 us in FP32 inside a factorization, of
+// which 2.5 us load the blocks; per 16 columns 3100-3900 cycles of sweep and
+// 1400 cycles of hand-off.  A whole-tile factor of 32-column blocks with
+// v_readlane broadcasts, W_jj on the chain and the tile in memory took 145 us
+// for 256 columns and 367 us (FP32) for 512.
+template <class T>
+__global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n, int ld, int info_base,
+                                                       int *__restrict__ d_info, T *__restrict__ op)
+{
+    typedef typename MF<T>::v4 V4;
+    __shared__ DiagLds<T> ds;
+    __shared__ T x[DBN][OPI];
+    __shared__ __align__(16) T w[2][DB * DIAG_WP];
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) ds.fail = 0;
+    const int f = diag_factor<T, 8, DBN>(
+        A, n, ld, ds, [&](int i, int) { return x[i]; }, [&](int p) { return w[p & 1]; },
+        [&](int p, const V4 &b) { *(V4 *)(op + (int64_t)p * OPB + 4 * lane) = b; },
+        [&](int i, int p, const V4 &b) { *(V4 *)(op + (int64_t)p * OPB + (i - p) * OPI + 4 * lane) = b; });
+    if (threadIdx.x == 0 && f) atomicCAS(d_info, 0, info_base + f);
 }
 
 // ---------------------------------------------------------------------------

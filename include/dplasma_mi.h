@@ -289,7 +289,8 @@ int mi_dpotri_tiles(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
  * src/cores/core_zpotrf.c:68-74).  Matrix i is column-major, lda = n_i, at
  * element offset sum_{j<i} n_j^2 of dA; its right-hand side at offset
  * sum_{j<i} n_j of dB (dB may be NULL: factor only).  One persistent launch
- * works through the batch; with use_graph the launch is captured in a
+ * per size class (above 128, at most 128, at most 64) works through the
+ * batch; with use_graph the launches are captured in a
  * hipGraph on the first call for given (dA, dB) and replayed after. */
 typedef struct mi_batch_s mi_batch_t;
 /* n[i] = lo + (splitmix64 word i of seed) mod (hi - lo + 1) */
@@ -301,11 +302,13 @@ int mi_dbatch_spd(mi_ctx_t *ctx, int count, const int *n, uint64_t seed, double 
 int mi_batch_create(mi_ctx_t *ctx, int count, const int *n, mi_batch_t **plan);
 int mi_batch_destroy(mi_batch_t *plan);
 int mi_batch_extent(const mi_batch_t *plan, int64_t *a_elems, int64_t *b_elems);
-/* tile shape: matrices with n <= nsplit use 64-row strips, the others
- * 128-row strips; wg_per_cu = 1 or 2 persistent workgroups per CU */
+/* launch shape: wg_per_cu = 1 or 2 persistent workgroups per CU (twice as
+ * many for the matrices of at most 64); nsplit is stored but changes nothing
+ * (the kernels choose by the order of a matrix).  Results do not depend on
+ * the shape. */
 int mi_batch_set_shape(mi_batch_t *plan, int nsplit, int wg_per_cu);
 int mi_batch_get_shape(const mi_batch_t *plan, int *nsplit, int *wg_per_cu);
-/* Times each candidate shape on a copy of (dA0, dB0) in (dA, dB) and keeps
+/* Times each number of workgroups per CU on a copy of (dA0, dB0) in (dA, dB) and keeps
  * the fastest; *choice = its index.  dA/dB are overwritten. */
 int mi_dbatch_autotune(mi_batch_t *plan, const double *dA0, const double *dB0, double *dA, double *dB,
                        int *choice);

@@ -177,3 +177,56 @@ def test_wavefront_inverses_at_block_edges(dev, po, N, NB, trans, unit, dtype):
     ref = np.linalg.solve(L.T if trans == 112 else L, B.astype(np.float64))
     eps = 2.0 ** -53 if dtype == np.float64 else EPS32
     assert np.abs(x - ref).max() <= 16 * (N + 16) * eps * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("solve", [True, False])
+def test_batched_block_edges(dev, dtype, solve):
+    """Orders around the 16-column blocks, the size classes (64, 128) and the
+    128-column panels, every upper triangle NaN; one matrix without a positive
+    pivot in the middle (its right-hand side stays).  G^T G / n + I has a
+    condition below 6: n eps times a small factor."""
+    ns = [1, 15, 16, 17, 47, 48, 49, 63, 64, 65, 111, 112, 113, 127, 128, 129, 143, 144, 145, 240, 256, 257, 272, 383,
+          384, 385, 400, 530, 641, 897, 1009]
+    bad = ns.index(145)
+    rng = np.random.default_rng(3)
+    As, bs = [], []
+    for n in ns:
+        G = rng.standard_normal((n, n))
+        As.append((G.T @ G / n + np.eye(n)).astype(dtype))
+        bs.append(rng.uniform(-0.5, 0.5, n).astype(dtype))
+    As[bad][130, 130] = -1.0
+    flat = []
+    for A in As:
+        M = A.copy()
+        M[np.triu_indices(M.shape[0], 1)] = np.nan
+        flat.append(M.ravel(order="F"))
+    a, b = np.concatenate(flat), np.concatenate(bs)
+    p = ctypes.c_void_p()
+    dev.check(dev.M.mi_batch_create(dev.h, len(ns), (ctypes.c_int * len(ns))(*ns), ctypes.byref(p)), "create")
+    da, db = dev.upload(a), dev.upload(b)
+    fn = dev.M.mi_dposv_batched if dtype == np.float64 else dev.M.mi_sposv_batched
+    try:
+        dev.check(fn(p, da, db if solve else None, 0), "posv_batched")
+        ra, rb = dev.download(da, a.shape, dtype), dev.download(db, b.shape, dtype)
+        info = (ctypes.c_int * len(ns))()
+        dev.check(dev.M.mi_batch_info(p, info), "info")
+    finally:
+        dev.M.mi_batch_destroy(p)
+        dev.free(da)
+        dev.free(db)
+    eps = 2.0 ** -53 if dtype == np.float64 else EPS32
+    ao = bo = 0
+    for i, n in enumerate(ns):
+        L, x = ra[ao:ao + n * n].reshape((n, n), order="F"), rb[bo:bo + n]
+        assert np.isnan(L[np.triu_indices(n, 1)]).all(), n
+        if i == bad:
+            assert info[i] == 131 and np.array_equal(x, bs[i])
+        else:
+            assert info[i] == 0, n
+            ref = np.linalg.cholesky(As[i].astype(np.float64))
+            assert np.abs(np.tril(L) - ref).max() <= 16 * (n + 16) * eps * np.abs(ref).max(), n
+            want = np.linalg.solve(As[i].astype(np.float64), bs[i].astype(np.float64)) if solve else bs[i]
+            assert np.abs(x - want).max() <= 64 * (n + 16) * eps * max(1.0, np.abs(want).max()), n
+        ao += n * n
+        bo += n
