@@ -132,6 +132,12 @@ def libs():
     _sig(M, "mi_dposv_lapack", i, [vp, i, i, i, vp, i, vp, i, i, pi])
     _sig(M, "mi_dsym_lapack_to_tiles", i, [vp, i, i, vp, i, i, vp])
     _sig(M, "mi_dsym_tiles_to_lapack", i, [vp, i, i, i, vp, vp, i])
+    _sig(M, "mi_ssym_lapack_to_tiles", i, [vp, i, i, vp, i, i, vp])
+    _sig(M, "mi_ssym_tiles_to_lapack", i, [vp, i, i, i, vp, vp, i])
+    for n in ("mi_dgp_nll", "mi_sgp_nll"):
+        _sig(M, n, i, [vp, i, i, vp, i, vp, vp, vp, pi])
+    for n in ("mi_dgp_nll_grad", "mi_sgp_nll_grad"):
+        _sig(M, n, i, [vp, i, i, vp, vp, vp, vp, vp, vp, i])
     _sig(M, "mi_spotrf_tiles", i, [vp, i, i, vp, pi])
     _sig(M, "mi_spotrf_step_potrf", i, [vp, i, i, vp, i, pi])
     _sig(M, "mi_dsposv_tiles", i, [vp, i, i, vp, i, vp, i, vp, i, i, pi, pi])

@@ -469,10 +469,8 @@ GJob<T> job(const T *A, int aform, const T *B, const T *Cin, T *Cout, T alpha, T
 }
 
 template <class T>
-int adjoint_tiles(mi_ctx_t *c, int N, int NB, const T *dL, T *dG)
+int adjoint_plan_run(Ctx *c, int N, int NB, const T *dL, T *dG)
 {
-    if (N <= 0) return 0;
-    if (NB <= 0) { set_error("bad tile size"); return -2; }
     const int MT = (N + NB - 1) / NB;
     const int64_t T2 = (int64_t)NB * NB;
     hipStream_t s = c->s_main;
@@ -610,7 +608,6 @@ int adjoint_tiles(mi_ctx_t *c, int N, int NB, const T *dL, T *dG)
     T *part = (T *)ws_get(c, WS_ADJ_PART, (size_t)part_elems * sizeof(T));
     if (!part) return -3;
 
-    MI_CHECK(hipEventRecord(c->t0, s));
     for (const Launch &l : pl.plan) {
         if (l.kind == 2) {
             const int64_t n = (int64_t)MT * T2;
@@ -642,9 +639,19 @@ int adjoint_tiles(mi_ctx_t *c, int N, int NB, const T *dL, T *dG)
             }
         }
     }
-    MI_CHECK(hipEventRecord(c->t1, s));
-    int rc = mi_synchronize(c);
+    return 0;
+}
+
+template <class T>
+int adjoint_tiles(mi_ctx_t *c, int N, int NB, const T *dL, T *dG)
+{
+    if (N <= 0) return 0;
+    if (NB <= 0) { set_error("bad tile size"); return -2; }
+    MI_CHECK(hipEventRecord(c->t0, c->s_main));
+    int rc = adjoint_plan_run<T>(c, N, NB, dL, dG);
     if (rc) return rc;
+    MI_CHECK(hipEventRecord(c->t1, c->s_main));
+    if ((rc = mi_synchronize(c))) return rc;
     float ms = 0.f;
     MI_CHECK(hipEventElapsedTime(&ms, c->t0, c->t1));
     c->last_ms = ms;
@@ -697,6 +704,17 @@ __global__ __launch_bounds__(256) void k_copy_lower_tiles(const double *__restri
 
 
 }  // namespace
+
+namespace mi {
+template <> int adjoint_enqueue<double>(Ctx *c, int N, int NB, const double *dL, double *dG)
+{
+    return adjoint_plan_run<double>(c, N, NB, dL, dG);
+}
+template <> int adjoint_enqueue<float>(Ctx *c, int N, int NB, const float *dL, float *dG)
+{
+    return adjoint_plan_run<float>(c, N, NB, dL, dG);
+}
+}  // namespace mi
 
 extern "C" {
 

@@ -176,6 +176,15 @@ int trsm_abort_error();
 // wait = false: enqueue only (both streams joined into s_main); *info is
 // then 0 and the factorization's info is left in d_info[0].
 int spotrf_tiles_split(Ctx *c, int N, int NB, float *dT, int *info, bool bf16_split, bool wait = true);
+// Factorization (mi_dpotrf_tiles / mi_spotrf_tiles) enqueued only, both
+// streams joined into s_main; its info is left in d_info[0].
+template <class T> int potrf_enqueue(Ctx *c, int N, int NB, T *dT);
+// Column-major array <-> packed lower tile image (mi_lapack.hip), enqueued.
+template <class E>
+int sym_stage_enqueue(Ctx *c, hipStream_t st, bool to_image, int uplo, int N, int NB, E *dT, E *dA, int lda);
+// The blocked reverse of the factorization (mi_adjoint.hip), enqueued on s_main
+// (its plan's tables are uploaded first, synchronously).
+template <class T> int adjoint_enqueue(Ctx *c, int N, int NB, const T *dL, T *dG);
 // Reads, once per device and with that device current, the device address of
 // the fixed scratch of mi_dpotrf_tiles_noalloc (mi_potrf.hip).
 void noalloc_setup(int device);

@@ -42,17 +42,17 @@ __device__ inline void tile_of(int64_t t, int MT, int &m, int &n)
 // One 32 x 32 block of tile t = blockIdx.x (block blockIdx.y of the tile's
 // ceil(NB/32)^2).  TO_IMAGE: column-major A -> image T; otherwise T's lower
 // triangle (the factor) -> A's uplo triangle.
-template <bool TO_IMAGE, bool UPPER>
-__global__ __launch_bounds__(256) void k_sym_stage(double *__restrict__ T, double *__restrict__ A, int N, int NB,
-                                                   int MT, int64_t lda)
+template <class E, bool TO_IMAGE, bool UPPER>
+__global__ __launch_bounds__(256) void k_sym_stage(E *__restrict__ T, E *__restrict__ A, int N, int NB, int MT,
+                                                   int64_t lda)
 {
-    __shared__ double buf[32][33];
+    __shared__ E buf[32][33];
     const int sb = (NB + 31) / 32;
     int m, n;
     tile_of(blockIdx.x, MT, m, n);
     const int r0 = (blockIdx.y % sb) * 32, c0 = (blockIdx.y / sb) * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    double *Tt = T + (int64_t)blockIdx.x * NB * NB;
+    E *Tt = T + (int64_t)blockIdx.x * NB * NB;
     // image element (r, c) of this tile: global (m NB + r, n NB + c)
     auto in_tile = [&](int r, int c) { return r < NB && c < NB; };
     auto in_tri = [&](int r, int c) {
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void k_sym_stage(double *__restrict__ T, doubl
             const int r = r0 + tx, c = c0 + y;
             const int64_t a = (int64_t)(n * NB + c) * lda + (m * NB + r);
             if (TO_IMAGE) {
-                if (in_tile(r, c)) Tt[(int64_t)c * NB + r] = in_tri(r, c) ? A[a] : 0.0;
+                if (in_tile(r, c)) Tt[(int64_t)c * NB + r] = in_tri(r, c) ? A[a] : E(0);
             } else if (in_tri(r, c)) {
                 A[a] = Tt[(int64_t)c * NB + r];
             }
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void k_sym_stage(double *__restrict__ T, doubl
     if (TO_IMAGE) {
         for (int y = ty; y < 32; y += 8) {                // A column m NB + r0 + y, rows n NB + c0 + tx
             const int r = r0 + y, c = c0 + tx;
-            buf[y][tx] = in_tri(r, c) ? A[(int64_t)(m * NB + r) * lda + (n * NB + c)] : 0.0;
+            buf[y][tx] = in_tri(r, c) ? A[(int64_t)(m * NB + r) * lda + (n * NB + c)] : E(0);
         }
         __syncthreads();
         for (int y = ty; y < 32; y += 8) {                // image column c0 + y, rows r0 + tx
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void k_sym_stage(double *__restrict__ T, doubl
     } else {
         for (int y = ty; y < 32; y += 8) {
             const int r = r0 + tx, c = c0 + y;
-            buf[tx][y] = in_tile(r, c) ? Tt[(int64_t)c * NB + r] : 0.0;
+            buf[tx][y] = in_tile(r, c) ? Tt[(int64_t)c * NB + r] : E(0);
         }
         __syncthreads();
         for (int y = ty; y < 32; y += 8) {
@@ -109,28 +109,8 @@ int check_args(const char *f, int uplo, int N, int lda, int NB)
 
 int stage(mi_ctx_t *c, int to_image, int uplo, int N, int NB, double *dT, double *dA, int lda)
 {
-    const int MT = (N + NB - 1) / NB;
-    const int sb = (NB + 31) / 32;
-    const dim3 grid((unsigned)((int64_t)MT * (MT + 1) / 2), (unsigned)(sb * sb));
-    if (sb * sb > 65535) { set_error("tile size NB = %d too large for the staging grid", NB); return -6; }
-    const double bytes = 2.0 * 8.0 * ((double)N * (N + 1) / 2);
-    const bool up = uplo == UPLO_UPPER;
-    if (to_image) {
-        if (up)
-            MI_LAUNCH(c, c->s_main, "dsym_stage_in", 0.0, bytes,
-                      k_sym_stage<true, true><<<grid, 256, 0, c->s_main>>>(dT, dA, N, NB, MT, lda));
-        else
-            MI_LAUNCH(c, c->s_main, "dsym_stage_in", 0.0, bytes,
-                      k_sym_stage<true, false><<<grid, 256, 0, c->s_main>>>(dT, dA, N, NB, MT, lda));
-    } else {
-        if (up)
-            MI_LAUNCH(c, c->s_main, "dsym_stage_out", 0.0, bytes,
-                      k_sym_stage<false, true><<<grid, 256, 0, c->s_main>>>(dT, dA, N, NB, MT, lda));
-        else
-            MI_LAUNCH(c, c->s_main, "dsym_stage_out", 0.0, bytes,
-                      k_sym_stage<false, false><<<grid, 256, 0, c->s_main>>>(dT, dA, N, NB, MT, lda));
-    }
-    return mi_synchronize(c);
+    int rc = sym_stage_enqueue<double>(c, c->s_main, to_image, uplo, N, NB, dT, dA, lda);
+    return rc ? rc : mi_synchronize(c);
 }
 
 // packed image of the N x N matrix (MT(MT+1)/2 tiles of NB x NB)
@@ -141,6 +121,48 @@ int alloc_image(mi_ctx_t *c, int N, int NB, double **dT)
 }
 
 }  // namespace
+
+namespace mi {
+template <class E>
+int sym_stage_enqueue(Ctx *c, hipStream_t st, bool to_image, int uplo, int N, int NB, E *dT, E *dA, int lda)
+{
+    const int MT = (N + NB - 1) / NB;
+    const int sb = (NB + 31) / 32;
+    const dim3 grid((unsigned)((int64_t)MT * (MT + 1) / 2), (unsigned)(sb * sb));
+    if (sb * sb > 65535) { set_error("tile size NB = %d too large for the staging grid", NB); return -6; }
+    const double bytes = 2.0 * sizeof(E) * ((double)N * (N + 1) / 2);
+    const bool up = uplo == UPLO_UPPER;
+    const bool d = sizeof(E) == 8;
+    const char *name = to_image ? (d ? "dsym_stage_in" : "ssym_stage_in") : (d ? "dsym_stage_out" : "ssym_stage_out");
+    if (to_image && up)
+        MI_LAUNCH(c, st, name, 0.0, bytes, (k_sym_stage<E, true, true><<<grid, 256, 0, st>>>(dT, dA, N, NB, MT, lda)));
+    else if (to_image)
+        MI_LAUNCH(c, st, name, 0.0, bytes, (k_sym_stage<E, true, false><<<grid, 256, 0, st>>>(dT, dA, N, NB, MT, lda)));
+    else if (up)
+        MI_LAUNCH(c, st, name, 0.0, bytes, (k_sym_stage<E, false, true><<<grid, 256, 0, st>>>(dT, dA, N, NB, MT, lda)));
+    else
+        MI_LAUNCH(c, st, name, 0.0, bytes, (k_sym_stage<E, false, false><<<grid, 256, 0, st>>>(dT, dA, N, NB, MT, lda)));
+    return 0;
+}
+template int sym_stage_enqueue<double>(Ctx *, hipStream_t, bool, int, int, int, double *, double *, int);
+template int sym_stage_enqueue<float>(Ctx *, hipStream_t, bool, int, int, int, float *, float *, int);
+}  // namespace mi
+
+extern "C" int mi_ssym_lapack_to_tiles(mi_ctx_t *c, int uplo, int N, const float *dA, int lda, int NB, float *dT)
+{
+    int rc = check_args("mi_ssym_lapack_to_tiles", uplo, N, lda, NB);
+    if (rc || N == 0) return rc;
+    rc = sym_stage_enqueue<float>(c, c->s_main, true, uplo, N, NB, dT, const_cast<float *>(dA), lda);
+    return rc ? rc : mi_synchronize(c);
+}
+
+extern "C" int mi_ssym_tiles_to_lapack(mi_ctx_t *c, int uplo, int N, int NB, const float *dT, float *dA, int lda)
+{
+    int rc = check_args("mi_ssym_tiles_to_lapack", uplo, N, lda, NB);
+    if (rc || N == 0) return rc;
+    rc = sym_stage_enqueue<float>(c, c->s_main, false, uplo, N, NB, const_cast<float *>(dT), dA, lda);
+    return rc ? rc : mi_synchronize(c);
+}
 
 extern "C" int mi_dsym_lapack_to_tiles(mi_ctx_t *c, int uplo, int N, const double *dA, int lda, int NB,
                                        double *dT)

@@ -1495,6 +1495,17 @@ int task_update_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, in
 }
 size_t task_winv_elems(int NB) { return potrf_ws_elems(NB) / 2; }
 
+template <> int potrf_enqueue<double>(Ctx *c, int N, int NB, double *dT)
+{
+    int info;
+    return potrf_tiles<double>(c, N, NB, dT, &info, false, nullptr, false, half_tile_hmb(NB), false);
+}
+template <> int potrf_enqueue<float>(Ctx *c, int N, int NB, float *dT)
+{
+    int info;
+    return spotrf_tiles_split(c, N, NB, dT, &info, g_supdate == 1, false);
+}
+
 int spotrf_tiles_split(Ctx *c, int N, int NB, float *dT, int *info, bool bf16_split, bool wait)
 {
     return potrf_tiles<float>(c, N, NB, dT, info, bf16_split, nullptr, false, bf16_split ? half_tile_hmb(NB) : 0,

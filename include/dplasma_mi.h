@@ -180,6 +180,8 @@ int mi_dposv_lapack(mi_ctx_t *ctx, int uplo, int N, int NRHS, double *dA, int ld
  * zero), and the lower triangle of dT back to A's uplo triangle. */
 int mi_dsym_lapack_to_tiles(mi_ctx_t *ctx, int uplo, int N, const double *dA, int lda, int NB, double *dT);
 int mi_dsym_tiles_to_lapack(mi_ctx_t *ctx, int uplo, int N, int NB, const double *dT, double *dA, int lda);
+int mi_ssym_lapack_to_tiles(mi_ctx_t *ctx, int uplo, int N, const float *dA, int lda, int NB, float *dT);
+int mi_ssym_tiles_to_lapack(mi_ctx_t *ctx, int uplo, int N, int NB, const float *dT, float *dA, int lda);
 
 /* Single task-class launches (one step k of the factorization), for tests:
  *   POTRF(k)            src/zpotrf_L.jdf:91-208
@@ -280,6 +282,24 @@ int mi_spotrf_adjoint_tiles(mi_ctx_t *ctx, int N, int NB, const float *dL, float
  * trtri + lauum there).  *info = i > 0 if L(i,i) == 0 (dT unchanged).
  * Blocking. */
 int mi_dpotri_tiles(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
+
+/* Gaussian-process negative log marginal likelihood of y under the covariance
+ * K (dense row-major in device memory, leading dimension ldk; only its lower
+ * triangle is read): dT receives the factor (MT(MT+1)/2 tiles), dy (N values,
+ * y on entry) a = L^-1 y, dout[0..1] sum log L_ii and a^T a in FP64, so that
+ * nll = dout[1] / 2 + dout[0] + N/2 log 2 pi.  *info as mi_dpotrf_tiles (then
+ * the outputs are not valid).  NB a multiple of 32, at most 960.  Blocking. */
+int mi_dgp_nll(mi_ctx_t *ctx, int N, int NB, const double *dK, int ldk, double *dT, double *dy, double *dout,
+               int *info);
+int mi_sgp_nll(mi_ctx_t *ctx, int N, int NB, const float *dK, int ldk, float *dT, float *dy, double *dout, int *info);
+/* Its gradient times the device scalar *dscale: from the factor dT and a of
+ * the call above, dalpha = K^-1 y (N values) and dK = the symmetric dnll/dK
+ * (both triangles, row-major, ldk); dG: MT(MT+1)/2 tiles of scratch.
+ * Blocking. */
+int mi_dgp_nll_grad(mi_ctx_t *ctx, int N, int NB, const double *dT, const double *da, double *dalpha,
+                    const double *dscale, double *dG, double *dK, int ldk);
+int mi_sgp_nll_grad(mi_ctx_t *ctx, int N, int NB, const float *dT, const float *da, float *dalpha, const float *dscale,
+                    float *dG, float *dK, int ldk);
 
 /* ------------------------------------------------------------ batched */
 /* Many independent SPD systems of uneven orders n_i in [1, 1024], each
