@@ -221,6 +221,15 @@ struct mi_ctx_s : public mi::Ctx {};
         }                                                                         \
     } while (0)
 
+namespace mi {
+// Dynamic LDS of a kernel beyond 64 KB is asked for before its launch.
+inline int set_lds(const void *f, size_t bytes)
+{
+    if (bytes > 65536) MI_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return 0;
+}
+}  // namespace mi
+
 // Launch with optional event bracketing for the profiler.
 // The last error is cleared right before the launch, so that the check
 // after it reports this launch and not an earlier ignored failure.

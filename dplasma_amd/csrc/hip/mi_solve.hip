@@ -1163,12 +1163,6 @@ int g_wave_solve = 1;   // 1: one-launch wavefront solve when NB % 32 == 0; 0: p
 // real-time counter (default 10 s; 0 = give up at once)
 long long g_wave_wait_ticks = 1000000000LL;
 
-int set_lds(const void *f, size_t bytes)
-{
-    if (bytes > 65536) MI_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    return 0;
-}
-
 template <class T> struct SN;
 template <> struct SN<double> {
     static constexpr const char *diag = "dtrsm_diag", *gemv = "dtrsm_gemv", *inv = "dtrsm_inv_diag",
