@@ -406,6 +406,7 @@ __global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n
     __shared__ DiagLds<T> ds;
     __shared__ T x[DBN][OPI];
     __shared__ __align__(16) T w[2][DB * DIAG_WP];
+    __builtin_amdgcn_s_setprio(2);
     const int lane = threadIdx.x & 63;
     if (threadIdx.x == 0) ds.fail = 0;
     const int f = diag_factor<T, 8, DBN>(
@@ -435,6 +436,7 @@ __global__ __launch_bounds__(256, 2) void k_panel_solve(T *__restrict__ Tt, int 
                                                        int w, const T *__restrict__ op, int g0, int gt, int m0)
 {
     typedef typename MF<T>::v4 V4;
+    __builtin_amdgcn_s_setprio(2);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int fr = lane & 15, fk = lane >> 4;
     const int g = blockIdx.x;

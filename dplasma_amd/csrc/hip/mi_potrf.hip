@@ -435,6 +435,7 @@ struct UpdArgs {
     int N, NB, MT, k;
     int n_begin, m_off, nsub;                      // whole tiles
     int c0, w, g0, gr, nc, m0;                     // panel (w > 0)
+    int prio;                                      // wave priority (on the chain of panels: above the bulk)
 };
 // Workgroup -> block; false: nothing to do.
 __device__ __forceinline__ bool update_decode(const UpdArgs &u, int BMX, int *m, int *n, int *r_base, int *c_base,
@@ -483,6 +484,7 @@ __global__ __launch_bounds__(S::NT, OCC) void k_update_lds(T *__restrict__ Tt, U
     __shared__ __align__(1024) unsigned char lds[S::LDS];
     int m, n, r_base, c_base, rows_m, cols_n;
     bool diag;
+    if (u.prio) __builtin_amdgcn_s_setprio(2);
     if (!update_decode(u, S::BM, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
     const int64_t sz = (int64_t)u.NB * u.NB, off = (int64_t)u.c0 * u.NB;
     update_block_lds<S, T>(lds, Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
@@ -1229,7 +1231,7 @@ int launch_panel(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k, T *
         if (c1 >= n || (!diag && ntile <= 0)) continue;
         const double fl = 2.0 * below * w * (n - c1) + (diag ? (double)w * (n - c1) * (n - c1 + 1.0) : 0.0);
         const double by = (below + (diag ? 0.5 * (n - c1) : 0.0)) * (2.0 * (n - c1) + w) * sizeof(T);
-        UpdArgs u{N, NB, MT, k, 0, 0, 0, c0, w, 0, 0, 0, m0};
+        UpdArgs u{N, NB, MT, k, 0, 0, 0, c0, w, 0, 0, 0, m0, 1};
         auto grid = [&](int bm) -> int64_t {
             u.g0 = diag ? (n - c1 + bm - 1) / bm : 0;
             u.gr = (NB + bm - 1) / bm;
@@ -1296,7 +1298,7 @@ int launch_update_run(Ctx *c, hipStream_t s, T *dT, int N, int NB, int MT, int k
                   k_update_bf16x3<<<(unsigned)grid, 256, 0, s>>>((float *)dT, N, NB, MT, k, n_begin, m_off,
                                                                  nsub));
     else {
-        UpdArgs u{N, NB, MT, k, n_begin, m_off, 0, 0, 0, 0, 0, 0, 0};
+        UpdArgs u{N, NB, MT, k, n_begin, m_off, 0, 0, 0, 0, 0, 0, 0, la ? 1 : 0};
         return launch_update_blocks<T>(c, s, la ? KN<T>::update_la : KN<T>::update, fl, by, dT, u, NB, [&](int bm) {
             u.nsub = (NB + bm - 1) / bm;
             return ntiles * u.nsub * u.nsub;
@@ -1336,11 +1338,25 @@ constexpr size_t potrf_ws_elems(int NB) { return (size_t)2 * ((NB + DB - 1) / DB
 // two-step look-ahead over two streams (src/zpotrf_L.jdf's priorities give
 // the panel the critical path):
 //   panel stream, step k:  [wait: column k+1 updated by step k-1]
-//                          column k+1 updated by step k (SYRK + GEMMs),
+//                          column k+1 updated by step k (SYRK + GEMMs)
+//                          -> event for the main stream,
 //                          POTRF(k+1), TRSM(k+1)
-//   main stream, step k:   [wait: TRSM(k)]
+//   main stream, step k:   [wait: column k+1 updated by step k]
 //                          column k+2 updated by step k  -> event for the panel,
 //                          columns k+3.. updated by step k (the bulk)
+// The bulk starts after column k+1 and not beside it: that column is on the
+// chain and takes 16 us alone, 37 us next to the bulk (N = 4096, NB = 256).
+//
+// Once a whole update is at most ONE_STREAM_WORK multiply-adds (FP64; twice
+// that in FP32), about 100 us, it is one launch on the chain: no event (each
+// about 10 us on the GPU and 4 us of host time), no column of its own before
+// the rest.  A factorization that starts there uses the main stream only.
+// Both together: dpotrf N = 378, NB = 93 260 -> 218 us; N = 4096, NB = 256
+// 1.86 -> 1.77 ms; FP32 N = 10000, NB = 512 5.71 -> 5.37 ms (with the waves'
+// priorities below).  Half or twice the limit: within 1%, four times it FP32
+// N = 10000 5.7 ms.
+// The waves of the chain's kernels run at a higher priority than the bulk's,
+// which share their SIMDs (FP32 N = 10000 5.66 -> 5.45 ms).
 // Every tile gets its updates in step order and no two launches touch the
 // same tile at once; the panel chain waits for one column of the bulk of
 // step k-1, not for all of it.
@@ -1354,6 +1370,7 @@ constexpr size_t potrf_ws_elems(int NB) { return (size_t)2 * ((NB + DB - 1) / DB
 // wider than that (rounded down to a multiple of 32, at least 32).  0: SB.
 // The entry points without one use NB / 2 for NB >= 512 (a multiple of 64),
 // which only matters for the tile sizes they take.
+constexpr double ONE_STREAM_WORK = 2147483648.0;
 constexpr int half_tile_hmb(int NB) { return (NB >= 512 && NB % 64 == 0) ? NB / 2 : 0; }
 
 template <class T>
@@ -1381,45 +1398,54 @@ int potrf_tiles(Ctx *c, int N, int NB, T *dT, int *info, bool bf16_split, T *ws,
         split = (__bf16 *)ws_get(c, WS_BF16_PANEL, (size_t)(MT - 2) * 2 * NB * NB * sizeof(__bf16));
         if (!split) return -3;
     }
+    // steps from k1 on run on one stream
+    int k1 = 0;
+    const double one = 0.5 * NB * NB * NB * sizeof(T) / 8;
+    while (k1 < MT - 1 && (MT - k1 - 1.0) * (MT - k1) * one > ONE_STREAM_WORK) k1++;
+    const hipStream_t sp = k1 > 0 ? c->s_panel : c->s_main;
     auto panel = [&](int k) -> int {
-        return launch_panel<T>(c, c->s_panel, dT, N, NB, MT, k, ws + (k & 1) * wsz, sb, true, k + 1, MT - k - 1);
+        return launch_panel<T>(c, sp, dT, N, NB, MT, k, ws + (k & 1) * wsz, sb, true, k + 1, MT - k - 1);
+    };
+    auto pass = [&](hipEvent_t e, hipStream_t from, hipStream_t to) -> int {
+        MI_CHECK(hipEventRecord(e, from));
+        MI_CHECK(hipStreamWaitEvent(to, e, 0));
+        return 0;
     };
 
     MI_CHECK(hipEventRecord(c->t0, c->s_main));
     k_fill_int<<<1, 64, 0, c->s_main>>>(c->d_info, 0, 1);
-    hipEvent_t start = ev();
-    MI_CHECK(hipEventRecord(start, c->s_main));
-    MI_CHECK(hipStreamWaitEvent(c->s_panel, start, 0));
+    if (sp != c->s_main && (rc = pass(ev(), c->s_main, sp))) return rc;
 
-    // panel 0
     if ((rc = panel(0))) return rc;
-    hipEvent_t pk = ev();                          // TRSM(k) done
-    MI_CHECK(hipEventRecord(pk, c->s_panel));
     hipEvent_t col_ready = nullptr;                // column k+1 updated by step k-1
 
     for (int k = 0; k < MT - 1; k++) {
-        // panel stream: column k+1 by step k, then the next panel
-        if (col_ready) MI_CHECK(hipStreamWaitEvent(c->s_panel, col_ready, 0));
-        if ((rc = launch_update<T>(c, c->s_panel, dT, N, NB, MT, k, k + 1, k + 2, bf16_split, true))) return rc;
+        if (k >= k1) {
+            if (k == k1 && k > 0 && (rc = pass(ev(), c->s_main, sp))) return rc;
+            if ((rc = launch_update<T>(c, sp, dT, N, NB, MT, k, k + 1, MT, bf16_split, true))) return rc;
+            if ((rc = panel(k + 1))) return rc;
+            continue;
+        }
+        // panel stream: column k+1 by step k, then the next panel; main
+        // stream, once column k+1 is done: the look-ahead column k+2, then
+        // the bulk of step k
+        if (col_ready) MI_CHECK(hipStreamWaitEvent(sp, col_ready, 0));
+        if ((rc = launch_update<T>(c, sp, dT, N, NB, MT, k, k + 1, k + 2, bf16_split, true))) return rc;
+        if ((rc = pass(ev(), sp, c->s_main))) return rc;
         if ((rc = panel(k + 1))) return rc;
-        hipEvent_t pk_next = ev();
-        MI_CHECK(hipEventRecord(pk_next, c->s_panel));
-        // main stream: the look-ahead column k+2, then the bulk of step k
-        MI_CHECK(hipStreamWaitEvent(c->s_main, pk, 0));
         col_ready = nullptr;
-        const __bf16 *sp = (split && k + 2 < MT) ? split : nullptr;
-        if (sp && (rc = launch_split_panel(c, c->s_main, (const float *)dT, N, NB, MT, k, k + 2, split))) return rc;
+        const __bf16 *im = (split && k + 2 < MT) ? split : nullptr;
+        if (im && (rc = launch_split_panel(c, c->s_main, (const float *)dT, N, NB, MT, k, k + 2, split))) return rc;
         if (k + 2 < MT) {
-            if ((rc = launch_update<T>(c, c->s_main, dT, N, NB, MT, k, k + 2, k + 3, bf16_split, false, sp, k + 2)))
+            if ((rc = launch_update<T>(c, c->s_main, dT, N, NB, MT, k, k + 2, k + 3, bf16_split, false, im, k + 2)))
                 return rc;
             col_ready = ev();
             MI_CHECK(hipEventRecord(col_ready, c->s_main));
         }
-        if ((rc = launch_update<T>(c, c->s_main, dT, N, NB, MT, k, k + 3, MT, bf16_split, false, sp, k + 2)))
+        if ((rc = launch_update<T>(c, c->s_main, dT, N, NB, MT, k, k + 3, MT, bf16_split, false, im, k + 2)))
             return rc;
-        pk = pk_next;
     }
-    MI_CHECK(hipStreamWaitEvent(c->s_main, pk, 0));
+    if (sp != c->s_main && (rc = pass(ev(), sp, c->s_main))) return rc;
     MI_CHECK(hipEventRecord(c->t1, c->s_main));
     if (!wait) return 0;                           // info stays in d_info[0]
     int h_info = 0;

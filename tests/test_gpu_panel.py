@@ -230,3 +230,20 @@ def test_batched_block_edges(dev, dtype, solve):
             assert np.abs(x - want).max() <= 64 * (n + 16) * eps * max(1.0, np.abs(want).max()), n
         ao += n * n
         bo += n
+
+
+@pytest.mark.parametrize("N,NB,dtype", [(3584, 256, np.float64), (4101, 256, np.float64), (4700, 256, np.float64),
+                                        (2500, 93, np.float64), (5900, 256, np.float32), (6200, 320, np.float32)])
+def test_two_streams_then_one(dev, po, N, NB, dtype):
+    """Steps whose updates are large enough for a bulk beside the panels, none
+    to several of them, before the ones that run on one stream."""
+    A = po.dplgsy_full(N, float(N), 3872).astype(dtype).astype(np.float64)
+    ref = np.linalg.cholesky(A)
+    for _ in range(2):
+        L, info = factor(dev, A, NB, dtype)
+        assert info == 0
+        assert np.abs(L - ref).max() <= (1e-12 if dtype == np.float64 else 64 * EPS32) * np.abs(ref).max()
+    bad = A.copy()
+    bad[N - 3, N - 3] = -1.0
+    _, info = factor(dev, bad, NB, dtype)
+    assert info == N - 2
