@@ -108,49 +108,182 @@ template <int C, class T> __device__ __forceinline__ void fmac_rest(T *a, T m, T
     }
 }
 
-// 1 / sqrt(x); NaN for x <= 0, NaN and infinity (and in FP32 for denormals,
-// which v_rsq_f32 takes for zero)
-__device__ __forceinline__ double rsq_refined(double x)
+// The sweep over a 16 x 16 block, four copies of it side by side in the rows
+// of 16 lanes: lane fr holds row fr of D in v[] and row fr of the identity in
+// x[].  Column c: v[c] becomes L(fr, c), x[c] becomes W(c, fr) (W = L^{-1});
+// both arrays lose the multiple of the column.  Entries above the diagonal
+// hold arbitrary values throughout and never reach another lane.
+//
+// A lone wave issues one instruction every four cycles and waits out every
+// dependent one, so the order of the instructions is the sweep's time.  It
+// is laid down here, at compile time: the chain from pivot to pivot (broadcast,
+// reciprocal root, its correction, the scaled column, the next pivot) with
+// the FMAs of earlier columns in its gaps, those on v first, those on x
+// behind them as far as they fill gaps; what is left of x comes last.  Alone
+// on its SIMD a sweep takes 2340 cycles (FP64; 389 instructions, 16 of them
+// the 16-cycle root) and 2090 (FP32).  The root's correction is one
+// third-order step in FP64 (v_rsq_f64 is good to about 2^-26) and one Newton
+// step in FP32; a pivot <= 0, infinite or NaN (in FP32 also a denormal, which
+// v_rsq_f32 takes for zero) comes out as NaN.
+//
+// The instructions are volatile, so that this order stays; the two wait
+// states between a write and its read by DPP, and the one after a root, are
+// part of the plan and not the compiler's to insert.
+enum SweepOp { S_BCAST, S_RSQ, S_T, S_E, S_U, S_W, S_RD, S_COL, S_PIVOT, S_V, S_XS, S_X, S_NOP };
+struct SweepStep { int op, c, j; };
+struct SweepPlan {
+    SweepStep step[512] = {};
+    int n = 0;
+};
+constexpr SweepPlan sweep_plan(bool f64)
 {
-    // v_rsq_f64 is good to about 2^-26; one third-order step leaves rounding
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-(x * y), y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
+    SweepPlan p{};
+    SweepStep vq[128] = {}, xq[160] = {};              // FMAs on v and x in their order
+    int vn = 0, v0 = 0, xn = 0, x0 = 0;
+    int col = -8;                                      // place of the latest S_COL, and its column
+    int colc = -1;
+    auto put = [&](int op, int c, int j) {
+        p.step[p.n].op = op;
+        p.step[p.n].c = c;
+        p.step[p.n].j = j;
+        p.n++;
+    };
+    // one FMA if there is one; a lane broadcast must not read a register
+    // that one of the two instructions before it wrote
+    auto fill = [&]() -> bool {
+        const bool fresh = p.n - col <= 2;
+        if (v0 < vn && !(fresh && vq[v0].c == colc)) {
+            put(S_V, vq[v0].c, vq[v0].j);
+            v0++;
+            return true;
+        }
+        if (x0 < xn && !(xq[x0].op == S_X && fresh && xq[x0].c == colc)) {
+            put(xq[x0].op, xq[x0].c, xq[x0].j);
+            x0++;
+            return true;
+        }
+        return false;
+    };
+    auto gap = [&](int want, int need) {
+        for (int i = 0; i < want; i++)
+            if (!fill() && i < need) put(S_NOP, 0, 0);
+    };
+    put(S_NOP, 0, 0);
+    put(S_NOP, 0, 0);
+    for (int c = 0; c < DB; c++) {
+        put(S_BCAST, c, 0);
+        gap(1, 0);
+        put(S_RSQ, c, 0);
+        gap(4, 1);
+        put(S_T, c, 0);
+        gap(2, 0);
+        put(S_E, c, 0);
+        gap(1, 0);
+        put(S_U, c, 0);
+        if (f64) put(S_W, c, 0);
+        gap(1, 0);
+        put(S_RD, c, 0);
+        xq[xn].op = S_XS;
+        xq[xn].c = c;
+        xn++;
+        gap(1, 0);
+        while (v0 < vn && vq[v0].j <= c + 1) fill();   // what the next pivot still lacks
+        put(S_COL, c, 0);
+        col = p.n - 1;
+        colc = c;
+        for (int j = c + 2; j < DB; j++) {
+            vq[vn].c = c;
+            vq[vn].j = j;
+            vn++;
+        }
+        for (int j = c + 1; j < DB; j++) {
+            xq[xn].op = S_X;
+            xq[xn].c = c;
+            xq[xn].j = j;
+            xn++;
+        }
+        if (c + 1 < DB) {
+            gap(2, 2);
+            put(S_PIVOT, c, c + 1);
+            gap(4, 2);
+        }
+    }
+    gap(2, 2);
+    while (fill()) {}
+    return p;
 }
-__device__ __forceinline__ float rsq_refined(float x)
+// Wait states: two instructions between a write of v[c] and its read by DPP,
+// one between a root and its first use.
+constexpr bool sweep_plan_ok(const SweepPlan &p)
 {
-    const float y = __builtin_amdgcn_rsqf(x);
-    const float e = fmaf(-(x * y), y, 1.0f);
-    return fmaf(y * e, 0.5f, y);
+    int wrote[DB] = {}, root = -1;
+    for (int i = 0; i < DB; i++) wrote[i] = -1;
+    for (int i = 0; i < p.n; i++) {
+        const SweepStep &t = p.step[i];
+        if ((t.op == S_BCAST || t.op == S_PIVOT || t.op == S_V || t.op == S_X) && i - wrote[t.c] < 3) return false;
+        if (t.op == S_T && i - root < 2) return false;
+        if (t.op == S_RSQ) root = i;
+        if (t.op == S_COL) wrote[t.c] = i;
+        if (t.op == S_PIVOT || t.op == S_V) wrote[t.j] = i;
+    }
+    return true;
 }
+template <class T> struct SweepPlanOf {
+    static constexpr SweepPlan plan = sweep_plan(sizeof(T) == 8);
+    static_assert(sweep_plan_ok(plan), "wait states of the sweep");
+};
+template <class T> struct SweepTmp { T p, t, e, u, w, rd[DB]; };
 
-// One column of the sweep over a 16 x 16 block, four copies of it side by
-// side in the rows of 16 lanes: lane fr holds row fr of D in v[] and row fr
-// of the identity in x[].  Column C: v[C] becomes L(fr, C), x[C] becomes
-// W(C, fr) (W = L^{-1}); both arrays lose the multiple of the column.
-// Entries above the diagonal hold arbitrary values throughout and never
-// reach another lane.  A lone wave issues one instruction every four
-// cycles, so the column costs its instruction count: the two FMA per later
-// column, and the pivot's chain.  Returns 1 / L(C, C).
-template <int C, class T> __device__ __forceinline__ T sweep_column(T *v, T *x)
+#define MI_SW(f64, f32, ...)                                                       \
+    do {                                                                           \
+        if constexpr (sizeof(T) == 8) asm volatile(f64 __VA_ARGS__);               \
+        else asm volatile(f32 __VA_ARGS__);                                        \
+    } while (0)
+template <class T, int I> __device__ __forceinline__ void sweep_step(T *v, T *x, SweepTmp<T> &t)
 {
-    const T rd = rsq_refined(row_bcast<C>(v[C]));
-    const T m = v[C] * rd;
-    if constexpr (C + 1 < DB) fmac_bcast<C + 1, 1>(v, m, m);    // the next pivot first
-    x[C] = x[C] * rd;
-    fmac_rest<C + 2>(v, m, m);
-    fmac_rest<C + 1>(x, m, x[C]);
-    v[C] = m;
-    return rd;
+    constexpr SweepStep s = SweepPlanOf<T>::plan.step[I];
+    constexpr int c = s.c, j = s.j;
+    if constexpr (s.op == S_NOP) asm volatile("s_nop 0");
+    else if constexpr (s.op == S_BCAST)
+        MI_SW("v_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf",
+              "v_mov_b32_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf", : "=v"(t.p) : "v"(v[c]), "n"(c));
+    else if constexpr (s.op == S_RSQ) MI_SW("v_rsq_f64 %0, %1", "v_rsq_f32 %0, %1", : "=v"(t.rd[c]) : "v"(t.p));
+    else if constexpr (s.op == S_T)
+        MI_SW("v_mul_f64 %0, -%1, %2", "v_mul_f32 %0, -%1, %2", : "=v"(t.t) : "v"(t.p), "v"(t.rd[c]));
+    else if constexpr (s.op == S_E)
+        MI_SW("v_fma_f64 %0, %1, %2, 1.0", "v_fma_f32 %0, %1, %2, 1.0", : "=v"(t.e) : "v"(t.t), "v"(t.rd[c]));
+    else if constexpr (s.op == S_U)
+        MI_SW("v_mul_f64 %0, %1, %2", "v_mul_f32 %0, %1, %2", : "=v"(t.u) : "v"(t.rd[c]), "v"(t.e));
+    else if constexpr (s.op == S_W) asm volatile("v_fma_f64 %0, %1, %2, 0.5" : "=v"(t.w) : "v"(t.e), "s"(T(0.375)));
+    else if constexpr (s.op == S_RD) {
+        if constexpr (sizeof(T) == 8) asm volatile("v_fmac_f64 %0, %1, %2" : "+v"(t.rd[c]) : "v"(t.u), "v"(t.w));
+        else asm volatile("v_fma_f32 %0, %1, 0.5, %0" : "+v"(t.rd[c]) : "v"(t.u));
+    } else if constexpr (s.op == S_COL)
+        MI_SW("v_mul_f64 %0, %0, %1", "v_mul_f32 %0, %0, %1", : "+v"(v[c]) : "v"(t.rd[c]));
+    else if constexpr (s.op == S_XS)
+        MI_SW("v_mul_f64 %0, %0, %1", "v_mul_f32 %0, %0, %1", : "+v"(x[c]) : "v"(t.rd[c]));
+    else if constexpr (s.op == S_X)
+        MI_SW("v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf",
+              "v_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf",
+              : "+v"(x[j]) : "v"(v[c]), "v"(x[c]), "n"(j));
+    else
+        MI_SW("v_fmac_f64_dpp %0, -%1, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf",
+              "v_fmac_f32_dpp %0, -%1, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf",
+              : "+v"(v[j]) : "v"(v[c]), "n"(j));
+}
+#undef MI_SW
+template <class T, int... I>
+__device__ __forceinline__ void sweep_steps(T *v, T *x, SweepTmp<T> &t, std::integer_sequence<int, I...>)
+{
+    (sweep_step<T, I>(v, x, t), ...);
 }
 // True when a pivot was not an ordinary positive number: its NaN reciprocal
 // root reaches every later column.
-template <class T, int... C>
-__device__ __forceinline__ bool sweep_fast(T *v, T *x, std::integer_sequence<int, C...>)
+template <class T> __device__ __forceinline__ bool sweep_fast(T *v, T *x)
 {
-    T rd = T(0);
-    ((rd = sweep_column<C>(v, x)), ...);
-    return rd != rd;
+    SweepTmp<T> t;
+    sweep_steps(v, x, t, std::make_integer_sequence<int, SweepPlanOf<T>::plan.n>());
+    return t.rd[DB - 1] != t.rd[DB - 1];
 }
 
 // The same sweep with square root and division, for blocks with a pivot that
@@ -221,7 +354,10 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
                                            OX &&out_x)
 {
     typedef typename MF<T>::v4 V4;
-    constexpr int NK = NW - 1;                              // worker waves
+    // worker waves; of eight, wave 4 is none: it shares the SIMD of wave 0,
+    // where every MFMA would hold up the sweep
+    constexpr bool APART = NW == 8;
+    constexpr int NK = APART ? NW - 2 : NW - 1;
     constexpr int NBLK = NBK * (NBK + 1) / 2 - 1;           // blocks besides (0, 0)
     constexpr int SLOTS = (NBLK + NK - 1) / NK;
     int tid = threadIdx.x;
@@ -287,7 +423,7 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
         for (int p = 0; p < nb; p++) {
 #pragma unroll
             for (int c = 0; c < DB; c++) x[c] = fr == c ? T(1) : T(0);
-            if (__any(sweep_fast(v, x, std::make_integer_sequence<int, DB>()))) {
+            if (__any(sweep_fast(v, x))) {
                 int fail = 0;
 #pragma unroll
                 for (int c = 0; c < DB; c++) {
@@ -327,11 +463,12 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
     } else {
         // slot u: block t = wave + NK u of the list (0,0) (1,0) .. (NBK-1,0)
         // (1,1) (2,1) .. ; bi, bj are wave-uniform, bj = -1 where there is none
+        const int worker = !APART || wave < 4 ? wave : wave == 4 ? NBK * NBK : wave - 1;
         V4 blk[SLOTS];
         int bi[SLOTS], bj[SLOTS];
 #pragma unroll
         for (int u = 0; u < SLOTS; u++) {
-            int t = wave + NK * u, j = 0;
+            int t = worker + NK * u, j = 0;
             while (j < NBK && t >= NBK - j) { t -= NBK - j; j++; }
             bj[u] = j < NBK && j + t < nb ? j : -1;
             bi[u] = j + t;
@@ -371,7 +508,7 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
                     out_x(bi[u], p, -blk[u]);
                 }
             // what wave 0 left: L_pp, W_p and X(p + 1, p)
-            if (wave == NK) {
+            if (wave == (APART ? 4 : NK)) {
                 out_w(p, w);
                 if (p + 1 < nb) {
                     const V4 mx = get(xl(p + 1, p));
@@ -393,27 +530,207 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
 // op: the operand images for k_panel_solve (see OPB); info = info_base + j of
 // the first non-positive pivot j (1-based), as CORE_dpotrf reports it.
 //
-// Measured (n = 128): 20 us in FP64, 21 us in FP32 inside a factorization, of
-// which 2.5 us load the blocks; per 16 columns 3100-3900 cycles of sweep and
-// 1400 cycles of hand-off.  A whole-tile factor of 32-column blocks with
-// v_readlane broadcasts, W_jj on the chain and the tile in memory took 145 us
-// for 256 columns and 367 us (FP32) for 512.
+// As diag_factor, but laid out for the shortest chain, since nothing else of
+// a panel runs beside it.  The four rows of 16 lanes of a sweep hold the same
+// D and different blocks in x: what becomes W = L^{-1} for the identity
+// becomes X = C L^{-T} for the rows of a block C below.  Waves 0 and 1 sweep
+// D_p together with the identity and all blocks C(i, p):
+//   wave 0   I, C(p+1, p) .. C(p+3, p), then D_{p+1} -= X X^T,
+//   wave 1   C(p+4, p) .. C(p+7, p).
+// Nothing is solved through W, and one exchange through LDS hands X(., p) to
+//   waves 2, 3, 6, 7 (the other two SIMDs): C(i, p+1) -= X(i, p) X(p+1, p)^T
+//            for the next sweep, then, while it runs, the rest of the blocks,
+//            which they hold in registers;
+//   waves 4, 5 (beside the sweeping waves, without products): the stores.
+// An MFMA on a sweeping wave's SIMD would hold it up: FP64 products and FP64
+// FMAs share their units.
+// A block's rows travel as rows of 16 elements, XP apart.
+//
+// n = 128, FP64, cycles a 16-column step (clock reads included): sweep 2450,
+// X out and barrier 440, D_{p+1} beside C(., p+1) 1000 - 1600, rows read back
+// 440.  With the solve through W on wave 0's chain and products on its SIMD:
+// 3100 - 3900 + 750 + 1500 + 400.  In a factorization 20.5 -> 17.5 us
+// (N = 4096, NB = 256), 14.0 -> 11.6 us for 93 columns; FP32 14.2 -> 12.6 us
+// (N = 3200, NB = 320).
 template <class T>
-__global__ __launch_bounds__(512, 2) void k_diag_factor(T *__restrict__ A, int n, int ld, int info_base,
+__global__ __launch_bounds__(512, sizeof(T) == 8 ? 2 : 4) void k_diag_factor(T *__restrict__ A, int n, int ld, int info_base,
                                                        int *__restrict__ d_info, T *__restrict__ op)
 {
     typedef typename MF<T>::v4 V4;
-    __shared__ DiagLds<T> ds;
-    __shared__ T x[DBN][OPI];
-    __shared__ __align__(16) T w[2][DB * DIAG_WP];
+    constexpr int XP = DIAG_WP, XS = DB * XP;
+    // FP32: 31 KB, what two workgroups of the trailing update leave of a CU
+    __shared__ __align__(16) T xr[2][DBN][XS];             // by p & 1: X(i, p), W_p (by columns) for i = 0
+    __shared__ __align__(16) T cr[DBN][XS];                // C(i, p + 1) for the sweep
+    __shared__ __align__(16) T ll1[XS];                    // L_pp of odd p (even p: cr[0])
+    __shared__ __align__(16) T dl[XS];                     // D_{p+1}
+    __shared__ T hd[OPI];                                  // D_{p+1} before step p, [s][lane]
+    __shared__ int fail;
     __builtin_amdgcn_s_setprio(2);
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) ds.fail = 0;
-    const int f = diag_factor<T, 8, DBN>(
-        A, n, ld, ds, [&](int i, int) { return x[i]; }, [&](int p) { return w[p & 1]; },
-        [&](int p, const V4 &b) { *(V4 *)(op + (int64_t)p * OPB + 4 * lane) = b; },
-        [&](int i, int p, const V4 &b) { *(V4 *)(op + (int64_t)p * OPB + (i - p) * OPI + 4 * lane) = b; });
-    if (threadIdx.x == 0 && f) atomicCAS(d_info, 0, info_base + f);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4;
+    const int nb = (n + DB - 1) / DB;
+    if (threadIdx.x == 0) fail = 0;
+
+    // element (r, c) of A; past n the identity, so that a ragged block
+    // factors like a whole one
+    auto elem = [&](int r, int c) -> T {
+        const T a = A[(int64_t)min(c, n - 1) * ld + min(r, n - 1)];
+        return r < n && c < n ? a : (r == c ? T(1) : T(0));
+    };
+    auto row_out = [&](T *img, const T *v) {               // row fr of a block
+#pragma unroll
+        for (int c = 0; c < DB; c++) img[fr * XP + c] = v[c];
+    };
+    auto row_in = [&](const T *img, T *v) {
+#pragma unroll
+        for (int c = 0; c < DB; c++) v[c] = img[fr * XP + c];
+    };
+    // operand / accumulator registers of a block kept by rows
+    auto get = [&](const T *img) -> V4 {
+        V4 b;
+#pragma unroll
+        for (int q = 0; q < 4; q++) b[q] = img[fr * XP + MF<T>::row(q, fk)];
+        return b;
+    };
+    auto put = [&](T *img, const V4 &b) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) img[fr * XP + MF<T>::row(q, fk)] = b[q];
+    };
+    auto prod = [&](V4 c, const V4 &xj, const V4 &xi) -> V4 {    // C - X_i X_j^T
+#pragma unroll
+        for (int s = 0; s < 4; s++) c = MF<T>::mfma(-xj[s], xi[s], c);
+        return c;
+    };
+
+    // every role runs the same two barriers a step
+    if (wave < 2) {
+        __builtin_amdgcn_s_setprio(3);
+        T v[DB], x[DB];
+        const int g = 4 * wave + fk;                       // block p + g of the step; 0: the identity
+        auto unit = [&]() {
+#pragma unroll
+            for (int c = 0; c < DB; c++) x[c] = fr == c ? T(1) : T(0);
+        };
+#pragma unroll
+        for (int c = 0; c < DB; c++) v[c] = elem(fr, c);
+        if (fk == 0) row_out(dl, v);                       // by both waves, the same values
+        if (g == 0) {
+            unit();
+        } else if (g < nb) {
+#pragma unroll
+            for (int c = 0; c < DB; c++) x[c] = elem(DB * g + fr, c);
+            row_out(cr[g], x);
+        } else {
+            unit();
+        }
+        for (int p = 0; p < nb; p++) {
+            const bool mine = p + g < nb;
+            if (__any(sweep_fast(v, x))) {
+                int f = 0;
+                row_in(dl, v);
+                if (g > 0 && mine) row_in(cr[p + g], x);
+                else unit();
+                sweep_exact(v, x, fr, &f, std::make_integer_sequence<int, DB>());
+                if (f && tid == 0) fail = DB * p + f;
+            }
+            if (mine) row_out(xr[p & 1][g == 0 ? 0 : p + g], x);
+            __syncthreads();
+            if (fail) break;
+            if (wave == 1) {
+                if (fk == 0) row_out(p & 1 ? ll1 : cr[0], v);
+            } else if (p + 1 < nb) {
+                V4 d0;
+#pragma unroll
+                for (int q = 0; q < 4; q++) d0[q] = hd[64 * q + lane];
+                const V4 xx = get(xr[p & 1][p + 1]);
+                put(dl, prod(d0, xx, xx));
+            }
+            __syncthreads();
+            if (p + 1 < nb) {
+                row_in(dl, v);
+                if (g > 0 && p + 1 + g < nb) row_in(cr[p + 1 + g], x);
+                else unit();
+            }
+        }
+    } else if ((wave & 3) >= 2) {
+        // slot u: block t = worker + 4 u of the list (1,1) (2,1) .. (7,1) (2,2)
+        // (3,2) .. ; bi, bj are wave-uniform, bj = -1 where there is none
+        constexpr int NK = 4, SLOTS = (DBN * (DBN - 1) / 2 + NK - 1) / NK;
+        const int worker = (wave & 1) + 2 * (wave >> 2);
+        int at[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) at[q] = MF<T>::row(q, fk) * ld + fr;
+        V4 blk[SLOTS];
+        int bi[SLOTS], bj[SLOTS];
+#pragma unroll
+        for (int u = 0; u < SLOTS; u++) {
+            int t = worker + NK * u, j = 1;
+            while (j < DBN && t >= DBN - j) { t -= DBN - j; j++; }
+            bj[u] = j < DBN && j + t < nb ? j : -1;
+            bi[u] = j + t;
+            if (bj[u] >= 0) {
+                const T *b = A + (int64_t)DB * j * ld + DB * bi[u];
+                if (DB * bi[u] + DB <= n) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) blk[u][q] = b[at[q]];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) blk[u][q] = elem(DB * bi[u] + fr, DB * j + MF<T>::row(q, fk));
+                }
+            }
+        }
+        auto put_d = [&](const V4 &b) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) hd[64 * q + lane] = b[q];
+        };
+        if (bj[0] == 1 && bi[0] == 1) put_d(blk[0]);
+        for (int p = 0; p < nb; p++) {
+            const T (*xp)[XS] = xr[p & 1];
+            __syncthreads();
+            if (fail) break;
+#pragma unroll
+            for (int u = 0; u < SLOTS; u++)
+                if (bj[u] == p + 1 && bi[u] > p + 1) put(cr[bi[u]], prod(blk[u], get(xp[p + 1]), get(xp[bi[u]])));
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < SLOTS; u++)
+                if (bj[u] > p + 1) {
+                    blk[u] = prod(blk[u], get(xp[bj[u]]), get(xp[bi[u]]));
+                    if (bj[u] == p + 2 && bi[u] == p + 2) put_d(blk[u]);
+                }
+        }
+    } else {
+        for (int p = 0; p < nb; p++) {
+            __syncthreads();
+            if (fail) break;
+            __syncthreads();
+            for (int i = p + 1 + (wave & 1); i < nb; i += 2) {
+                const V4 b = get(xr[p & 1][i]);
+                const int r = DB * i + fr;
+                if (r < n) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) A[(int64_t)(DB * p + MF<T>::row(q, fk)) * ld + r] = b[q];
+                }
+                *(V4 *)(op + (int64_t)p * OPB + (i - p) * OPI + 4 * lane) = -b;
+            }
+            if (wave == 4) {
+                V4 w;
+#pragma unroll
+                for (int q = 0; q < 4; q++) w[q] = xr[p & 1][0][MF<T>::row(q, fk) * XP + fr];
+                *(V4 *)(op + (int64_t)p * OPB + 4 * lane) = w;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int c = 4 * u + fk;
+                    if (c <= fr && DB * p + fr < n) A[(int64_t)(DB * p + c) * ld + DB * p + fr] = (p & 1 ? ll1 : cr[0])[fr * XP + c];
+                }
+            }
+        }
+    }
+    if (tid == 0 && fail) atomicCAS(d_info, 0, info_base + fail);
 }
 
 // ---------------------------------------------------------------------------
