@@ -899,16 +899,21 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
     // any of them is still the sentinel (for the last block too: a cheaper
     // poll of one value per producer wave first costs one more round trip
     // per link, 1-2 % of a sweep)
-    // true once this wait has to end without its values: the abort word is
-    // set, or this wait outlived its budget (then it sets the word)
     int *abort_word = ticket + 1;
     // (global-memory pointers: a generic one would make every later wait
     // for a vector load a wait for all of them)
     typedef __attribute__((address_space(1))) int GI;
-    auto give_up = [&](long long t_end) -> bool {
+    // the abort word, read beside the X that a wait reads again: one round
+    // trip to memory a turn
+    auto read_abort = [&]() -> int {
         GI *ap = (GI *)abort_word;
         asm volatile("" : "+v"(ap));
-        if (__hip_atomic_load(ap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return true;
+        return __hip_atomic_load(ap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // true once this wait has to end without its values: the abort word is
+    // set (ab), or this wait outlived its budget (then it sets the word)
+    auto give_up = [&](int ab, long long t_end) -> bool {
+        if (__any(ab)) return true;
         if (wait_ticks > 0 && (long long)__builtin_amdgcn_s_memrealtime() < t_end) return false;
         GI *wp = (GI *)abort_word;
         asm volatile("" : "+v"(wp));
@@ -919,7 +924,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
         constexpr int NH = sizeof(bx) / sizeof(bx[0]);
         const T *xh = xs + (int64_t)h * (WV_RB * RHSB);
         const long long t_end = (long long)__builtin_amdgcn_s_memrealtime() + wait_ticks;
-        if (wait_ticks == 0) (void)give_up(t_end);   // a zero budget ends every wait at once
+        if (wait_ticks == 0) (void)give_up(0, t_end);   // a zero budget ends every wait at once
         for (;;) {
             int ok = 1;
             if constexpr (sizeof(T) == 8) {
@@ -946,9 +951,9 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
                         bx[hl][2 * kp + 1] = __builtin_bit_cast(T, hi);
                     }
             }
+            const int ab = read_abort();
             if (__all(ok)) break;
-            if (__any(give_up(t_end))) break;
-            __builtin_amdgcn_s_sleep(1);
+            if (give_up(ab, t_end)) break;
         }
 #pragma unroll
         for (int hl = 0; hl < NH; hl++)
@@ -1008,12 +1013,12 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
             if (!ready(xc)) {
                 // the bounded wait of wait_x, reading into the same registers
                 const long long t_end = (long long)__builtin_amdgcn_s_memrealtime() + wait_ticks;
-                if (wait_ticks == 0) (void)give_up(t_end);
+                if (wait_ticks == 0) (void)give_up(0, t_end);
                 for (;;) {
-                    if (__any(give_up(t_end))) break;
-                    __builtin_amdgcn_s_sleep(1);
                     read_x(blk(s), xc);
+                    const int ab = read_abort();
                     if (ready(xc)) break;
+                    if (give_up(ab, t_end)) break;
                 }
             }
             T bx[2][8];
@@ -1119,6 +1124,436 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
             wv_store(xg + wv_xs<T, TRANS>(rb, fr), x[t][q]);
             if (r0 + rb < N && fr < nr) B[(int64_t)fr * ldb + r0 + rb] = x[t][q];
         }
+}
+
+// ---------------------------------------------------------------------------
+// The same wavefront for at most R <= 4 right-hand sides, on the VALU.  An
+// MFMA spends its 64 (FP64) cycles on 16 columns whatever their number, and a
+// link's 128 x 128 product then is 4096 cycles of a SIMD; with one column it
+// is 128 FMA.  L and M_g enter a lane as 16-byte pieces (VEC elements), X as
+// the broadcast source of a DPP FMA (lane i of each row of 16):
+//   forward    wave w, columns 16 w .. of the earlier block: a lane holds VEC
+//              rows, piece i is column CPL i + hw (FP32: the half waves hw
+//              take every other column); the eight waves' sums meet in LDS.
+//   backward, and the products with W_g and M_g
+//              wave w, rows 16 w .. of the block: lane (fr, fk) holds row fr,
+//              piece q covers the columns VEC (4 q + fk) ..; the four lane
+//              groups' sums meet by shuffles.
+//   backward, catch-up (COLS)
+//              wave w, columns 16 w .. of the block, whose sums a lane keeps
+//              for its VEC rows of the earlier block: whole columns load as
+//              1 KB runs (16 columns x 64 bytes an instruction instead: FP64
+//              252 us a sweep at N = 8192, against 167).
+// So the last link needs no barrier: each wave waits for the 128 values,
+// forms its 16 rows and stores them.  Rows past N are stored as zeros.
+//
+// Bound by the memory while many blocks are behind the front, then by the
+// links (one hand-off through memory and 0.2 us of FMAs each).  One
+// right-hand side, a sweep forward / backward, us, MFMA kernel -> this:
+//   FP64  N = 32768 1630 / 1703 -> 939 / 940 (4.3 GB: 4.6 TB/s)
+//         N = 8192   369 / 393  -> 142 / 167
+//   FP32  N = 3200    91 / 98   ->  31 / 33
+#define WV_FMAC(f64, f32, i)                                                                                       \
+    if constexpr (sizeof(T) == 8) asm volatile(f64 " %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"        \
+                                               : "+v"(a) : "v"(x), "v"(l), "n"(i));                                \
+    else asm volatile(f32 " %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(x), "v"(l), "n"(i))
+template <int I, class T> __device__ __forceinline__ void wv_fmac(T &a, T x, T l)
+{
+    WV_FMAC("v_fmac_f64_dpp", "v_fmac_f32_dpp", I);
+}
+#undef WV_FMAC
+// a[e][r] += (value of lane i of x[e or 0][r]) * l[i][e], pieces I of l
+template <class T, int XV, int R, class V, int... I>
+__device__ __forceinline__ void wv_fma(T (&a)[16 / sizeof(T)][R], T (&x)[XV][R], const V *l, std::integer_sequence<int, I...>)
+{
+    // two wait states between the last write of x and its first DPP read
+#pragma unroll
+    for (int e = 0; e < XV; e++)
+#pragma unroll
+        for (int r = 0; r < R; r++) asm volatile("" : "+v"(x[e][r]));
+    asm volatile("s_nop 1");
+    auto piece = [&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+#pragma unroll
+        for (int e = 0; e < (int)(16 / sizeof(T)); e++)
+#pragma unroll
+            for (int r = 0; r < R; r++) wv_fmac<i>(a[e][r], x[XV == 1 ? 0 : e][r], (T)l[i][e]);
+    };
+    (piece(std::integral_constant<int, I>()), ...);
+}
+
+template <class T, bool TRANS, int R>
+__global__ __launch_bounds__(512, 1) void k_trsm_vec(const T *__restrict__ Tt, int N, int NB, int MT,
+                                                    const T *__restrict__ W128, const T *__restrict__ Mlink,
+                                                    T *__restrict__ B, int ldb, int nr, T *__restrict__ xs,
+                                                    int *__restrict__ ticket, long long wait_ticks)
+{
+    typedef typename WvSent<T>::U U;
+    constexpr int VEC = 16 / (int)sizeof(T), NL = 32 / VEC;   // elements of a piece, pieces of a lane
+    constexpr int LPC = 128 / VEC, CPL = 64 / LPC;            // forward: lanes a column, columns a load
+    constexpr bool COLS = TRANS && sizeof(T) * R <= 16;       // backward by whole columns, as registers allow
+    constexpr bool LATE_M = sizeof(T) == 8 && TRANS && R > 1;        // no registers for M_g beside two blocks of L
+    constexpr int XV = TRANS ? VEC : 1;                       // values of X a lane and right-hand side
+    constexpr int NBUF = sizeof(T) == 8 || R == 4 ? 2 : 3;    // blocks of L in flight
+    constexpr bool TWO = sizeof(T) * R > 16;                  // the waves' sums go through LDS in two turns
+    constexpr int NP = TRANS ? 1 : (TWO ? 4 : 8) * CPL;
+    typedef T vec __attribute__((ext_vector_type(VEC)));
+    typedef std::make_integer_sequence<int, NL> Pieces;
+    __shared__ __align__(16) T Ws[16384];                     // op(W)(row, VEC c + e) at (128 c + row) VEC + e
+    __shared__ __align__(16) T Ps[NP][R][128];                // partial sums; then (backward) y
+    __shared__ int s_g;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4, fq = fr % NL;
+    const int nwg = (N + WV_RB - 1) / WV_RB;
+    if (tid == 0) {
+        int *tp = ticket;
+        asm volatile("" : "+v"(tp));
+        s_g = atomicAdd(tp, 1);
+    }
+    __syncthreads();
+    const int g = __builtin_amdgcn_readfirstlane(TRANS ? nwg - 1 - s_g : s_g);
+    const int r0 = g * WV_RB, nprev = TRANS ? nwg - 1 - g : g;
+    auto blk = [&](int s) { return TRANS ? nwg - 1 - s : s; };   // the s-th earlier block
+    const int64_t T2 = (int64_t)NB * NB;
+    // first element of tile column n, minus n tiles (so that tile row m adds m)
+    auto col_tiles = [&](int n) { return ((int64_t)n * MT - (int64_t)n * (n - 1) / 2 - n) * T2; };
+
+    // ---- pieces of L against earlier block h
+    int64_t lane_off;
+    int ti[4] = {0, 0, 0, 0}, wi[4] = {0, 0, 0, 0};           // tile and place in it of 32-groups (forward: of the columns)
+    int lm_t = 0, lm_r = 0;                                   // COLS: tile and place in it of the lane's rows
+    if constexpr (COLS) {
+        const int col = min(r0 + 16 * wave, (N - 1) & ~15), n = col / NB, row = (nwg - 1) * WV_RB + VEC * (lane % LPC);
+        lane_off = col_tiles(n) + (int64_t)(col - n * NB + lane / LPC) * NB;
+        lm_t = row / NB;
+        lm_r = row - lm_t * NB;
+    } else if (!TRANS) {
+        const int hw = lane / LPC, row = min(r0 + VEC * (lane % LPC), (N - 1) / VEC * VEC), m = row / NB;
+        lane_off = m * T2 + (row - m * NB) + (int64_t)hw * NB;
+        ti[0] = (16 * wave) / NB;
+        wi[0] = 16 * wave - ti[0] * NB;
+    } else {
+        const int col = min(r0 + 16 * wave + fr, N - 1), n = col / NB;
+        lane_off = col_tiles(n) + (int64_t)(col - n * NB) * NB + VEC * fk;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int row = max(nwg - 1, 0) * WV_RB + 32 * u;
+            ti[u] = row / NB;
+            wi[u] = row - ti[u] * NB;
+        }
+    }
+    // loads the pieces of the next block in order; the places move on
+    auto load_l = [&](vec (&l)[NL], int h) {
+        if constexpr (COLS) {
+            const int row = h * WV_RB + VEC * (lane % LPC), over = max(row - (N - 1) / VEC * VEC, 0), m = (row - over) / NB;
+            const bool edge = (h + 1) * WV_RB > N;            // the last rows of the matrix
+            const T *p = Tt + lane_off + (edge ? m * T2 + (row - over - m * NB) : lm_t * T2 + lm_r);
+#pragma unroll
+            for (int i = 0; i < NL; i++) l[i] = *(const vec *)(p + (int64_t)(CPL * i) * NB);
+            if (edge)
+#pragma unroll
+                for (int i = 0; i < NL; i++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) l[i][e] = row + e < N ? l[i][e] : T(0);
+            lm_r -= WV_RB;
+            while (lm_r < 0) { lm_r += NB; lm_t--; }
+        } else if (!TRANS) {
+            const T *p = Tt + col_tiles(ti[0]) + (int64_t)wi[0] * NB + lane_off;
+#pragma unroll
+            for (int i = 0; i < NL; i++) l[i] = *(const vec *)(p + (int64_t)(CPL * i) * NB);
+            wi[0] += WV_RB;
+            while (wi[0] >= NB) { wi[0] -= NB; ti[0]++; }
+        } else if ((h + 1) * WV_RB <= N) {
+#pragma unroll
+            for (int q = 0; q < NL; q++) {
+                const int u = 4 * VEC * q / 32;
+                l[q] = *(const vec *)(Tt + lane_off + ti[u] * T2 + wi[u] + 4 * VEC * q % 32);
+            }
+        } else {                                              // the last rows of the matrix
+#pragma unroll
+            for (int q = 0; q < NL; q++) {
+                const int row = min(h * WV_RB + VEC * (4 * q + fk), (N - 1) / VEC * VEC), m = row / NB;
+                const vec v = *(const vec *)(Tt + lane_off - VEC * fk + m * T2 + (row - m * NB));
+#pragma unroll
+                for (int e = 0; e < VEC; e++) l[q][e] = row + e < N ? v[e] : T(0);
+            }
+        }
+        if (TRANS && !COLS) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                wi[u] -= WV_RB;
+                while (wi[u] < 0) { wi[u] += NB; ti[u]--; }
+            }
+        }
+    };
+
+    // ---- X of an earlier block: XV consecutive values a lane
+    typedef __attribute__((address_space(1))) const unsigned long long G8;
+    typedef __attribute__((address_space(1))) const unsigned int G4;
+    auto read1 = [&](const T *p) -> U {
+        if constexpr (sizeof(T) == 8) return __hip_atomic_load((G8 *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else return __hip_atomic_load((G4 *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto read_v = [&](const T *xh, U (&x)[VEC][R], int c) {   // from column c
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const T *p = xh + r * 128 + c;
+            if constexpr (sizeof(T) == 8) {
+#pragma unroll
+                for (int e = 0; e < VEC; e++) x[e][r] = read1(p + e);
+            } else {
+#pragma unroll
+                for (int e = 0; e < VEC; e += 2) {
+                    const unsigned long long b = __hip_atomic_load((G8 *)(p + e), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    x[e][r] = (U)b;
+                    x[e + 1][r] = (U)(b >> 32);
+                }
+            }
+        }
+    };
+    auto read_x = [&](int h, U (&x)[XV][R]) {
+        const T *xh = xs + (int64_t)h * (WV_RB * RHSB);
+        if constexpr (TRANS) {
+            read_v(xh, x, COLS ? VEC * (lane % LPC) : VEC * (4 * fq + fk));
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) x[0][r] = read1(xh + r * 128 + 16 * wave + CPL * fq + lane / LPC);
+        }
+    };
+    auto ready = [&](auto &x) {
+        int ok = 1;
+        for (auto &xe : x)
+#pragma unroll
+            for (int r = 0; r < R; r++) ok &= xe[r] != WvSent<T>::v;
+        return __all(ok);
+    };
+    // Reads x again until it is complete, the abort word is set, or this wait
+    // outlived its budget (then it sets the word; a zero budget ends every
+    // wait at once).  X and the abort word are read together: one round trip
+    // to memory a turn.
+    typedef __attribute__((address_space(1))) int GI;
+    auto wait = [&](auto &x, auto &&again) {
+        if (wait_ticks > 0 && ready(x)) return;
+        const long long t_end = (long long)__builtin_amdgcn_s_memrealtime() + wait_ticks;
+        for (;;) {
+            again();
+            GI *ap = (GI *)(ticket + 1);
+            asm volatile("" : "+v"(ap));
+            const int ab = __hip_atomic_load(ap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (wait_ticks > 0 && ready(x)) return;
+            if (__any(ab)) return;
+            if (wait_ticks > 0 && (long long)__builtin_amdgcn_s_memrealtime() < t_end) continue;
+            __hip_atomic_store(ap, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+    };
+    auto value = [&](auto &u, auto &v) {
+#pragma unroll
+        for (int e = 0; e < (int)(sizeof(v) / sizeof(v[0])); e++)
+#pragma unroll
+            for (int r = 0; r < R; r++) v[e][r] = __builtin_bit_cast(T, u[e][r]);
+    };
+
+    // ---- link matrix: row 16 w + fr, piece q
+    vec lm[NL];
+    auto load_m = [&]() {
+        const T *Mg = Mlink + (int64_t)g * 16384;
+#pragma unroll
+        for (int q = 0; q < NL; q++) {
+            const int c = VEC * (4 * q + fk), row = 16 * wave + fr;
+            if (TRANS) {
+                lm[q] = *(const vec *)(Mg + row * 128 + c);
+            } else {
+#pragma unroll
+                for (int e = 0; e < VEC; e++) lm[q][e] = Mg[(c + e) * 128 + row];
+            }
+        }
+    };
+    if (!LATE_M && nprev > 0) load_m();
+    // right-hand side, by columns VEC (4 q + fk)
+    T bv[VEC][R];
+#pragma unroll
+    for (int e = 0; e < VEC; e++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int row = r0 + VEC * (4 * fq + fk) + e;
+            const T v = B[(int64_t)min(r, nr - 1) * ldb + min(row, N - 1)];
+            bv[e][r] = row < N && r < nr ? v : T(0);
+        }
+    {
+        const T *Wg = W128 + (int64_t)g * 16384;
+        if (TRANS) {
+#pragma unroll
+            for (int i = 0; i < 16384 / VEC / 512; i++) {     // op(W)(row, k) = W(k, row) at 128 row + k
+                const int e = 512 * i + tid, c = e % (128 / VEC), row = e / (128 / VEC);
+                *(vec *)&Ws[(128 * c + row) * VEC] = *(const vec *)(Wg + row * 128 + VEC * c);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                const int e = 512 * i + tid, row = e & 127, k = e >> 7;
+                Ws[(128 * (k / VEC) + row) * VEC + k % VEC] = Wg[e];
+            }
+        }
+    }
+
+    // ---- every earlier block but the last: L and X read ahead
+    T acc[VEC][R];
+    auto clear = [&]() {
+#pragma unroll
+        for (int e = 0; e < VEC; e++)
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[e][r] = T(0);
+    };
+    clear();
+    T cs[COLS ? NL : 1][R];                                   // COLS: sums of column CPL i + lane / LPC
+#pragma unroll
+    for (auto &ci : cs)
+#pragma unroll
+        for (T &c : ci) c = T(0);
+    if (nprev > 1) {
+        const int last = nprev - 2;
+        vec l[NBUF][NL];
+        U xr[NBUF][XV][R];
+        int next = 0;
+        // past the last block the last one is read again
+        auto fetch = [&](vec (&lb)[NL], U (&xb)[XV][R]) {
+            if (next <= last) {
+                load_l(lb, blk(next));
+                read_x(blk(next), xb);
+            }
+            next++;
+        };
+        auto consume = [&](int s, vec (&lb)[NL], U (&xb)[XV][R]) {
+            wait(xb, [&]() { read_x(blk(s), xb); });
+            T x[XV][R];
+            value(xb, x);
+            if constexpr (COLS) {
+#pragma unroll
+                for (int e = 0; e < VEC; e++)
+#pragma unroll
+                    for (int i = 0; i < NL; i++)
+#pragma unroll
+                        for (int r = 0; r < R; r++) cs[i][r] = fma(lb[i][e], x[e][r], cs[i][r]);
+            } else {
+                wv_fma<T, XV, R>(acc, x, lb, Pieces());
+            }
+        };
+#pragma unroll
+        for (int b = 0; b < NBUF - 1; b++) fetch(l[b], xr[b]);
+        for (int s = 0; s <= last; s += NBUF) {
+#pragma unroll
+            for (int b = 0; b < NBUF; b++) {
+                if (s + b <= last) {
+                    fetch(l[(b + NBUF - 1) % NBUF], xr[(b + NBUF - 1) % NBUF]);
+                    consume(s + b, l[b], xr[b]);
+                }
+            }
+        }
+    }
+
+    if (LATE_M && nprev > 0) load_m();
+
+    // sum over the four lane groups (and a lane's VEC sums)
+    auto groups = [&](int r) -> T {
+        T v = acc[0][r];
+#pragma unroll
+        for (int e = 1; e < VEC; e++) v += acc[e][r];
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    // ---- y = b - sums, by columns VEC (4 q + fk)
+    if constexpr (COLS) {
+        // over the LPC lanes of a column: half the columns go to the partner
+        // lane in each of the first steps
+        int i0 = 0;
+#pragma unroll
+        for (int n = NL / 2, x = LPC / 2; n > 0; n /= 2, x /= 2) {
+            const bool up = lane & x;
+            i0 += up ? n : 0;
+#pragma unroll
+            for (int i = 0; i < n; i++)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const T keep = up ? cs[i + n][r] : cs[i][r], send = up ? cs[i][r] : cs[i + n][r];
+                    cs[i][r] = keep + __shfl_xor(send, x);
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            cs[0][r] += __shfl_xor(cs[0][r], 2);
+            cs[0][r] += __shfl_xor(cs[0][r], 1);
+            if ((lane & 3) == 0) Ps[0][r][16 * wave + CPL * i0 + lane / LPC] = cs[0][r];
+        }
+    } else if constexpr (TRANS) {
+        T v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = groups(r);
+        if (fk == 0)
+#pragma unroll
+            for (int r = 0; r < R; r++) Ps[0][r][16 * wave + fr] = v[r];
+    } else {
+        const int slot = (TWO ? wave & 3 : wave) * CPL + lane / LPC;
+        auto part = [&](int r) -> vec * { return (vec *)&Ps[slot][r][VEC * (lane % LPC)]; };
+        if (!TWO || wave >= 4)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int e = 0; e < VEC; e++) (*part(r))[e] = acc[e][r];
+        if constexpr (TWO) {
+            __syncthreads();
+            if (wave < 4)
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) (*part(r))[e] += acc[e][r];
+        }
+    }
+    __syncthreads();
+    T y[VEC][R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        vec sum = *(const vec *)&Ps[0][r][VEC * (4 * fq + fk)];
+#pragma unroll
+        for (int p = 1; p < NP; p++) sum += *(const vec *)&Ps[p][r][VEC * (4 * fq + fk)];
+#pragma unroll
+        for (int e = 0; e < VEC; e++)
+            y[e][r] = r0 + VEC * (4 * fq + fk) + e < N ? bv[e][r] - sum[e] : T(0);
+    }
+    // ---- z = op(W_g) y
+    vec lw[NL];
+#pragma unroll
+    for (int q = 0; q < NL; q++) lw[q] = *(const vec *)&Ws[(128 * (4 * q + fk) + 16 * wave + fr) * VEC];
+    clear();
+    wv_fma<T, VEC, R>(acc, y, lw, Pieces());
+    T z[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) z[r] = groups(r);
+    // ---- x = z - M_g X(last earlier block)
+    if (nprev > 0) {
+        const T *xh = xs + (int64_t)blk(nprev - 1) * (WV_RB * RHSB);
+        U xl[VEC][R];
+        const int c = VEC * (4 * fq + fk);
+        read_v(xh, xl, c);
+        wait(xl, [&]() { read_v(xh, xl, c); });
+        T x[VEC][R];
+        value(xl, x);
+        clear();
+        wv_fma<T, VEC, R>(acc, x, lm, Pieces());
+#pragma unroll
+        for (int r = 0; r < R; r++) z[r] -= groups(r);
+    }
+    const int row = r0 + 16 * wave + fr;
+    if (fk == 0) {
+        T *xg = xs + (int64_t)g * (WV_RB * RHSB) + 16 * wave + fr;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const bool in = row < N && r < nr;
+            wv_store(xg + r * 128, in ? z[r] : T(0));
+            if (in) B[(int64_t)r * ldb + row] = z[r];
+        }
+    }
 }
 
 // Before each wavefront launch: staging filled with the sentinel, ticket 0
@@ -1293,12 +1728,22 @@ int trsm_enqueue(Ctx *c, hipStream_t s, int trans, int N, int NB, const T *dT, c
             T *Bj = dB + (int64_t)j0 * ldb;
             if (j0 > 0 || !first_reset_done)
                 k_wave_reset<T><<<(unsigned)std::min<int64_t>((nst + 255) / 256, 1024), 256, 0, s>>>(xs, nst, ticket);
-            MI_LAUNCH(c, s, SN<T>::wave, 1.0 * N * N * nr, 0.5 * N * (double)N * sizeof(T),
-                      (trans == 111
-                       ? k_trsm_wave<T, false, 8><<<nwg, 512, 0, s>>>(dT, N, NB, MT, W128, Mf, Bj, ldb, nr, xs,
-                                                                      ticket, g_wave_wait_ticks)
-                       : k_trsm_wave<T, true, 8><<<nwg, 512, 0, s>>>(dT, N, NB, MT, W128, Mb, Bj, ldb, nr, xs,
-                                                                     ticket, g_wave_wait_ticks)));
+            const bool fwd = trans == 111;
+            auto launch = [&](auto kernel) -> int {
+                MI_LAUNCH(c, s, SN<T>::wave, 1.0 * N * N * nr, 0.5 * N * (double)N * sizeof(T),
+                          (kernel<<<nwg, 512, 0, s>>>(dT, N, NB, MT, W128, fwd ? Mf : Mb, Bj, ldb, nr, xs, ticket,
+                                                      g_wave_wait_ticks)));
+                return 0;
+            };
+            // on the VALU up to 4 columns, where it is faster than 16 columns
+            // of MFMA (FP64, both sweeps, us: N = 6000 258, 338, 474 with 1,
+            // 2, 4 right-hand sides against 660; N = 16000 829, 905, 1200
+            // against 1635)
+            if (nr == 1) rc = fwd ? launch(k_trsm_vec<T, false, 1>) : launch(k_trsm_vec<T, true, 1>);
+            else if (nr == 2) rc = fwd ? launch(k_trsm_vec<T, false, 2>) : launch(k_trsm_vec<T, true, 2>);
+            else if (nr <= 4) rc = fwd ? launch(k_trsm_vec<T, false, 4>) : launch(k_trsm_vec<T, true, 4>);
+            else rc = fwd ? launch(k_trsm_wave<T, false, 8>) : launch(k_trsm_wave<T, true, 8>);
+            if (rc) return rc;
         }
         return 0;
     }
