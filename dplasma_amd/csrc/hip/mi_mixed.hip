@@ -254,31 +254,36 @@ __global__ __launch_bounds__(256) void k_dsymm_resid(const double *__restrict__ 
 // P2 contributions to a chunk are summed in LDS in a fixed order.
 // k_symm_sum then forms R = B - sum_n P1(m, n) - sum_m' P2(m', m) for each
 // row, in a fixed order, so the result is deterministic.
-// Partials per tile: P1 [NB][16], P2 [NB][16], |A| row sums [NB], column
-// sums [NB] -- 34 NB doubles at tile_index(m, n) * 34 NB.
-constexpr int SY_PART = 34;    // partial doubles per tile row index
+//
+// Too few tiles to fill the chip: S workgroups share a tile's columns (P2 and
+// the column sums are then disjoint, P1 and the row sums S partials).  N =
+// 3200, NB = 320 (55 tiles of ten chunks): 114 -> 35 us for S = 9.
+// Partials per tile, at tile_index(m, n) * sy_part(S) NB doubles: P1 [S][NB][16],
+// P2 [NB][16], |A| row sums [S][NB], column sums [NB].
+__host__ __device__ constexpr int64_t sy_part(int S) { return 17 * (S + 1); }
 
 template <bool ABS>
 __global__ __launch_bounds__(256, 2) void k_symm_part(const double *__restrict__ A, int N, int NB, int MT,
                                                      const double *__restrict__ X, int ldx, int nr,
-                                                     double *__restrict__ P)
+                                                     double *__restrict__ P, int S)
 {
     constexpr int CW = 32;                       // columns per chunk
     __shared__ double Tb[4][CW * 33];            // per wave: 32 x 32 block of A, [column][row], stride 33
     __shared__ double red[4][CW * 16 + CW];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int fr = lane & 15, fk = lane >> 4;
-    int t = blockIdx.x, n = 0;
+    const int sp = blockIdx.x % S;               // share of the tile's columns
+    int t = blockIdx.x / S, n = 0;
     while (t >= MT - n) { t -= MT - n; n++; }
     const int m = n + t;
     const bool dg = (m == n);
     const int rows_m = tile_rows(N, NB, MT, m), cols_n = tile_rows(N, NB, MT, n);
     const int64_t ti = tile_index(MT, m, n);
     const double *At = A + ti * (int64_t)NB * NB;
-    double *P1 = P + ti * (int64_t)SY_PART * NB;
-    double *P2 = P1 + 16 * NB;
-    double *A1 = P2 + 16 * NB;
-    double *A2 = A1 + NB;
+    double *P0 = P + ti * sy_part(S) * NB, *P1 = P0 + (int64_t)sp * 16 * NB;
+    double *P2 = P0 + (int64_t)S * 16 * NB;
+    double *A1 = P2 + 16 * NB + (int64_t)sp * NB;
+    double *A2 = P2 + 16 * NB + (int64_t)S * NB;
     const int jc = min(fr, nr - 1);              // clamped right-hand side of this lane
     const bool jok = fr < nr;
     const double *Xn = X + (int64_t)jc * ldx + (int64_t)n * NB;
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void k_symm_part(const double *__restrict__
         }
     };
     const int nch = (NB + CW - 1) / CW;
-    for (int ch = 0; ch < nch; ch++) {
+    for (int ch = nch * sp / S; ch < nch * (sp + 1) / S; ch++) {
         const int c0 = CW * ch;
         // b-operands of P1: X_n(c0 + 4 u + fk, fr)
         double xn[8];
@@ -479,7 +484,7 @@ __device__ inline void lds_rd8(unsigned a, double (&x)[8])
 template <bool ABS, int RT>
 __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict__ A, int N, int MT,
                                                       const double *__restrict__ X, int ldx, int nr,
-                                                      double *__restrict__ P)
+                                                      double *__restrict__ P, int S)
 {
     constexpr int CW = 16;                       // columns per chunk
     constexpr int TB = RT * 128;                 // tile order
@@ -493,7 +498,8 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, w = tid >> 6, fr = lane & 15, fk = lane >> 4;
-    int t = blockIdx.x, n = 0;
+    const int sp = blockIdx.x % S;               // share of the tile's columns
+    int t = blockIdx.x / S, n = 0;
     while (t >= MT - n) { t -= MT - n; n++; }
     const int m = n + t;
     const bool dg = m == n;
@@ -501,10 +507,10 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
     const bool edge = dg || rows_m < TB || cols_n < TB;      // workgroup-uniform
     const int64_t ti = tile_index(MT, m, n);
     const double *At = A + ti * (int64_t)TB * TB;
-    double *P1 = P + ti * (int64_t)SY_PART * TB;
-    double *P2 = P1 + 16 * TB;
-    double *A1 = P2 + 16 * TB;
-    double *A2 = A1 + TB;
+    double *P0 = P + ti * sy_part(S) * TB, *P1 = P0 + sp * 16 * TB;
+    double *P2 = P0 + S * 16 * TB;
+    double *A1 = P2 + 16 * TB + sp * TB;
+    double *A2 = P2 + 16 * TB + S * TB;
     const int jc = min(fr, nr - 1);              // clamped right-hand side of this lane
     const double jm = fr < nr ? 1.0 : 0.0;
     const double *Xn = X + (int64_t)jc * ldx + (int64_t)n * TB;
@@ -624,7 +630,8 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
             if (fk == 0) Rw[CW * 16 + fr] = a2;
         }
     };
-    const int nch = (cols_n + CW - 1) / CW;
+    // this share's chunks, ch0 .. nch - 1
+    const int all = (cols_n + CW - 1) / CW, ch0 = all * sp / S, nch = all * (sp + 1) / S;
     // b-operands of P1 for chunk ch, X_n(16 ch + 4 u + fk, fr), read one
     // chunk ahead, before that chunk's own loads
     double xr[4];
@@ -654,7 +661,7 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
         // xn in registers before the loads below are issued, so that no
         // wait for it waits for them
         asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(xn[2]), "+v"(xn[3])::"memory");
-        if (ch > 0) store_pend(c0 - CW);
+        if (ch > ch0) store_pend(c0 - CW);
         // the next chunk; after the last one, this chunk again (from L2)
         read_xn(min(ch + 1, nch - 1));
         dload(Sn, min(ch + 1, nch - 1));
@@ -672,13 +679,15 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
             pend = ((((((v[0] + v[1]) + v[2]) + v[3]) + v[4]) + v[5]) + v[6]) + v[7];
         }
     };
-    read_xn(0);
-    dload(S0, 0);
-    for (int ch = 0; ch < nch; ch += 2) {
+    if (ch0 < nch) {
+        read_xn(ch0);
+        dload(S0, ch0);
+    }
+    for (int ch = ch0; ch < nch; ch += 2) {
         step(ch, S0, S1);
         if (ch + 1 < nch) step(ch + 1, S1, S0);
     }
-    if (nch > 0) store_pend((nch - 1) * CW);
+    if (ch0 < nch) store_pend((nch - 1) * CW);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // the last, unused loads
     // element q of p1[i] in lane (fr, fk): P1(rw0 + 16 i + 4 q + fk, fr)
 #pragma unroll
@@ -694,27 +703,71 @@ __global__ __launch_bounds__(512, 1) void k_symm_part2(const double *__restrict_
     }
 }
 
-// R (ldr) = B (ldb) - (P1 + P2 sums) for nr right-hand sides; thread = (row,
-// right-hand side), partials summed over n = 0..m, then m' = m..MT-1.
+// R (ldr) = B (ldb) - (P1 + P2 sums) for nr right-hand sides.  Sixteen lanes
+// a row: LP (a power of two, at most 16 / nr) lanes share the partials of a
+// right-hand side -- tiles n = 0..m with their shares, then m' = m..MT-1 --
+// in turn, four loads in flight each, and add up by shuffles: a fixed order.
 __global__ __launch_bounds__(256) void k_symm_sum(const double *__restrict__ P, int N, int NB, int MT,
                                                  const double *__restrict__ B, int ldb, double *__restrict__ R,
-                                                 int ldr, int nr, double *__restrict__ rowabs)
+                                                 int ldr, int nr, int LP, double *__restrict__ rowabs, int S)
 {
     const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (e >= (int64_t)N * 16) return;
-    const int row = (int)(e >> 4), j = (int)(e & 15);
+    const bool in = e < (int64_t)N * 16;
+    const int row = in ? (int)(e >> 4) : N - 1, l = (int)(e & 15), j = l / LP, k = l - j * LP;
     const int m = row / NB, r = row - m * NB;
-    const int64_t stride = (int64_t)SY_PART * NB;
-    double s = 0.0;
-    for (int n = 0; n <= m; n++) s += P[tile_index(MT, m, n) * stride + (int64_t)r * 16 + j];
-    for (int mm = m; mm < MT; mm++) s += P[tile_index(MT, mm, m) * stride + 16 * (int64_t)NB + (int64_t)r * 16 + j];
-    if (j < nr) R[(int64_t)j * ldr + row] = B[(int64_t)j * ldb + row] - s;
-    if (rowabs && j == 0) {
-        double a = 0.0;
-        for (int n = 0; n <= m; n++) a += P[tile_index(MT, m, n) * stride + 32 * (int64_t)NB + r];
-        for (int mm = m; mm < MT; mm++) a += P[tile_index(MT, mm, m) * stride + 33 * (int64_t)NB + r];
-        rowabs[row] = a;
+    const int64_t stride = sy_part(S) * NB;
+    // element o1 of the shares of tiles (m, 0 .. m), w elements a row, then o2
+    // of tiles (m .., m)
+    auto sum = [&](int64_t o1, int64_t o2, int w) -> double {
+        double s = 0.0;
+        if (S == 1 && LP == 1) {                    // plain runs
+            for (int n = 0; n <= m; n++) s += P[tile_index(MT, m, n) * stride + o1];
+            for (int mm = m; mm < MT; mm++) s += P[tile_index(MT, mm, m) * stride + o2];
+            return s;
+        }
+        int n = 0, sp = k, mm = m;                  // next share (sp of tile n), or tile mm of the second run
+        bool first = true;
+        auto next = [&]() -> const double * {
+            while (first && sp >= S) {
+                sp -= S;
+                if (++n > m) {
+                    first = false;
+                    mm = m + sp;
+                }
+            }
+            const double *p = nullptr;
+            if (first) {
+                p = P + tile_index(MT, m, n) * stride + o1 + (int64_t)sp * w * NB;
+                sp += LP;
+            } else if (mm < MT) {
+                p = P + tile_index(MT, mm, m) * stride + o2;
+                mm += LP;
+            }
+            return p;
+        };
+        for (;;) {
+            const double *p[4];
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) p[u] = next();
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = p[u] ? *p[u] : 0.0;
+#pragma unroll
+            for (int u = 0; u < 4; u++) s += v[u];
+            if (!p[3]) break;
+        }
+        return s;
+    };
+    double s = 0.0, a = 0.0;
+    if (j < nr) s = sum((int64_t)r * 16 + j, (int64_t)S * 16 * NB + (int64_t)r * 16 + j, 16);
+    if (rowabs && j == 0) a = sum((int64_t)(S + 1) * 16 * NB + r, (int64_t)(S + 1) * 16 * NB + (int64_t)S * NB + r, 1);
+    for (int o = LP / 2; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        a += __shfl_xor(a, o);
     }
+    if (!in || k != 0) return;
+    if (j < nr) R[(int64_t)j * ldr + row] = B[(int64_t)j * ldb + row] - s;
+    if (rowabs && j == 0) rowabs[row] = a;
 }
 
 // out[j] = max_i |V(i, j)| for the nc columns of V (M x nc, ld); NaN wins.
@@ -817,24 +870,30 @@ int dsymm_resid(Ctx *c, hipStream_t s, int N, int NB, const double *dA, int NRHS
     // loads need an even NB (16-byte aligned pairs)
     if (NB >= 64 && NB <= 512 && NB % 2 == 0) {
         const int64_t ntile = (int64_t)MT * (MT + 1) / 2;
-        double *P = (double *)ws_get(c, WS_MX_PART, (size_t)ntile * SY_PART * NB * sizeof(double));
+        const bool lds_chunks = NB % 128 == 0 && g_symm_kernel;
+        // shares of a tile: as many as bring the workgroups to about two a
+        // CU (one or three: within 1% of the solve of 3200), at most one a
+        // chunk (LDS chunks: two)
+        const int S = (int)std::min<int64_t>(lds_chunks ? NB / 32 : (NB + 31) / 32,
+                                             std::max<int64_t>(1, 512 / ntile));
+        double *P = (double *)ws_get(c, WS_MX_PART, (size_t)(ntile * sy_part(S) * NB) * sizeof(double));
         if (!P) return -3;
         for (int j0 = 0; j0 < NRHS; j0 += 16) {
             const int nr = NRHS - j0 < 16 ? NRHS - j0 : 16;
             double *ra = j0 == 0 ? rowabs : nullptr;
             const double *Xj = dX + (int64_t)j0 * ldx;
-            if (NB % 128 == 0 && g_symm_kernel) {
+            if (lds_chunks) {
                 // whole-chunk LDS loads (k_symm_part2), NB = 128 .. 512
                 const double fl = 2.0 * N * (double)N * nr, by = 8.0 * (double)ntile * NB * NB;
-                const unsigned gr = (unsigned)ntile;
+                const unsigned gr = (unsigned)(ntile * S);
 #define MI_SYMM2(RT)                                                                                             \
     do {                                                                                                         \
         if (ra)                                                                                                  \
             MI_LAUNCH(c, s, "dsymm_part", fl, by,                                                                \
-                      k_symm_part2<true, RT><<<gr, 512, 0, s>>>(dA, N, MT, Xj, ldx, nr, P));                    \
+                      k_symm_part2<true, RT><<<gr, 512, 0, s>>>(dA, N, MT, Xj, ldx, nr, P, S));                    \
         else                                                                                                     \
             MI_LAUNCH(c, s, "dsymm_part", fl, by,                                                                \
-                      k_symm_part2<false, RT><<<gr, 512, 0, s>>>(dA, N, MT, Xj, ldx, nr, P));                   \
+                      k_symm_part2<false, RT><<<gr, 512, 0, s>>>(dA, N, MT, Xj, ldx, nr, P, S));                   \
     } while (0)
                 switch (NB / 128) {
                 case 1: MI_SYMM2(1); break;
@@ -845,13 +904,14 @@ int dsymm_resid(Ctx *c, hipStream_t s, int N, int NB, const double *dA, int NRHS
 #undef MI_SYMM2
             } else if (ra)
                 MI_LAUNCH(c, s, "dsymm_part", 2.0 * N * (double)N * nr, 8.0 * (double)ntile * NB * NB,
-                          k_symm_part<true><<<(unsigned)ntile, 256, 0, s>>>(dA, N, NB, MT, Xj, ldx, nr, P));
+                          k_symm_part<true><<<(unsigned)(ntile * S), 256, 0, s>>>(dA, N, NB, MT, Xj, ldx, nr, P, S));
             else
                 MI_LAUNCH(c, s, "dsymm_part", 2.0 * N * (double)N * nr, 8.0 * (double)ntile * NB * NB,
-                          k_symm_part<false><<<(unsigned)ntile, 256, 0, s>>>(dA, N, NB, MT, Xj, ldx, nr, P));
-            MI_LAUNCH(c, s, "dsymm_sum", 0.0, 8.0 * 2.0 * (double)ntile * 16 * NB,
+                          k_symm_part<false><<<(unsigned)(ntile * S), 256, 0, s>>>(dA, N, NB, MT, Xj, ldx, nr, P, S));
+            const int lp = nr <= 1 ? 16 : nr <= 2 ? 8 : nr <= 4 ? 4 : nr <= 8 ? 2 : 1;
+            MI_LAUNCH(c, s, "dsymm_sum", 0.0, 8.0 * (S + 1.0) * (double)ntile * 16 * NB,
                       k_symm_sum<<<(unsigned)(((int64_t)N * 16 + 255) / 256), 256, 0, s>>>(
-                          P, N, NB, MT, dB + (int64_t)j0 * ldb, ldb, dR + (int64_t)j0 * ldr, ldr, nr, ra));
+                          P, N, NB, MT, dB + (int64_t)j0 * ldb, ldb, dR + (int64_t)j0 * ldr, ldr, nr, lp, ra, S));
         }
         return 0;
     }
