@@ -266,15 +266,26 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
     *bn = s - (*bm) * nsub;
 }
 
-// The workgroup's waves form a WR x WC grid over its BMX x BMX block, each
-// wave a (BMX/WR) x (BMX/WC) sub-block of 16x16 MFMA tiles.
-// One block: C(r_base.., c_base..) -= A(r_base.., 0:K) B(c_base.., 0:K)^T, all
-// of them column-major with leading dimension NB; rows_m / cols_n bound the
-// rows of A and C / the rows of B and columns of C; diag: only row >= column.
-template <class T, int BMX, int WR, int WC>
+// One 64 x 64 block by 2 x 2 waves: C(r_base.., c_base..) -= A(r_base.., 0:K)
+// B(c_base.., 0:K)^T, all of them column-major with leading dimension NB;
+// rows_m / cols_n bound the rows of A and C / the rows of B and columns of C;
+// diag: only row >= column.  For tiles that update_block_lds does not take:
+// any leading dimension, K and alignment.
+//
+// Loads are unconditional, from addresses clamped into the tile: rows past
+// the matrix only reach parts of C that are not stored, and A is zeroed past
+// K.  Operands wait in registers RING stages ahead, so that a short K (a
+// tile of 93 columns is six stages) is not a chain of memory latencies; C is
+// the MFMAs' start.  PAIR: even NB and aligned pairs of rows, two a load.
+// dpotrf N = 378, NB = 93: 13.2 us a launch with masked loads one stage ahead
+// and C at the end, 9.5 us now; N = 3900, NB = 367 2.09 -> 1.84 ms in FP64,
+// 1.66 -> 1.35 ms in FP32.
+constexpr int RING = 3;
+template <class T, bool PAIR>
 __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, int NB, int K, int rows_m, int cols_n,
                                              int r_base, int c_base, bool diag)
 {
+    constexpr int BMX = 64, WR = 2, WC = 2;
     // rows padded by 128 bytes: the four lane groups of a fragment read (k
     // rows 4s + l/16) then fall on alternating halves of the LDS banks
     constexpr int LP = BMX + 128 / (int)sizeof(T);
@@ -285,134 +296,97 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
     typedef typename MF<T>::v2 V2;
     constexpr int HR = BMX / WR, HC = BMX / WC;       // rows / columns per wave
     constexpr int TR = HR / 16, TC = HC / 16;         // 16x16 MFMA tiles per wave
-    constexpr int PR = BMX / 2;                       // element pairs per k row of a panel
-    constexpr int SP = BK * PR / NT;                  // pairs staged per thread and operand
-    static_assert(TR % 2 == 0 && SP * NT == BK * PR, "wave grid does not fit the block");
+    constexpr int W = PAIR ? 2 : 1;                   // rows of a load
+    typedef T VW __attribute__((ext_vector_type(W)));
+    constexpr int SP = BK * BMX / W / NT;             // loads per thread, operand and stage
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WC, wn = wave % WC;
+    const int fr = lane & 15, fk = lane >> 4;
 
-    const bool full = (r_base + BMX <= rows_m) && (c_base + BMX <= cols_n) && (K % BK == 0) && !(NB & 1);
-
-    V4 acc[TR][TC];
-#pragma unroll
-    for (int i = 0; i < TR; i++)
-#pragma unroll
-        for (int j = 0; j < TC; j++) acc[i][j] = V4{T(0), T(0), T(0), T(0)};
-
-    // global -> register staging in element pairs: pair e = tid + NT*i,
-    // k row kk = e / PR, rows 2*(e % PR) and 2*(e % PR) + 1
-    V2 ra[SP], rb[SP];
-    auto gload = [&](int k0) {
-        if (full) {
-#pragma unroll
-            for (int i = 0; i < SP; i++) {
-                const int e = tid + NT * i;
-                const int kk = e / PR, r = (e % PR) * 2;
-                ra[i] = *(const V2 *)(Ap + (int64_t)(k0 + kk) * NB + r_base + r);
-                rb[i] = *(const V2 *)(Bp + (int64_t)(k0 + kk) * NB + c_base + r);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < SP; i++) {
-                const int e = tid + NT * i;
-                const int kk = e / PR, r = (e % PR) * 2;
-                const int kg = k0 + kk;
-                T a0 = T(0), a1 = T(0), b0 = T(0), b1 = T(0);
-                if (kg < K) {
-                    const T *ac = Ap + (int64_t)kg * NB;
-                    const T *bc = Bp + (int64_t)kg * NB;
-                    if (r_base + r < rows_m) a0 = ac[r_base + r];
-                    if (r_base + r + 1 < rows_m) a1 = ac[r_base + r + 1];
-                    if (c_base + r < cols_n) b0 = bc[c_base + r];
-                    if (c_base + r + 1 < cols_n) b1 = bc[c_base + r + 1];
-                }
-                ra[i] = V2{a0, a1};
-                rb[i] = V2{b0, b1};
-            }
-        }
-    };
-    auto lstore = [&](int buf) {
+    // load e = tid + NT i of a stage: k row kk, rows r .. r + W - 1
+    constexpr int LR = BMX / W;
+    const int kk0 = tid / LR, r = (tid % LR) * W;     // kk = kk0 + (NT / LR) i
+    const int last_a = PAIR ? (rows_m - 1) & ~1 : rows_m - 1, last_b = PAIR ? (cols_n - 1) & ~1 : cols_n - 1;
+    const T *ap = Ap + min(r_base + r, last_a), *bp = Bp + min(c_base + r, last_b);
+    VW ra[RING][SP], rb[RING][SP];
+    auto gload = [&](VW (&xa)[SP], VW (&xb)[SP], int st) {
 #pragma unroll
         for (int i = 0; i < SP; i++) {
-            const int e = tid + NT * i;
-            const int kk = e / PR, r = (e % PR) * 2;
-            *(V2 *)&As[buf][kk][r] = V2{-ra[i].x, -ra[i].y};     // -A: the MFMA accumulates C - A B^T
-            *(V2 *)&Bs[buf][kk][r] = rb[i];
+            const int64_t o = (int64_t)min(st * BK + kk0 + (NT / LR) * i, K - 1) * NB;
+            xa[i] = *(const VW *)(ap + o);
+            xb[i] = *(const VW *)(bp + o);
         }
     };
-
-    // MFMA row tiles 2p and 2p+1 of a wave interleave their rows: row i of
-    // tile 2p+t is row 32p + 2i + t of the wave's rows, so that a lane holds
-    // two consecutive rows of one column and C moves as element pairs
-    // full off-diagonal blocks start from C (loaded with the first operands)
-    // and end with a plain store; the others accumulate -A B^T from zero
-    const int fr0 = lane & 15, fk0 = lane >> 4;
-    const bool pre = full && !diag;
-    if (pre) {
+    auto lstore = [&](const VW (&xa)[SP], const VW (&xb)[SP], int st) {
 #pragma unroll
-        for (int p = 0; p < TR / 2; p++)
-#pragma unroll
-            for (int j = 0; j < TC; j++) {
-                const int row = r_base + wm * HR + 32 * p + 2 * fr0;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const V2 c = *(const V2 *)&Cp[(int64_t)(c_base + wn * HC + j * 16 + MF<T>::row(q, fk0)) * NB + row];
-                    acc[2 * p][j][q] = c.x;
-                    acc[2 * p + 1][j][q] = c.y;
-                }
-            }
-    }
+        for (int i = 0; i < SP; i++) {
+            const int kk = kk0 + (NT / LR) * i;
+            const bool in = st * BK + kk < K;
+            *(VW *)&As[st & 1][kk][r] = in ? -xa[i] : VW(T(0));      // -A: the MFMA accumulates C - A B^T
+            *(VW *)&Bs[st & 1][kk][r] = xb[i];
+        }
+    };
     const int nstage = (K + BK - 1) / BK;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    const int fr = lane & 15, fk = lane >> 4;
-    for (int st = 0; st < nstage; st++) {
-        const int buf = st & 1;
-        if (st + 1 < nstage) gload((st + 1) * BK);
+#pragma unroll
+    for (int u = 0; u < RING; u++) gload(ra[u], rb[u], u);
+
+    // MFMA row tiles 0 and 1 of a wave interleave their rows: row i of tile t
+    // is row 2i + t of the wave's rows.  Fed (B, A), element q of lane l holds
+    // row 2 (l % 16) + t and column row(q, l / 16) of each 16x16 tile.
+    V4 acc[TR][TC];
+    const int row0 = r_base + wm * HR + 2 * fr, col0 = c_base + wn * HC;
+    const int cr = min(row0, last_a);
+#pragma unroll
+    for (int j = 0; j < TC; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const T *c = &Cp[(int64_t)min(col0 + j * 16 + MF<T>::row(q, fk), cols_n - 1) * NB + cr];
+            if constexpr (PAIR) {
+                const V2 v = *(const V2 *)c;
+                acc[0][j][q] = v.x;
+                acc[1][j][q] = v.y;
+            } else {
+                acc[0][j][q] = c[0];
+                acc[1][j][q] = c[cr + 1 < rows_m ? 1 : 0];
+            }
+        }
+    auto stage = [&](VW (&xa)[SP], VW (&xb)[SP], int st) {
+        // one barrier a stage: a wave that stores stage st has passed the
+        // barrier of stage st - 1, which no wave reaches before it is done
+        // with stage st - 2
+        lstore(xa, xb, st);
+        __syncthreads();
+        gload(xa, xb, st + RING);
 #pragma unroll
         for (int kq = 0; kq < BK / 4; kq++) {
-            T a[TR], b[TC];
+            T b[TC];
+            const V2 v = *(const V2 *)&As[st & 1][kq * 4 + fk][wm * HR + 2 * fr];
+            const T a[TR] = {v.x, v.y};
 #pragma unroll
-            for (int p = 0; p < TR / 2; p++) {
-                const V2 v = *(const V2 *)&As[buf][kq * 4 + fk][wm * HR + 32 * p + 2 * fr];
-                a[2 * p] = v.x;
-                a[2 * p + 1] = v.y;
-            }
-#pragma unroll
-            for (int j = 0; j < TC; j++) b[j] = Bs[buf][kq * 4 + fk][wn * HC + j * 16 + fr];
+            for (int j = 0; j < TC; j++) b[j] = Bs[st & 1][kq * 4 + fk][wn * HC + j * 16 + fr];
 #pragma unroll
             for (int i = 0; i < TR; i++)
 #pragma unroll
-                for (int j = 0; j < TC; j++)
-                    acc[i][j] = MF<T>::mfma(b[j], a[i], acc[i][j]);   // C^T: lanes walk rows
+                for (int j = 0; j < TC; j++) acc[i][j] = MF<T>::mfma(b[j], a[i], acc[i][j]);   // C^T: lanes walk rows
         }
-        if (st + 1 < nstage) lstore(buf ^ 1);
-        __syncthreads();
+    };
+    for (int st = 0; st < nstage; st += RING) {
+#pragma unroll
+        for (int u = 0; u < RING; u++)
+            if (st + u < nstage) stage(ra[u], rb[u], st + u);
     }
 
-    // epilogue: the MFMA was fed (B, A), so element q of lane l holds row
-    // 2 (l % 16) + t (tile 2p + t) and column row(q, l / 16) of each 16x16
-    // tile: a store walks row pairs
 #pragma unroll
-    for (int p = 0; p < TR / 2; p++) {
-        const int rr = r_base + wm * HR + 32 * p + 2 * fr;
+    for (int j = 0; j < TC; j++)
 #pragma unroll
-        for (int j = 0; j < TC; j++)
+        for (int q = 0; q < 4; q++) {
+            const int col = col0 + j * 16 + MF<T>::row(q, fk);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int col = c_base + wn * HC + j * 16 + MF<T>::row(q, fk);
-                if (pre) {
-                    *(V2 *)&Cp[(int64_t)col * NB + rr] = V2{acc[2 * p][j][q], acc[2 * p + 1][j][q]};
-                } else {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-                        const int r = rr + t;
-                        if (r < rows_m && col < cols_n && (!diag || r >= col)) Cp[(int64_t)col * NB + r] += acc[2 * p + t][j][q];
-                    }
-                }
+            for (int t = 0; t < TR; t++) {
+                const int rr = row0 + t;
+                if (rr < rows_m && col < cols_n && (!diag || rr >= col)) Cp[(int64_t)col * NB + rr] = acc[t][j][q];
             }
-    }
+        }
 }
 
 // workgroup id -> position in the launch's list of blocks: consecutive ids
@@ -465,16 +439,17 @@ __device__ __forceinline__ bool update_decode(const UpdArgs &u, int BMX, int *m,
 }
 
 // operands staged through registers: any leading dimension and alignment
-template <class T, int BMX, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC, 2) void k_update_mfma(T *__restrict__ Tt, UpdArgs u)
+template <class T, bool PAIR>
+__global__ __launch_bounds__(256, 2) void k_update_mfma(T *__restrict__ Tt, UpdArgs u)
 {
     int m, n, r_base, c_base, rows_m, cols_n;
     bool diag;
-    if (!update_decode(u, BMX, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
+    if (u.prio) __builtin_amdgcn_s_setprio(2);
+    if (!update_decode(u, 64, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
     const int64_t sz = (int64_t)u.NB * u.NB, off = (int64_t)u.c0 * u.NB;
-    update_block<T, BMX, WR, WC>(Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
-                                 Tt + tile_index(u.MT, m, n) * sz, u.NB, u.w > 0 ? u.w : u.NB, rows_m, cols_n, r_base,
-                                 c_base, diag);
+    update_block<T, PAIR>(Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
+                          Tt + tile_index(u.MT, m, n) * sz, u.NB, u.w > 0 ? u.w : u.NB, rows_m, cols_n, r_base, c_base,
+                          diag);
 }
 
 // operands straight into LDS (mi_update.hpp)
@@ -520,7 +495,7 @@ template <> struct UpdShapes<float> {
 // so the update carries about 16 significant bits per operand instead of 8,
 // at three BF16 MFMAs per product.  Used by the mixed-precision solve, whose
 // FP64 refinement recovers the rest.  Work decomposition, XCD grouping,
-// SYRK masking and the C-preload epilogue as k_update_mfma; K in chunks of
+// SYRK masking and C as the MFMAs' start as k_update_mfma; K in chunks of
 // 32, split once per workgroup while staged into LDS as [row][k] bf16 rows
 // (row pitch 40 bf16 = 80 B: 16-byte aligned fragment reads, spread banks).
 // MFMA operand layout: A(i, k) and B(k, j) for lane l in i (resp. j) = l % 16,
@@ -1151,8 +1126,10 @@ int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, dou
         MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Big, T, occ><<<(unsigned)g, Big::NT, 0, s>>>(dT, u)));
     else if (update_lds_ok<Small>(dT, u.NB, K))
         MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Small, T, 2><<<(unsigned)g, Small::NT, 0, s>>>(dT, u)));
+    else if (u.NB % 2 == 0 && ((uintptr_t)dT & (2 * sizeof(T) - 1)) == 0)
+        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, true><<<(unsigned)g, 256, 0, s>>>(dT, u)));
     else
-        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, 64, 2, 2><<<(unsigned)g, 256, 0, s>>>(dT, u)));
+        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, false><<<(unsigned)g, 256, 0, s>>>(dT, u)));
     return 0;
 }
 
