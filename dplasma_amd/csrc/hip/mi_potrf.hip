@@ -266,7 +266,7 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
     *bn = s - (*bm) * nsub;
 }
 
-// One 64 x 64 block by 2 x 2 waves: C(r_base.., c_base..) -= A(r_base.., 0:K)
+// One block of 32 WR rows and columns by WR x 2 waves: C(r_base.., c_base..) -= A(r_base.., 0:K)
 // B(c_base.., 0:K)^T, all of them column-major with leading dimension NB;
 // rows_m / cols_n bound the rows of A and C / the rows of B and columns of C;
 // diag: only row >= column.  For tiles that update_block_lds does not take:
@@ -281,11 +281,11 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
 // and C at the end, 9.5 us now; N = 3900, NB = 367 2.09 -> 1.84 ms in FP64,
 // 1.66 -> 1.35 ms in FP32.
 constexpr int RING = 3;
-template <class T, bool PAIR>
+template <class T, bool PAIR, int WR>
 __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, int NB, int K, int rows_m, int cols_n,
                                              int r_base, int c_base, bool diag)
 {
-    constexpr int BMX = 64, WR = 2, WC = 2;
+    constexpr int BMX = 32 * WR, WC = 2;
     // rows padded by 128 bytes: the four lane groups of a fragment read (k
     // rows 4s + l/16) then fall on alternating halves of the LDS banks
     constexpr int LP = BMX + 128 / (int)sizeof(T);
@@ -439,15 +439,15 @@ __device__ __forceinline__ bool update_decode(const UpdArgs &u, int BMX, int *m,
 }
 
 // operands staged through registers: any leading dimension and alignment
-template <class T, bool PAIR>
-__global__ __launch_bounds__(256, 2) void k_update_mfma(T *__restrict__ Tt, UpdArgs u)
+template <class T, bool PAIR, int WR>
+__global__ __launch_bounds__(128 * WR, 2) void k_update_mfma(T *__restrict__ Tt, UpdArgs u)
 {
     int m, n, r_base, c_base, rows_m, cols_n;
     bool diag;
     if (u.prio) __builtin_amdgcn_s_setprio(2);
-    if (!update_decode(u, 64, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
+    if (!update_decode(u, 32 * WR, &m, &n, &r_base, &c_base, &rows_m, &cols_n, &diag)) return;
     const int64_t sz = (int64_t)u.NB * u.NB, off = (int64_t)u.c0 * u.NB;
-    update_block<T, PAIR>(Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
+    update_block<T, PAIR, WR>(Tt + tile_index(u.MT, m, u.k) * sz + off, Tt + tile_index(u.MT, n, u.k) * sz + off,
                           Tt + tile_index(u.MT, m, n) * sz, u.NB, u.w > 0 ? u.w : u.NB, rows_m, cols_n, r_base, c_base,
                           diag);
 }
@@ -475,15 +475,23 @@ __global__ __launch_bounds__(S::NT, OCC) void k_update_lds(T *__restrict__ Tt, U
 //         BK 16 x 2 and four: 120; BK 32 x 2: 126
 // and of N = 4096, NB = 256 (64 x 64 blocks, 37.3 / 58.5 TF before): BK 16 x
 // 3: 41.3 / 62.6 TF, x 4: 39.6 / 61.2, BK 8 x 8: 38.3 / 60.9.
+//
+// A launch of at most 256 blocks of 64 x 64 leaves CUs idle and the others on
+// a chain of K / 16 stages: 32 x 32 blocks instead (dpotrf N = 4096, NB = 256
+// 1.67 -> 1.57 ms; posv N = 6000, NB = 512 4.20 -> 4.07 ms; 128 blocks 1.57 and
+// 4.15, 600 1.56 and 3.98, but FP32 N = 3200 2.41 -> 2.43 from 400 on).
+constexpr int64_t TINY_BLOCKS = 256;
 template <class T> struct UpdShapes;
 template <> struct UpdShapes<double> {
     typedef UpdShape<double, 128, 2, 4, 16, 2, 2, 2> big;
     typedef UpdShape<double, 64, 2, 2, 16, 3, 2, 1> small;
+    typedef UpdShape<double, 32, 2, 2, 32, 3, 1, 2> tiny;
     static constexpr int occ = 4;
 };
 template <> struct UpdShapes<float> {
     typedef UpdShape<float, 128, 2, 2, 16, 4, 4, 4> big;
     typedef UpdShape<float, 64, 2, 2, 16, 3, 2, 1> small;
+    typedef UpdShape<float, 32, 2, 2, 32, 3, 1, 2> tiny;
     static constexpr int occ = 2;
 };
 
@@ -1113,6 +1121,7 @@ int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, dou
 {
     typedef typename UpdShapes<T>::big Big;
     typedef typename UpdShapes<T>::small Small;
+    typedef typename UpdShapes<T>::tiny Tiny;
     constexpr int occ = UpdShapes<T>::occ;
     // a launch of fewer than two 128 x 128 blocks per CU leaves the chip
     // idle: 64 x 64 blocks give four times the workgroups at a quarter of
@@ -1120,16 +1129,28 @@ int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, dou
     int64_t g = grid(Big::BM);
     const bool big = g >= 512 && update_lds_ok<Big>(dT, u.NB, K);
     if (!big) g = grid(Small::BM);
+    const bool few = !big && g <= TINY_BLOCKS;
+    const bool tiny = few && update_lds_ok<Tiny>(dT, u.NB, K), small = !tiny && update_lds_ok<Small>(dT, u.NB, K);
+    if (tiny || (few && !small)) g = grid(32);
     if (g > 0x7fffffff) { set_error("update grid too large"); return -3; }
     if (g <= 0) return 0;
     if (big)
         MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Big, T, occ><<<(unsigned)g, Big::NT, 0, s>>>(dT, u)));
-    else if (update_lds_ok<Small>(dT, u.NB, K))
+    else if (tiny)
+        MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Tiny, T, 3><<<(unsigned)g, Tiny::NT, 0, s>>>(dT, u)));
+    else if (small)
         MI_LAUNCH(c, s, name, fl, by, (k_update_lds<Small, T, 2><<<(unsigned)g, Small::NT, 0, s>>>(dT, u)));
-    else if (u.NB % 2 == 0 && ((uintptr_t)dT & (2 * sizeof(T) - 1)) == 0)
-        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, true><<<(unsigned)g, 256, 0, s>>>(dT, u)));
-    else
-        MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, false><<<(unsigned)g, 256, 0, s>>>(dT, u)));
+    else {
+        const bool pair = u.NB % 2 == 0 && ((uintptr_t)dT & (2 * sizeof(T) - 1)) == 0;
+        if (few && pair)
+            MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, true, 1><<<(unsigned)g, 128, 0, s>>>(dT, u)));
+        else if (few)
+            MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, false, 1><<<(unsigned)g, 128, 0, s>>>(dT, u)));
+        else if (pair)
+            MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, true, 2><<<(unsigned)g, 256, 0, s>>>(dT, u)));
+        else
+            MI_LAUNCH(c, s, name, fl, by, (k_update_mfma<T, false, 2><<<(unsigned)g, 256, 0, s>>>(dT, u)));
+    }
     return 0;
 }
 
