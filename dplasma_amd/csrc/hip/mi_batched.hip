@@ -540,10 +540,30 @@ int batch_class(int n) { return n > 128 ? 0 : n > 64 ? 1 : 2; }
 template <class T>
 int batch_enqueue(mi_batch_t *p, T *dA, T *dB, hipStream_t s)
 {
+    mi_ctx_t *c = p->ctx;
+    auto count = [&](int cls) { return p->first[cls + 1] - p->first[cls]; };
     k_batch_reset<<<1, 64, 0, s>>>(p->d_counter);
-    for (int cls = 0; cls < BATCH_CLASSES; cls++)
-        batch_launch<T>(p, cls, p->first[cls], p->first[cls + 1] - p->first[cls],
-                        (cls == 2 ? 2 : 1) * p->wg_per_cu * p->cus, dA, dB, p->d_counter + cls, s);
+    // The classes below the largest run beside it, on the second stream (a
+    // branch of the graph): a class of a few hundred matrices is one wave of
+    // workgroups, each as long as its matrix.  Calls, one after the other ->
+    // together: 100 matrices of 1 .. 200 186 -> 140 us (FP32 148 -> 114), 1000
+    // FP32 ones of 8 .. 200 178 -> 167, 64 of 1 .. 100 92 -> 85.
+    int big = 0;
+    while (big < BATCH_CLASSES - 1 && count(big) == 0) big++;
+    hipStream_t s2 = s;
+    for (int cls = big + 1; cls < BATCH_CLASSES; cls++)
+        if (count(cls) > 0) s2 = c->s_panel;
+    if (s2 != s) {
+        MI_CHECK(hipEventRecord(c->ev_ring[0], s));
+        MI_CHECK(hipStreamWaitEvent(s2, c->ev_ring[0], 0));
+    }
+    for (int cls = big; cls < BATCH_CLASSES; cls++)
+        batch_launch<T>(p, cls, p->first[cls], count(cls), (cls == 2 ? 2 : 1) * p->wg_per_cu * p->cus, dA, dB,
+                        p->d_counter + cls, cls == big ? s : s2);
+    if (s2 != s) {
+        MI_CHECK(hipEventRecord(c->ev_ring[1], s2));
+        MI_CHECK(hipStreamWaitEvent(s, c->ev_ring[1], 0));
+    }
     MI_CHECK(hipGetLastError());
     return 0;
 }
