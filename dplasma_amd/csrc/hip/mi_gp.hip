@@ -98,6 +98,15 @@ template <class T> int solve(Ctx *c, int trans, int N, int NB, const T *dT, T *x
     return trsm_enqueue<T>(c, s, trans, N, NB, dT, W, 1, x, N);
 }
 
+// the span between the context's events, for mi_last_span_ms
+int span(Ctx *c)
+{
+    float ms = 0.f;
+    MI_CHECK(hipEventElapsedTime(&ms, c->t0, c->t1));
+    c->last_ms = ms;
+    return 0;
+}
+
 template <class T>
 int enqueue_nll(Ctx *c, int N, int NB, const T *dK, int ldk, T *dT, T *dy, double *dout, int *h_info)
 {
@@ -125,6 +134,7 @@ int gp_nll(mi_ctx_t *c, int N, int NB, const T *dK, int ldk, T *dT, T *dy, doubl
     const int rs = mi_synchronize(c);
     if (rc || rs) return rc ? rc : rs;
     *info = h_info;
+    if ((rc = span(c))) return rc;                 // the factorization's, between its own events
     return h_info ? 0 : trsm_status(c);
 }
 
@@ -139,7 +149,9 @@ int enqueue_grad(Ctx *c, int N, int NB, const T *dT, const T *da, T *dalpha, con
     const dim3 grid((unsigned)((int64_t)MT * (MT + 1) / 2), (unsigned)((NB + 7) / 8));
     MI_LAUNCH(c, s, "gp_seed", 0.0, (double)MT * (MT + 1) / 2 * NB * NB * sizeof(T),
               (k_gp_seed<T><<<grid, 256, 0, s>>>(dT, N, NB, MT, da, dalpha, dscale, dG)));
+    MI_CHECK(hipEventRecord(c->t0, s));
     if ((rc = adjoint_enqueue<T>(c, N, NB, dT, dG))) return rc;
+    MI_CHECK(hipEventRecord(c->t1, s));
     // the symmetric gradient: both triangles from the lower tiles
     if ((rc = sym_stage_enqueue<T>(c, s, false, UPPER, N, NB, dG, dK, ldk))) return rc;
     return sym_stage_enqueue<T>(c, s, false, LOWER, N, NB, dG, dK, ldk);
@@ -153,6 +165,7 @@ int gp_nll_grad(mi_ctx_t *c, int N, int NB, const T *dT, const T *da, T *dalpha,
     rc = enqueue_grad<T>(c, N, NB, dT, da, dalpha, dscale, dG, dK, ldk);
     const int rs = mi_synchronize(c);
     if (rc || rs) return rc ? rc : rs;
+    if ((rc = span(c))) return rc;
     return trsm_status(c);
 }
 
