@@ -29,7 +29,7 @@ __device__ __forceinline__ void update_tail(std::integer_sequence<int, I...>, F 
 // rows of an operand column form one LDS read: the MFMA tiles 0 .. V-1 of a
 // group interleave their rows (row i of tile t is row V i + t of the group),
 // so a lane holds V consecutive rows of C.  CPS such vectors of C come in a
-// stage at the end.
+// stage at the start.
 template <class T, int BM_, int WR_, int WC_, int BK_, int ST_, int V_, int CPS_> struct UpdShape {
     static constexpr int BM = BM_, WR = WR_, WC = WC_, BK = BK_, ST = ST_, V = V_, CPS = CPS_;
     static constexpr int NW = WR * WC, NT = 64 * NW;
@@ -137,28 +137,27 @@ __device__ __forceinline__ void update_block_lds(unsigned char *lds, const T *Ap
                 for (int j = 0; j < S::TC; j++) acc[i][j] = MF<T>::mfma(b[j], a[i], acc[i][j]);
         }
     };
-    // C of a whole block comes in one vector a stage over the last NC stages
-    // (K >= NC BK), so that its traffic spreads over the products instead of
-    // standing before them
-    const bool late = whole && nst >= S::NC;
-    const int head = late ? nst - S::NC : nst;
-    int slot = 0;
-    for (int s = 0; s < head; s++) {
-        // stage s landed, and every wave is done with stage s - 1
-        if (s + ST - 2 < nst) wait_barrier<S::NI * (ST - 2)>();
-        else wait_barrier<0>();
+    // C of a whole block comes in CPS vectors a stage over the first NC stages,
+    // so that its traffic spreads over the products instead of standing before
+    // them.  (Over the last stages it is as fast, but then the products add up
+    // from zero: the matrix cores' rounding has a small bias, and where C and
+    // the sum nearly cancel everywhere, as for strongly correlated covariances,
+    // every element of the residual A - L L^T gets the same sign.  FP32
+    // likelihood gradient at N = 8192: error 1.1e-3 with C last, 3.5e-4 so; FP64
+    // 1.9e-12 and 0.9e-12.)
+    const bool early = whole && nst >= S::NC;
+    int slot = 0, first = 0;
+    auto next = [&](int s) {
         if (s + ST - 1 < nst) issue(slot == 0 ? ST - 1 : slot - 1);
-        compute(slot);
-        slot = slot == ST - 1 ? 0 : slot + 1;
-    }
-    if (late) {
+    };
+    if (early) {
         vec c[2][S::CPS];
         update_tail<S>(std::make_integer_sequence<int, S::NC>(), [&](auto tt) {
             constexpr int t = decltype(tt)::value, left = S::NC - 1 - t;
-            // younger than stage s: the later stages' loads and the C loads of
-            // the ST - 2 stages before this one
+            // younger than stage t: at least the later stages' loads and the C
+            // loads of the ST - 2 stages before this one
             wait_barrier<S::NI * (left < ST - 2 ? left : ST - 2) + S::CPS * (t < ST - 2 ? t : ST - 2)>();
-            if constexpr (left >= ST - 1) issue(slot == 0 ? ST - 1 : slot - 1);
+            next(t);
 #pragma unroll
             for (int e = 0; e < S::CPS; e++) c[t & 1][e] = *cvec(S::CPS * t + e);
             compute(slot);
@@ -170,9 +169,18 @@ __device__ __forceinline__ void update_block_lds(unsigned char *lds, const T *Ap
         });
 #pragma unroll
         for (int e = 0; e < S::CPS; e++) sub(S::CPS * (S::NC - 1) + e, c[(S::NC - 1) & 1][e]);
+        first = S::NC;
+    }
+    for (int s = first; s < nst; s++) {
+        // stage s landed, and every wave is done with stage s - 1
+        if (s + ST - 2 < nst) wait_barrier<S::NI * (ST - 2)>();
+        else wait_barrier<0>();
+        next(s);
+        compute(slot);
+        slot = slot == ST - 1 ? 0 : slot + 1;
     }
 
-    if (late) {
+    if (early) {
 #pragma unroll
         for (int t = 0; t < S::NC * S::CPS; t++) {
             const int p = t / (4 * S::TC), j = t / 4 % S::TC, q = t % 4;
