@@ -276,10 +276,16 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
 // the matrix only reach parts of C that are not stored, and A is zeroed past
 // K.  Operands wait in registers RING stages ahead, so that a short K (a
 // tile of 93 columns is six stages) is not a chain of memory latencies; C is
-// the MFMAs' start.  PAIR: even NB and aligned pairs of rows, two a load.
+// loaded with the first of them and waits in registers.  PAIR: even NB and
+// aligned pairs of rows, two a load.
 // dpotrf N = 378, NB = 93: 13.2 us a launch with masked loads one stage ahead
-// and C at the end, 9.5 us now; N = 3900, NB = 367 2.09 -> 1.84 ms in FP64,
-// 1.66 -> 1.35 ms in FP32.
+// and C loaded at the end, 9.5 us now; N = 3900, NB = 367 2.09 -> 1.81 ms in
+// FP64, 1.66 -> 1.31 ms in FP32.
+//
+// The products add up from zero and meet C once: as the MFMAs' start, C would
+// round at its own size every four columns (factor of N = 513, NB = 130 with a
+// dominant diagonal, error in units of the type's eps: FP64 4.6 against 2.3,
+// FP32 7.3 against 2.6).
 constexpr int RING = 3;
 template <class T, bool PAIR, int WR>
 __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, int NB, int K, int rows_m, int cols_n,
@@ -322,7 +328,7 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
         for (int i = 0; i < SP; i++) {
             const int kk = kk0 + (NT / LR) * i;
             const bool in = st * BK + kk < K;
-            *(VW *)&As[st & 1][kk][r] = in ? -xa[i] : VW(T(0));      // -A: the MFMA accumulates C - A B^T
+            *(VW *)&As[st & 1][kk][r] = in ? -xa[i] : VW(T(0));      // -A: the MFMA accumulates -A B^T
             *(VW *)&Bs[st & 1][kk][r] = xb[i];
         }
     };
@@ -333,7 +339,7 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
     // MFMA row tiles 0 and 1 of a wave interleave their rows: row i of tile t
     // is row 2i + t of the wave's rows.  Fed (B, A), element q of lane l holds
     // row 2 (l % 16) + t and column row(q, l / 16) of each 16x16 tile.
-    V4 acc[TR][TC];
+    V4 acc[TR][TC], cv[TR][TC];
     const int row0 = r_base + wm * HR + 2 * fr, col0 = c_base + wn * HC;
     const int cr = min(row0, last_a);
 #pragma unroll
@@ -343,13 +349,17 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
             const T *c = &Cp[(int64_t)min(col0 + j * 16 + MF<T>::row(q, fk), cols_n - 1) * NB + cr];
             if constexpr (PAIR) {
                 const V2 v = *(const V2 *)c;
-                acc[0][j][q] = v.x;
-                acc[1][j][q] = v.y;
+                cv[0][j][q] = v.x;
+                cv[1][j][q] = v.y;
             } else {
-                acc[0][j][q] = c[0];
-                acc[1][j][q] = c[cr + 1 < rows_m ? 1 : 0];
+                cv[0][j][q] = c[0];
+                cv[1][j][q] = c[cr + 1 < rows_m ? 1 : 0];
             }
         }
+#pragma unroll
+    for (int i = 0; i < TR; i++)
+#pragma unroll
+        for (int j = 0; j < TC; j++) acc[i][j] = V4{T(0), T(0), T(0), T(0)};
     auto stage = [&](VW (&xa)[SP], VW (&xb)[SP], int st) {
         // one barrier a stage: a wave that stores stage st has passed the
         // barrier of stage st - 1, which no wave reaches before it is done
@@ -384,7 +394,8 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
 #pragma unroll
             for (int t = 0; t < TR; t++) {
                 const int rr = row0 + t;
-                if (rr < rows_m && col < cols_n && (!diag || rr >= col)) Cp[(int64_t)col * NB + rr] = acc[t][j][q];
+                if (rr < rows_m && col < cols_n && (!diag || rr >= col))
+                    Cp[(int64_t)col * NB + rr] = cv[t][j][q] + acc[t][j][q];
             }
         }
 }
