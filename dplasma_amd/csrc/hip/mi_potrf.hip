@@ -273,8 +273,8 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
 // any leading dimension, K and alignment.
 //
 // Loads are unconditional, from addresses clamped into the tile: rows past
-// the matrix only reach parts of C that are not stored, and A is zeroed past
-// K.  Operands wait in registers RING stages ahead, so that a short K (a
+// the matrix only reach parts of C that are not stored, and both operands are
+// zeroed past K (0 times an infinity would not be 0).  Operands wait in registers RING stages ahead, so that a short K (a
 // tile of 93 columns is six stages) is not a chain of memory latencies; C is
 // loaded with the first of them and waits in registers.  PAIR: even NB and
 // aligned pairs of rows, two a load.
@@ -329,7 +329,7 @@ __device__ __forceinline__ void update_block(const T *Ap, const T *Bp, T *Cp, in
             const int kk = kk0 + (NT / LR) * i;
             const bool in = st * BK + kk < K;
             *(VW *)&As[st & 1][kk][r] = in ? -xa[i] : VW(T(0));      // -A: the MFMA accumulates -A B^T
-            *(VW *)&Bs[st & 1][kk][r] = xb[i];
+            *(VW *)&Bs[st & 1][kk][r] = in ? xb[i] : VW(T(0));
         }
     };
     const int nstage = (K + BK - 1) / BK;

@@ -46,3 +46,35 @@ def test_one_rounding_at_c(dev, N, NB, dtype):
             if m == k:
                 err = np.tril(err)
             assert (err <= tol).all(), (m, k, float((err / tol).max()))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("N,NB", [(30, 9), (200, 40), (300, 93), (700, 367)])
+def test_infinity_in_the_last_column(dev, N, NB, dtype):
+    """K is padded to whole stages by repeating its last column; an infinity
+    there still gives infinities, not 0 * inf."""
+    print(f"inf N={N} NB={NB} {dtype.__name__}", flush=True)
+    MT = (N + NB - 1) // NB
+    rng = np.random.default_rng(N)
+    T = rng.uniform(1.0, 2.0, MT * (MT + 1) // 2 * NB * NB).astype(dtype)
+
+    def tile(X, m, k):
+        i = k * MT - k * (k - 1) // 2 + (m - k)
+        return X[i * NB * NB:(i + 1) * NB * NB].reshape((NB, NB), order="F")
+
+    for m in range(1, MT):
+        tile(T, m, 0)[1, NB - 1] = np.inf
+    d = dev.upload(T)
+    fn = dev.M.mi_dpotrf_step_update if dtype == np.float64 else dev.M.mi_spotrf_step_update
+    dev.check(fn(dev.h, N, NB, d, 0, 1, MT), "update")
+    got = dev.download(d, T.shape, dtype)
+    dev.free(d)
+    for k in range(1, MT):
+        for m in range(k, MT):
+            tm, tn = min(NB, N - m * NB), min(NB, N - k * NB)
+            low = np.tril(np.ones((tm, tn), bool)) if m == k else np.ones((tm, tn), bool)
+            g = tile(got, m, k)[:tm, :tn]
+            inf = np.zeros((tm, tn), bool)
+            inf[1, :] = inf[:, 1] = True
+            assert (g[low & inf] == -np.inf).all()
+            assert np.isfinite(g[low & ~inf]).all()
