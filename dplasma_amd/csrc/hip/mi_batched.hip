@@ -1,5 +1,6 @@
 // mi_batched.hip -- many independent SPD systems of uneven sizes, factored
-// and solved in persistent launches (captured in a hipGraph for replay).
+// and solved in persistent launches (the largest class captured in a hipGraph
+// for replay).
 //
 // No counterpart in the reference (its batching growth path: each matrix
 // is dplasma_dposv, src/zposv_wrapper.c:63-113, on one tile; the per-matrix
@@ -463,7 +464,12 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_posv_batched(int count, const 
         }
         __syncthreads();
         const int q = sh.idx;
-        if (q >= count) break;
+        if (q >= count) {
+            // every workgroup takes one number past the end, the last of them
+            // the one below, and leaves the queue as it was found: empty
+            if (threadIdx.x == 0 && q == count + (int)gridDim.x - 1) atomicExch(counter, 0);
+            break;
+        }
         const int m = order[q];
         const int n = nsz[m];
         T *Am = A + aoff[m];
@@ -481,11 +487,6 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_posv_batched(int count, const 
 // Size classes of the queue (largest first): above 128, at most 128, at most 64.
 constexpr int BATCH_CLASSES = 3;
 
-__global__ void k_batch_reset(int *counter)
-{
-    if (threadIdx.x < BATCH_CLASSES) counter[threadIdx.x] = 0;
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -494,11 +495,13 @@ struct mi_batch_s {
     int count = 0;
     std::vector<int> n;
     int64_t a_elems = 0, b_elems = 0;
-    int *d_n = nullptr, *d_order = nullptr, *d_info = nullptr, *d_counter = nullptr;
+    int *d_n = nullptr, *d_order = nullptr, *d_info = nullptr;
+    int *d_counter = nullptr;                      // of the classes' queues, behind d_order
     int64_t *d_aoff = nullptr, *d_boff = nullptr;
     int first[BATCH_CLASSES + 1] = {0, 0, 0, 0};   // queue positions where the classes begin
     int nsplit = 128, wg_per_cu = 2, cus = 0;      // (nsplit: kept for mi_batch_get_shape only)
-    // captured graph of the last (A, B, type, grid) it ran on
+    hipEvent_t t2 = nullptr;                       // end of the smaller classes (plans of several classes)
+    // captured graph of the largest class, of the last (A, B, type, grid) it ran on
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     const void *g_a = nullptr, *g_b = nullptr;
@@ -517,12 +520,12 @@ void batch_drop_graph(mi_batch_t *p)
 }
 
 // One class: count matrices from queue position q0, at most `wgs` workgroups.
-template <class T>
-void batch_launch(mi_batch_t *p, int cls, int q0, int count, int wgs, T *dA, T *dB, int *counter, hipStream_t s)
+template <class T> int batch_launch(mi_batch_t *p, int cls, int q0, int count, int wgs, T *dA, T *dB, hipStream_t s)
 {
-    if (count <= 0) return;
+    if (count <= 0) return 0;
     const unsigned grid = (unsigned)std::max(1, std::min(count, wgs));
     const int *order = p->d_order + q0;
+    int *counter = p->d_counter + cls;
     constexpr bool f64 = sizeof(T) == 8;
     if (cls == 0)
         k_posv_batched<T, 8, 2, true, f64 ? 2 : 4><<<grid, 512, 0, s>>>(count, order, p->d_n, p->d_aoff, p->d_boff, dA,
@@ -533,39 +536,17 @@ void batch_launch(mi_batch_t *p, int cls, int q0, int count, int wgs, T *dA, T *
     else
         k_posv_batched<T, 4, 1, false, f64 ? 3 : 4><<<grid, 256, 0, s>>>(count, order, p->d_n, p->d_aoff, p->d_boff, dA, dB,
                                                                p->d_info, counter);
+    MI_CHECK(hipGetLastError());
+    return 0;
 }
 
 int batch_class(int n) { return n > 128 ? 0 : n > 64 ? 1 : 2; }
 
-template <class T>
-int batch_enqueue(mi_batch_t *p, T *dA, T *dB, hipStream_t s)
+// All matrices of a class
+template <class T> int batch_launch_class(mi_batch_t *p, int cls, T *dA, T *dB, hipStream_t s)
 {
-    mi_ctx_t *c = p->ctx;
-    auto count = [&](int cls) { return p->first[cls + 1] - p->first[cls]; };
-    k_batch_reset<<<1, 64, 0, s>>>(p->d_counter);
-    // The classes below the largest run beside it, on the second stream (a
-    // branch of the graph): a class of a few hundred matrices is one wave of
-    // workgroups, each as long as its matrix.  Calls, one after the other ->
-    // together: 100 matrices of 1 .. 200 186 -> 140 us (FP32 148 -> 114), 1000
-    // FP32 ones of 8 .. 200 178 -> 167, 64 of 1 .. 100 92 -> 85.
-    int big = 0;
-    while (big < BATCH_CLASSES - 1 && count(big) == 0) big++;
-    hipStream_t s2 = s;
-    for (int cls = big + 1; cls < BATCH_CLASSES; cls++)
-        if (count(cls) > 0) s2 = c->s_panel;
-    if (s2 != s) {
-        MI_CHECK(hipEventRecord(c->ev_ring[0], s));
-        MI_CHECK(hipStreamWaitEvent(s2, c->ev_ring[0], 0));
-    }
-    for (int cls = big; cls < BATCH_CLASSES; cls++)
-        batch_launch<T>(p, cls, p->first[cls], count(cls), (cls == 2 ? 2 : 1) * p->wg_per_cu * p->cus, dA, dB,
-                        p->d_counter + cls, cls == big ? s : s2);
-    if (s2 != s) {
-        MI_CHECK(hipEventRecord(c->ev_ring[1], s2));
-        MI_CHECK(hipStreamWaitEvent(s, c->ev_ring[1], 0));
-    }
-    MI_CHECK(hipGetLastError());
-    return 0;
+    return batch_launch<T>(p, cls, p->first[cls], p->first[cls + 1] - p->first[cls],
+                           (cls == 2 ? 2 : 1) * p->wg_per_cu * p->cus, dA, dB, s);
 }
 
 // the same kernel launched once per matrix (one workgroup each), in queue
@@ -575,17 +556,15 @@ int batch_run_loop(mi_batch_t *p, T *dA, T *dB)
 {
     mi_ctx_t *c = p->ctx;
     hipStream_t s = c->s_main;
+    int rc;
     if (p->count == 0) return 0;
     MI_CHECK(hipEventRecord(c->t0, s));
     for (int q = 0; q < p->count; q++) {
-        k_batch_reset<<<1, 64, 0, s>>>(p->d_counter);
         const int cls = q < p->first[1] ? 0 : q < p->first[2] ? 1 : 2;
-        batch_launch<T>(p, cls, q, 1, 1, dA, dB, p->d_counter, s);
+        if ((rc = batch_launch<T>(p, cls, q, 1, 1, dA, dB, s))) return rc;
     }
-    MI_CHECK(hipGetLastError());
     MI_CHECK(hipEventRecord(c->t1, s));
-    int rc = mi_synchronize(c);
-    if (rc) return rc;
+    if ((rc = mi_synchronize(c))) return rc;
     float ms = 0.f;
     MI_CHECK(hipEventElapsedTime(&ms, c->t0, c->t1));
     p->last_ms = ms;
@@ -593,19 +572,32 @@ int batch_run_loop(mi_batch_t *p, T *dA, T *dB)
     return 0;
 }
 
-template <class T>
-int batch_run(mi_batch_t *p, T *dA, T *dB, int use_graph)
+// The largest class on the main stream, as a graph when use_graph, and the
+// classes below it beside it on the second stream: a class of a few hundred
+// matrices is one wave of workgroups, each as long as its matrix.  Both
+// streams are idle when a call begins and waited for before it returns, so
+// nothing but the host's wait joins them.  (As a branch of one graph, with
+// events between the streams and a kernel that resets the queues, a replay
+// took 5 - 25 us longer, and the first call of a plan, or with new arrays,
+// another 70 us for the instantiation: 64 FP32 systems of 1 .. 100 120 and 57 us
+// a first and a later call, now 58 and 51; 1000 of 8 .. 200 201 and 132, now 117
+// and 110.  One class after the other: 100 FP64 systems of 1 .. 200 186 us, now
+// 109.)
+template <class T> int batch_enqueue(mi_batch_t *p, T *dA, T *dB, int use_graph)
 {
     mi_ctx_t *c = p->ctx;
     hipStream_t s = c->s_main;
     const int type = sizeof(T) == 8 ? 0 : 1;
-    int rc;
-    if (p->count == 0) return 0;
-    if (use_graph) {
+    int big = 0, rc;
+    while (p->first[big + 1] == 0) big++;
+    MI_CHECK(hipEventRecord(c->t0, s));
+    if (!use_graph) {
+        if ((rc = batch_launch_class<T>(p, big, dA, dB, s))) return rc;
+    } else {
         if (!p->exec || p->g_a != dA || p->g_b != dB || p->g_type != type || p->g_wg != p->wg_per_cu) {
             batch_drop_graph(p);
             MI_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            rc = batch_enqueue<T>(p, dA, dB, s);
+            rc = batch_launch_class<T>(p, big, dA, dB, s);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(s, &g);
             if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
@@ -617,19 +609,30 @@ int batch_run(mi_batch_t *p, T *dA, T *dB, int use_graph)
             p->g_type = type;
             p->g_wg = p->wg_per_cu;
         }
-        MI_CHECK(hipEventRecord(c->t0, s));
         MI_CHECK(hipGraphLaunch(p->exec, s));
-        MI_CHECK(hipEventRecord(c->t1, s));
-    } else {
-        MI_CHECK(hipEventRecord(c->t0, s));
-        if ((rc = batch_enqueue<T>(p, dA, dB, s))) return rc;
-        MI_CHECK(hipEventRecord(c->t1, s));
     }
-    if ((rc = mi_synchronize(c))) return rc;
-    float ms = 0.f;
+    MI_CHECK(hipEventRecord(c->t1, s));
+    if (!p->t2) return 0;                          // one class
+    for (int cls = big + 1; cls < BATCH_CLASSES; cls++)
+        if ((rc = batch_launch_class<T>(p, cls, dA, dB, c->s_panel))) return rc;
+    MI_CHECK(hipEventRecord(p->t2, c->s_panel));
+    return 0;
+}
+
+template <class T>
+int batch_run(mi_batch_t *p, T *dA, T *dB, int use_graph)
+{
+    mi_ctx_t *c = p->ctx;
+    if (p->count == 0) return 0;
+    const int rc = batch_enqueue<T>(p, dA, dB, use_graph);
+    // the wait comes first also after an error: the caller may free its arrays
+    const int rs = mi_synchronize(c);
+    if (rc || rs) return rc ? rc : rs;
+    float ms = 0.f, ms2 = 0.f;
     MI_CHECK(hipEventElapsedTime(&ms, c->t0, c->t1));
-    p->last_ms = ms;
-    c->last_ms = ms;
+    if (p->t2) MI_CHECK(hipEventElapsedTime(&ms2, c->t0, p->t2));
+    p->last_ms = std::max(ms, ms2);
+    c->last_ms = p->last_ms;
     return 0;
 }
 
@@ -645,6 +648,7 @@ int batch_autotune(mi_batch_t *p, const T *dA0, const T *dB0, T *dA, T *dB, int 
         for (int rep = 0; rep < 2; rep++) {         // the first run warms up
             MI_CHECK(hipMemcpyAsync(dA, dA0, (size_t)p->a_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
             if (dB) MI_CHECK(hipMemcpyAsync(dB, dB0, (size_t)p->b_elems * sizeof(T), hipMemcpyDeviceToDevice, c->s_main));
+            MI_CHECK(hipStreamSynchronize(c->s_main));
             int rc = batch_run<T>(p, dA, dB, 0);
             if (rc) return rc;
             t = p->last_ms;
@@ -708,13 +712,18 @@ int mi_batch_create(mi_ctx_t *c, int count, const int *n, mi_batch_t **plan)
     const size_t m = std::max(1, count);
     hipError_t e = hipSuccess;
     if (e == hipSuccess) e = hipMalloc(&p->d_n, m * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&p->d_order, m * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&p->d_order, (count + BATCH_CLASSES) * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&p->d_info, m * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&p->d_counter, BATCH_CLASSES * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&p->d_aoff, m * sizeof(int64_t));
     if (e == hipSuccess) e = hipMalloc(&p->d_boff, m * sizeof(int64_t));
+    int classes = 0;
+    for (int cls = 0; cls < BATCH_CLASSES; cls++) classes += p->first[cls + 1] > p->first[cls];
+    if (e == hipSuccess && classes > 1) e = hipEventCreate(&p->t2);
     if (e == hipSuccess && count) e = hipMemcpy(p->d_n, n, count * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess && count) e = hipMemcpy(p->d_order, order.data(), count * sizeof(int), hipMemcpyHostToDevice);
+    order.resize(count + BATCH_CLASSES, 0);          // the queues' counters behind it, at 0
+    p->d_counter = p->d_order + count;
+    if (e == hipSuccess)
+        e = hipMemcpy(p->d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess && count) e = hipMemcpy(p->d_aoff, ao.data(), count * sizeof(int64_t), hipMemcpyHostToDevice);
     if (e == hipSuccess && count) e = hipMemcpy(p->d_boff, bo.data(), count * sizeof(int64_t), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -731,10 +740,10 @@ int mi_batch_destroy(mi_batch_t *p)
 {
     if (!p) return 0;
     batch_drop_graph(p);
+    if (p->t2) (void)hipEventDestroy(p->t2);
     (void)hipFree(p->d_n);
     (void)hipFree(p->d_order);
     (void)hipFree(p->d_info);
-    (void)hipFree(p->d_counter);
     (void)hipFree(p->d_aoff);
     (void)hipFree(p->d_boff);
     delete p;

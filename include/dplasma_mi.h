@@ -310,8 +310,9 @@ int mi_sgp_nll_grad(mi_ctx_t *ctx, int N, int NB, const float *dT, const float *
  * element offset sum_{j<i} n_j^2 of dA; its right-hand side at offset
  * sum_{j<i} n_j of dB (dB may be NULL: factor only).  One persistent launch
  * per size class (above 128, at most 128, at most 64) works through the
- * batch; with use_graph the launches are captured in a
- * hipGraph on the first call for given (dA, dB) and replayed after. */
+ * batch, the classes side by side; with use_graph that of the largest class is
+ * captured in a hipGraph on the first call for given (dA, dB) and replayed
+ * after. */
 typedef struct mi_batch_s mi_batch_t;
 /* n[i] = lo + (splitmix64 word i of seed) mod (hi - lo + 1) */
 int mi_batch_sizes(uint64_t seed, int count, int lo, int hi, int *n);
