@@ -179,6 +179,8 @@ int spotrf_tiles_split(Ctx *c, int N, int NB, float *dT, int *info, bool bf16_sp
 // Factorization (mi_dpotrf_tiles / mi_spotrf_tiles) enqueued only, both
 // streams joined into s_main; its info is left in d_info[0].
 template <class T> int potrf_enqueue(Ctx *c, int N, int NB, T *dT);
+// Whether it takes tiles of NB: 0, or its error
+template <class T> int potrf_check(int NB);
 // Column-major array <-> packed lower tile image (mi_lapack.hip), enqueued.
 template <class E>
 int sym_stage_enqueue(Ctx *c, hipStream_t st, bool to_image, int uplo, int N, int NB, E *dT, E *dA, int lda);

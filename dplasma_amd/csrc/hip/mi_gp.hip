@@ -128,7 +128,7 @@ int gp_nll(mi_ctx_t *c, int N, int NB, const T *dK, int ldk, T *dT, T *dy, doubl
 {
     *info = 0;
     int rc = check("mi_gp_nll", N, NB, ldk), h_info = 0;
-    if (rc) return rc;
+    if (rc || (rc = potrf_check<T>(NB))) return rc;      // before anything is written
     rc = enqueue_nll<T>(c, N, NB, dK, ldk, dT, dy, dout, &h_info);
     // the wait comes first also after an error: the caller may free its arrays
     const int rs = mi_synchronize(c);

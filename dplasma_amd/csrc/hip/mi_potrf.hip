@@ -1531,6 +1531,16 @@ int task_update_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, in
 }
 size_t task_winv_elems(int NB) { return potrf_ws_elems(NB) / 2; }
 
+template <> int potrf_check<double>(int NB)
+{
+    const int hmb = half_tile_hmb(NB);
+    return check_diag<double>(hmb > 0 ? hmb : NB);
+}
+template <> int potrf_check<float>(int NB)
+{
+    const int hmb = g_supdate == 1 ? half_tile_hmb(NB) : 0;
+    return check_diag<float>(hmb > 0 ? hmb : NB);
+}
 template <> int potrf_enqueue<double>(Ctx *c, int N, int NB, double *dT)
 {
     int info;

@@ -288,7 +288,9 @@ int mi_dpotri_tiles(mi_ctx_t *ctx, int N, int NB, double *dT, int *info);
  * triangle is read): dT receives the factor (MT(MT+1)/2 tiles), dy (N values,
  * y on entry) a = L^-1 y, dout[0..1] sum log L_ii and a^T a in FP64, so that
  * nll = dout[1] / 2 + dout[0] + N/2 log 2 pi.  *info as mi_dpotrf_tiles (then
- * the outputs are not valid).  NB a multiple of 32, at most 960.  Blocking. */
+ * the outputs are not valid).  NB a multiple of 32, at most 960 (else -2), that
+ * mi_{d,s}potrf_tiles takes: in FP64 above 560 a multiple of 64 (else -4).
+ * Blocking. */
 int mi_dgp_nll(mi_ctx_t *ctx, int N, int NB, const double *dK, int ldk, double *dT, double *dy, double *dout,
                int *info);
 int mi_sgp_nll(mi_ctx_t *ctx, int N, int NB, const float *dK, int ldk, float *dT, float *dy, double *dout, int *info);
