@@ -21,6 +21,7 @@
 // A_mn^T X_m on FP64 MFMA into per-tile partials, and a second pass sums the
 // partials of each row in a fixed order.  Other tiles use a strip kernel
 // that reads every element twice (once per side of the diagonal).
+#include <algorithm>
 #include <cfloat>
 #include <chrono>
 #include <cmath>
@@ -871,15 +872,31 @@ int dsymm_resid(Ctx *c, hipStream_t s, int N, int NB, const double *dA, int NRHS
     if (NB >= 64 && NB <= 512 && NB % 2 == 0) {
         const int64_t ntile = (int64_t)MT * (MT + 1) / 2;
         const bool lds_chunks = NB % 128 == 0 && g_symm_kernel;
-        // shares of a tile: as many as bring the workgroups to about two a
-        // CU (one or three: within 1% of the solve of 3200), at most one a
-        // chunk (LDS chunks: two)
-        const int S = (int)std::min<int64_t>(lds_chunks ? NB / 32 : (NB + 31) / 32,
-                                             std::max<int64_t>(1, 512 / ntile));
-        double *P = (double *)ws_get(c, WS_MX_PART, (size_t)(ntile * sy_part(S) * NB) * sizeof(double));
+        const int most = lds_chunks ? NB / 32 : (NB + 31) / 32;   // one a chunk (LDS chunks: two)
+        // Shares of a tile.  Up to four right-hand sides as many as bring the
+        // workgroups to about two a CU (one or three: within 1% of the solve
+        // of 3200).  With more the sum of the partials, which fewer lanes
+        // share, costs as much as the products: the least estimated time, us,
+        // of a CU's tiles and of the sum (N = 4096, NB = 256, 16 right-hand
+        // sides: 63 us unshared, 81 with three; N = 3200, NB = 320: 133, and
+        // 79 with four).
+        auto shares = [&](int nr) -> int {
+            if (nr <= 4) return (int)std::min<int64_t>(most, std::max<int64_t>(1, 512 / ntile));
+            const double tile = lds_chunks ? 5e-4 * NB * NB : 0.33 * NB, slots = lds_chunks ? 256.0 : 512.0;
+            const double sum = 1e-4 * ntile * NB + (nr <= 8 ? 0.3 : 0.6) * MT;
+            double best = 1e300;
+            int bs = 1;
+            for (int S = 1; S <= most && (S == 1 || ntile * S <= 1024); S++) {
+                const double t = ceil(ntile * S / slots) / S * tile + S * sum + (S > 1 && nr > 8 ? 3.0 : 0.0);
+                if (t < best) { best = t; bs = S; }
+            }
+            return bs;
+        };
+        const int Smax = std::max(shares(std::min(NRHS, 16)), shares((NRHS - 1) % 16 + 1));
+        double *P = (double *)ws_get(c, WS_MX_PART, (size_t)(ntile * sy_part(Smax) * NB) * sizeof(double));
         if (!P) return -3;
         for (int j0 = 0; j0 < NRHS; j0 += 16) {
-            const int nr = NRHS - j0 < 16 ? NRHS - j0 : 16;
+            const int nr = NRHS - j0 < 16 ? NRHS - j0 : 16, S = shares(nr);
             double *ra = j0 == 0 ? rowabs : nullptr;
             const double *Xj = dX + (int64_t)j0 * ldx;
             if (lds_chunks) {
@@ -908,7 +925,8 @@ int dsymm_resid(Ctx *c, hipStream_t s, int N, int NB, const double *dA, int NRHS
             else
                 MI_LAUNCH(c, s, "dsymm_part", 2.0 * N * (double)N * nr, 8.0 * (double)ntile * NB * NB,
                           k_symm_part<false><<<(unsigned)(ntile * S), 256, 0, s>>>(dA, N, NB, MT, Xj, ldx, nr, P, S));
-            const int lp = nr <= 1 ? 16 : nr <= 2 ? 8 : nr <= 4 ? 4 : nr <= 8 ? 2 : 1;
+            // (one share, five to eight: the plain runs are as fast as two lanes)
+            const int lp = nr <= 1 ? 16 : nr <= 2 ? 8 : nr <= 4 ? 4 : nr <= 8 && S > 1 ? 2 : 1;
             MI_LAUNCH(c, s, "dsymm_sum", 0.0, 8.0 * (S + 1.0) * (double)ntile * 16 * NB,
                       k_symm_sum<<<(unsigned)(((int64_t)N * 16 + 255) / 256), 256, 0, s>>>(
                           P, N, NB, MT, dB + (int64_t)j0 * ldb, ldb, dR + (int64_t)j0 * ldr, ldr, nr, lp, ra, S));
