@@ -225,7 +225,7 @@ template <class T, int NW, int RT, bool MULTI> struct Batch {
             }
             const int f = diag_factor<T, NW, NW>(
                 A + (int64_t)p0 * n + p0, min(PW, n - p0), n, sh.ds, [&](int i, int j) { return limg(i, j); },
-                [&](int p) { return sh.w[p]; }, [](int, const V4 &) {}, [](int, int, const V4 &) {});
+                [&](int p) { return sh.w[p]; });
             if (f) return p0 + f;
             if constexpr (MULTI) {
                 int base = NW;

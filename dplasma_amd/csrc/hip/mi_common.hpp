@@ -58,20 +58,6 @@ template <> struct MF<float> {
     __device__ static inline int lane_of(int r) { return 16 * (r >> 2); }
 };
 
-// Wave-uniform copy of a value held by one lane (v_readlane_b32; two for a double).
-__device__ inline double readlane_d(double v, int lane)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ inline double readlane_t(double v, int lane) { return readlane_d(v, lane); }
-__device__ inline float readlane_t(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
 struct ProfRec {
     const char *name;
     hipEvent_t ev0, ev1;
@@ -91,8 +77,8 @@ struct ProfAgg {
 // Device workspaces owned by a context: grown on demand (ws_get), freed with
 // the context, so that calls on different contexts never share memory.
 enum WsId {
-    WS_POTRF_WINV = 0,  // diagonal-block inverses handed from POTRF(k) to TRSM(k)
-    WS_TRSM,            // solve: 32x32 and 128x128 block inverses, link matrices
+    WS_POTRF_WINV = 0,  // operand images handed from POTRF(k) to TRSM(k)
+    WS_TRSM,            // solve: 128x128 block inverses and link matrices, or 32x32 block inverses
     WS_MX_L32,          // mixed solve: FP32 tiles
     WS_MX_R32,          //   FP32 right-hand sides / corrections
     WS_MX_R64,          //   FP64 residual, norms, row sums
@@ -104,7 +90,6 @@ enum WsId {
     WS_ADJ_JOBS,        //   job table
     WS_ADJ_SEGS,        //   segment table
     WS_POTRI,           // inverse: the seed / result image
-    WS_DTD,             // task-insertion front-end: per-task diagonal-block inverses
     WS_BF16_PANEL,      // BF16-split FP32 factor: hi/lo images of one panel column
     WS_COUNT
 };
@@ -152,7 +137,8 @@ void prof_begin(Ctx *c, hipStream_t s, const char *name, double flops, double by
 void prof_end(Ctx *c, hipStream_t s, ProfRec *r);
 
 // Tile triangular solves (mi_solve.hip), enqueue only: trsm_prepare writes
-// the 32x32 diagonal-block inverses of L (trsm_ws_elems(N, NB) elements),
+// the block inverses and link matrices of the wavefront solve, or the 32x32
+// diagonal-block inverses of the per-tile one (trsm_ws_elems(N, NB) elements),
 // trsm_enqueue applies op(L)^{-1} (trans 111 / 112) to NRHS columns.
 size_t trsm_ws_elems(int N, int NB);
 template <class T> int trsm_prepare(Ctx *c, hipStream_t s, int unit, int N, int NB, const T *dT, T *W);
@@ -191,9 +177,8 @@ template <class T> int adjoint_enqueue(Ctx *c, int N, int NB, const T *dL, T *dG
 // the fixed scratch of mi_dpotrf_tiles_noalloc (mi_potrf.hip).
 void noalloc_setup(int device);
 // Single-tile tasks of the tile Cholesky on the packed lower FP64 image,
-// enqueued on s (mi_potrf.hip): POTRF(k) writes the inverses of its 32 x 32
-// diagonal blocks to Winv (task_winv_elems(NB) elements), which TRSM(m, k)
-// reads; update: A(m, n) -= A(m, k) A(n, k)^T, SYRK when m == n.
+// enqueued on s (mi_potrf.hip): POTRF(k) leaves its operand images in Winv
+// (task_winv_elems(NB) elements), which TRSM(m, k) reads; update: A(m, n) -= A(m, k) A(n, k)^T, SYRK when m == n.
 int task_prepare_fp64(int NB);
 int task_potrf_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int k, double *Winv);
 int task_trsm_fp64(Ctx *c, hipStream_t s, double *dT, int N, int NB, int m, int k, double *Winv);

@@ -9,10 +9,9 @@
 //   read  tile t  -> after the last writer of t              (RAW)
 //   write tile t  -> after the last writer and every reader
 //                    of t since that write                   (WAW, WAR)
-// POTRF(k) also writes the inverses of its 32 x 32 diagonal blocks to a
-// slot of its own, which TRSM(m, k) reads (tracked like a tile).  The tile
-// kernels are the ones of the fused factorization (mi_potrf.hip), one tile
-// per launch.  Tasks of one stream run in insertion order, so same-stream
+// POTRF(k) also leaves its operand images in a slot of its own, which
+// TRSM(m, k) reads (tracked like a tile).  The tile kernels are the ones of
+// the fused factorization (mi_potrf.hip), one tile a task.  Tasks of one stream run in insertion order, so same-stream
 // dependencies need no event.
 #include <vector>
 #include "mi_common.hpp"
@@ -41,7 +40,7 @@ struct mi_dtd_s {
     size_t wsz = 0;
     hipStream_t st[DTD_STREAMS] = {};
     int rr = 0;
-    std::vector<TileState> tiles;      // packed lower tiles, then the MT inverse slots
+    std::vector<TileState> tiles;      // packed lower tiles, then the MT image slots
     std::vector<hipEvent_t> events;    // every event recorded (destroyed at wait)
     long ntask = 0;
 };
@@ -123,7 +122,7 @@ int mi_dtd_create(mi_ctx_t *c, int N, int NB, double *dT, mi_dtd_t **out)
     if (hipMalloc(&d->winv, d->wsz * d->MT * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         delete d;
-        set_error("dtd: out of device memory for the block inverses");
+        set_error("dtd: out of device memory for the operand images");
         return -3;
     }
     for (auto &s : d->st) {

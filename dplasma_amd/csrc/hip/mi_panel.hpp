@@ -2,7 +2,7 @@
 // src/zpotrf_L.jdf:91-343), factored in sub-columns of SB columns:
 //   k_diag_factor   one workgroup: the w x w diagonal block of sub-column j
 //   k_panel_solve   X = C L_jj^{-T} for every row below it, 16 rows a wave
-//   k_panel_update  the remaining columns of the tile column -= X X_k^T
+//   k_update_*      the remaining columns of the tile column -= X X_k^T
 // (mi_potrf.hip launches them).  Everything works on 16 x 16 blocks held in
 // the accumulator layout of the 16x16x4 MFMA fed (B, A): element q of lane
 // l = 16 fk + fr is C(row fr, column row(q, fk)).  The same registers are,
@@ -366,8 +366,7 @@ __device__ __forceinline__ void invert_rows(T *v, T *x, T rd, std::integer_seque
 // hand-offs.
 // xl(i, p): LDS image ([s][lane]) of -X(i, p), valid until step p + 1 is
 // over; wl(p): W_p in LDS, image column t at t DIAG_WP, valid as long (both
-// may keep all steps); out_w(p, W_p), out_x(i, p, -X(i, p)): called by the
-// wave that has the block.  Returns the 1-based column of the first pivot
+// may keep all steps).  Returns the 1-based column of the first pivot
 // that is not positive, or 0, to every wave (ds.fail is 0 on entry and
 // ordered before this by a barrier).
 constexpr int DIAG_WP = DB + 2;                             // distinct banks for the writer of W
@@ -377,9 +376,8 @@ template <class T> struct DiagLds {
     __align__(16) T dl[DB][DIAG_WP];                        // D, [row][column]
     int fail;
 };
-template <class T, int NW, int NBK, class XL, class WL, class OW, class OX>
-__device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, DiagLds<T> &ds, XL &&xl, WL &&wl, OW &&out_w,
-                                           OX &&out_x)
+template <class T, int NW, int NBK, class XL, class WL>
+__device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, DiagLds<T> &ds, XL &&xl, WL &&wl)
 {
     typedef typename MF<T>::v4 V4;
     // worker waves; of eight, wave 4 is none: it shares the SIMD of wave 0,
@@ -543,18 +541,10 @@ __device__ __forceinline__ int diag_factor(T *__restrict__ A, int n, int ld, Dia
             __syncthreads();
 #pragma unroll
             for (int u = 0; u < SLOTS; u++)
-                if (bj[u] == p && bi[u] > p + 1) {
-                    store(bi[u], p, blk[u]);
-                    out_x(bi[u], p, -blk[u]);
-                }
-            // what wave 0 left: L_pp, W_p and X(p + 1, p)
+                if (bj[u] == p && bi[u] > p + 1) store(bi[u], p, blk[u]);
+            // what wave 0 left: L_pp and X(p + 1, p)
             if (wave == (APART ? 4 : NK)) {
-                out_w(p, w);
-                if (p + 1 < nb) {
-                    const V4 mx = get(xl(p + 1, p));
-                    store(p + 1, p, -mx);
-                    out_x(p + 1, p, mx);
-                }
+                if (p + 1 < nb) store(p + 1, p, -get(xl(p + 1, p)));
                 const T root = root_of(ds.ll[p & 1][fr][fr], ds.ll[p & 1][fr][DB]);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {

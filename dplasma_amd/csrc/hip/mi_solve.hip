@@ -693,19 +693,15 @@ __global__ __launch_bounds__(PREP_NT, 2) void k_wave_prep(const T *__restrict__ 
     }
 }
 
-// Index mappings of the wavefront solve.  The NW waves of a workgroup own
-// 128 / NW rows each, as TPW = 8 / NW MFMA row tiles of 16 rows.  With two
-// tiles (NW = 4), MFMA row i (0..15) of tile t (0, 1) is row wv_row(t, i) of
-// the wave's rows: forward, two consecutive rows belong to one lane (2 i + t),
-// so that the column-major L operands load as pairs.  With one tile (NW = 8)
-// row i is row i.  Element kq (0..7) of lane group f (0..3) of a 32-column
-// slice of the contraction is column wv_k(kq, f) of it: backward, four
-// consecutive columns belong to one lane, so that the rows of L (the
-// columns of L^T) load as runs of four.
-template <bool TRANS, int TPW> __device__ inline int wv_row(int t, int i)
-{
-    return TPW == 1 ? i : (TRANS ? 16 * t + i : 2 * i + t);
-}
+// Index mappings of the wavefront solve.  The eight waves of a workgroup own
+// 16 rows each, one MFMA row tile; while they catch up with earlier blocks,
+// 32 rows a pair of waves, two tiles: MFMA row i (0..15) of tile t (0, 1) is
+// row wv_row(t, i) of them (forward, two consecutive rows belong to one lane,
+// so that the column-major L operands load as pairs).  Element kq (0..7) of
+// lane group f (0..3) of a 32-column slice of the contraction is column
+// wv_k(kq, f) of it: backward, four consecutive columns belong to one lane,
+// so that the rows of L (the columns of L^T) load as runs of four.
+template <bool TRANS> __device__ inline int wv_row(int t, int i) { return TRANS ? 16 * t + i : 2 * i + t; }
 template <bool TRANS> __device__ inline int wv_k(int kq, int f) { return TRANS ? 16 * (kq >> 2) + 4 * f + (kq & 3) : 4 * kq + f; }
 
 // Four consecutive elements from p (16-byte aligned): one 16-byte load in
@@ -739,19 +735,17 @@ template <class T, bool TRANS> __device__ inline int wv_xs(int R, int j)
 // into the abort word flags[1] and goes on with whatever it read; every other
 // wait ends as soon as it sees that word set, so the launch always drains and
 // the host reports the failure.
-template <class T, bool TRANS, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ Tt, int N, int NB, int MT,
-                                                         const T *__restrict__ W128, const T *__restrict__ Mlink,
-                                                         T *__restrict__ B, int ldb, int nr, T *__restrict__ xs,
-                                                         int *__restrict__ ticket, long long wait_ticks)
+template <class T, bool TRANS>
+__global__ __launch_bounds__(512, 1) void k_trsm_wave(const T *__restrict__ Tt, int N, int NB, int MT,
+                                                     const T *__restrict__ W128, const T *__restrict__ Mlink,
+                                                     T *__restrict__ B, int ldb, int nr, T *__restrict__ xs,
+                                                     int *__restrict__ ticket, long long wait_ticks)
 {
     typedef typename MF<T>::v4 V4;
     typedef typename MF<T>::v2 V2;
     typedef typename WvSent<T>::U U;
-    constexpr int NT = 64 * NW;                   // threads
-    constexpr int RW = WV_RB / NW;                // rows per wave
-    constexpr int TPW = RW / 16;                  // MFMA row tiles per wave
-    static_assert(TPW == 1 || TPW == 2, "16 or 32 rows per wave");
+    constexpr int NT = 512;                       // threads
+    constexpr int RW = 16;                        // rows per wave
     __shared__ T Ws[128 * WV_WS];    // a-operands of the diagonal product: Ws[k * WV_WS + i] = op(W)(i, k)
     __shared__ T Ys[128][17];
     __shared__ int s_g;
@@ -789,12 +783,11 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
     const int frc = min(fr, max(nr, 1) - 1);
     // Catch-up layout: wave (rg, kh) = (wave / 2, wave % 2) takes rows
     // [32 rg, 32 rg + 32) of the block (two MFMA row tiles, rows
-    // wv_row<TRANS, 2>) against one half of each earlier block's columns
+    // wv_row<TRANS>) against one half of each earlier block's columns
     // (slices hb = 2 kh, 2 kh + 1): two rows per lane give 16-byte loads of L
     // forward, and each wave reads only its half of X.  The two halves of y
     // meet in LDS before z = W_g y, which (like the link product and the
     // stores) uses the layout of RW rows per wave.
-    static_assert(NW == 8, "the catch-up layout pairs eight waves");
     const int rg = wave >> 1, kh = wave & 1;
     const int rc = r0 + 32 * rg;                 // catch-up rows of this wave
     V4 acc[2];
@@ -802,7 +795,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
     for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int row = rc + wv_row<TRANS, 2>(t, MF<T>::row(q, fk));
+            const int row = rc + wv_row<TRANS>(t, MF<T>::row(q, fk));
             const T v = B[(int64_t)frc * ldb + min(row, N - 1)];
             acc[t][q] = (kh == 0 && row < N && fr < nr) ? v : T(0);
         }
@@ -810,30 +803,21 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
     // a-operands of one other block h: op(L)(row rc + wv_row(t, fr), column
     // 32 (2 kh + hl) + wv_k(kq, fk) of the block) as la[hl][kq][t]
     T la[2][8][2];
-    // (the addresses are clamped into the matrix).  FP64 zeroes what lies
-    // outside the matrix as the values arrive; FP32, whose loads run two
-    // blocks ahead, leaves that to mask_a, once the values are needed.
-    constexpr bool MASK_AT_LOAD = false;
+    // (the addresses are clamped into the matrix; mask_a zeroes what lies
+    // outside it once the values are needed)
     auto load_a = [&](T (&la)[2][8][2], int h) {
 #pragma unroll
         for (int hl = 0; hl < 2; hl++) {
             const int c0 = h * WV_RB + 32 * (2 * kh + hl);
             const int cc = min(c0, N - 1) & ~31;     // a valid 32-aligned block when c0 >= N
             const int rr = min(rc, N - 1) & ~31;
-            auto put = [&](int kq, int t, T v) {
-                if (MASK_AT_LOAD) {
-                    const int kk = wv_k<TRANS>(kq, fk), row = rc + wv_row<TRANS, 2>(t, fr);
-                    v = (c0 < N && c0 + kk < N && row < N) ? v : T(0);
-                }
-                la[hl][kq][t] = v;
-            };
             if (!TRANS) {
                 const T *pA = sym_elem(Tt, MT, NB, rr, cc) + 2 * fr;
 #pragma unroll
                 for (int kq = 0; kq < 8; kq++) {
                     const V2 v = *(const V2 *)(pA + (int64_t)(4 * kq + fk) * NB);
-                    put(kq, 0, v.x);
-                    put(kq, 1, v.y);
+                    la[hl][kq][0] = v.x;
+                    la[hl][kq][1] = v.y;
                 }
             } else {
                 const T *pA = sym_elem(Tt, MT, NB, cc, rr) + 4 * fk;
@@ -844,7 +828,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
                         T v[4];
                         wv_load4(pA + (int64_t)(16 * t + fr) * NB + 16 * kg, v);
 #pragma unroll
-                        for (int e = 0; e < 4; e++) put(4 * kg + e, t, v[e]);
+                        for (int e = 0; e < 4; e++) la[hl][4 * kg + e][t] = v[e];
                     }
             }
         }
@@ -858,39 +842,29 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
             for (int kq = 0; kq < 8; kq++)
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
-                    const int kk = wv_k<TRANS>(kq, fk), row = rc + wv_row<TRANS, 2>(t, fr);
+                    const int kk = wv_k<TRANS>(kq, fk), row = rc + wv_row<TRANS>(t, fr);
                     if (!(c0 < N && c0 + kk < N && row < N)) la[hl][kq][t] = T(0);
                 }
         }
     };
-    // a-operands of the link matrix: M_g(RW w + wv_row(t, fr), 32 hb + wv_k(kq, fk)),
+    // a-operands of the link matrix: M_g(RW w + fr, 32 hb + wv_k(kq, fk)),
     // column-major forward, row-major backward
-    T lm[4][8][TPW];
+    T lm[4][8];
     auto load_m = [&]() {
         const T *Mg = Mlink + (int64_t)g * 16384;
 #pragma unroll
         for (int hb = 0; hb < 4; hb++) {
             if (!TRANS) {
 #pragma unroll
-                for (int kq = 0; kq < 8; kq++) {
-                    if constexpr (TPW == 2) {
-                        const V2 v = *(const V2 *)(Mg + (32 * hb + 4 * kq + fk) * 128 + RW * wave + 2 * fr);
-                        lm[hb][kq][0] = v.x;
-                        lm[hb][kq][1] = v.y;
-                    } else {
-                        lm[hb][kq][0] = Mg[(32 * hb + 4 * kq + fk) * 128 + RW * wave + fr];
-                    }
-                }
+                for (int kq = 0; kq < 8; kq++) lm[hb][kq] = Mg[(32 * hb + 4 * kq + fk) * 128 + RW * wave + fr];
             } else {
 #pragma unroll
-                for (int t = 0; t < TPW; t++)
+                for (int kg = 0; kg < 2; kg++) {
+                    T v[4];
+                    wv_load4(Mg + (RW * wave + fr) * 128 + 32 * hb + 16 * kg + 4 * fk, v);
 #pragma unroll
-                    for (int kg = 0; kg < 2; kg++) {
-                        T v[4];
-                        wv_load4(Mg + (RW * wave + 16 * t + fr) * 128 + 32 * hb + 16 * kg + 4 * fk, v);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) lm[hb][4 * kg + e][t] = v[e];
-                    }
+                    for (int e = 0; e < 4; e++) lm[hb][4 * kg + e] = v[e];
+                }
             }
         }
     };
@@ -1082,27 +1056,22 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) Ys[32 * rg + wv_row<TRANS, 2>(t, MF<T>::row(q, fk))][fr] = acc[t][q];
+            for (int q = 0; q < 4; q++) Ys[32 * rg + wv_row<TRANS>(t, MF<T>::row(q, fk))][fr] = acc[t][q];
     __syncthreads();
     if (kh == 0)
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                T &y = Ys[32 * rg + wv_row<TRANS, 2>(t, MF<T>::row(q, fk))][fr];
+                T &y = Ys[32 * rg + wv_row<TRANS>(t, MF<T>::row(q, fk))][fr];
                 y = acc[t][q] + y;
             }
     __syncthreads();
-    V4 x[TPW];
-#pragma unroll
-    for (int t = 0; t < TPW; t++) x[t] = V4{T(0), T(0), T(0), T(0)};
+    V4 x = {T(0), T(0), T(0), T(0)};
 #pragma unroll 8
     for (int kq = 0; kq < 32; kq++) {
         const int kk = 4 * kq + fk;
-        const T b = Ys[kk][fr];
-#pragma unroll
-        for (int t = 0; t < TPW; t++)
-            x[t] = MF<T>::mfma(Ws[kk * WV_WS + RW * wave + wv_row<TRANS, TPW>(t, fr)], b, x[t]);
+        x = MF<T>::mfma(Ws[kk * WV_WS + RW * wave + fr], Ys[kk][fr], x);
     }
     // x_g = z - M_g X(last block)
     if (nprev > 0 && rw < N) {
@@ -1111,19 +1080,15 @@ __global__ __launch_bounds__(64 * NW, 1) void k_trsm_wave(const T *__restrict__ 
 #pragma unroll
         for (int hb = 0; hb < 4; hb++)
 #pragma unroll
-            for (int kq = 0; kq < 8; kq++)
-#pragma unroll
-                for (int t = 0; t < TPW; t++) x[t] = MF<T>::mfma(lm[hb][kq][t], bx[hb][kq], x[t]);
+            for (int kq = 0; kq < 8; kq++) x = MF<T>::mfma(lm[hb][kq], bx[hb][kq], x);
     }
     T *xg = xs + (int64_t)g * (WV_RB * RHSB);
 #pragma unroll
-    for (int t = 0; t < TPW; t++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int rb = RW * wave + wv_row<TRANS, TPW>(t, MF<T>::row(q, fk));
-            wv_store(xg + wv_xs<T, TRANS>(rb, fr), x[t][q]);
-            if (r0 + rb < N && fr < nr) B[(int64_t)fr * ldb + r0 + rb] = x[t][q];
-        }
+    for (int q = 0; q < 4; q++) {
+        const int rb = RW * wave + MF<T>::row(q, fk);
+        wv_store(xg + wv_xs<T, TRANS>(rb, fr), x[q]);
+        if (r0 + rb < N && fr < nr) B[(int64_t)fr * ldb + r0 + rb] = x[q];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1742,7 +1707,7 @@ int trsm_enqueue(Ctx *c, hipStream_t s, int trans, int N, int NB, const T *dT, c
             if (nr == 1) rc = fwd ? launch(k_trsm_vec<T, false, 1>) : launch(k_trsm_vec<T, true, 1>);
             else if (nr == 2) rc = fwd ? launch(k_trsm_vec<T, false, 2>) : launch(k_trsm_vec<T, true, 2>);
             else if (nr <= 4) rc = fwd ? launch(k_trsm_vec<T, false, 4>) : launch(k_trsm_vec<T, true, 4>);
-            else rc = fwd ? launch(k_trsm_wave<T, false, 8>) : launch(k_trsm_wave<T, true, 8>);
+            else rc = fwd ? launch(k_trsm_wave<T, false>) : launch(k_trsm_wave<T, true>);
             if (rc) return rc;
         }
         return 0;
