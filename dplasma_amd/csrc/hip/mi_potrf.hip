@@ -1135,11 +1135,15 @@ int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, dou
     typedef typename UpdShapes<T>::small Small;
     typedef typename UpdShapes<T>::tiny Tiny;
     constexpr int occ = UpdShapes<T>::occ;
-    // a launch of fewer than two 128 x 128 blocks per CU leaves the chip
+    // A launch of fewer than two 128 x 128 blocks per CU leaves the chip
     // idle: 64 x 64 blocks give four times the workgroups at a quarter of
-    // the chain
+    // the chain.  Where 128 does not divide the tile, blocks of 128 work for
+    // padding, and their ragged parts are the slow ones (step-0 update of N =
+    // 16000, us, 128 / 64: FP64 NB = 320 1798 / 1254, 192 1530 / 868, 336 1734
+    // / 1696; FP32 NB = 64 1712 / 306, 160 1422 / 623, 240 924 / 698; where it
+    // does, NB = 256 992 / 1020 and 563 / 593).
     int64_t g = grid(Big::BM);
-    const bool big = g >= 512 && update_lds_ok<Big>(dT, u.NB, K);
+    const bool big = g >= 512 && u.NB % Big::BM == 0 && update_lds_ok<Big>(dT, u.NB, K);
     if (!big) g = grid(Small::BM);
     const bool few = !big && g <= TINY_BLOCKS;
     const bool tiny = few && update_lds_ok<Tiny>(dT, u.NB, K), small = !tiny && update_lds_ok<Small>(dT, u.NB, K);
