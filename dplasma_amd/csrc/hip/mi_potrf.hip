@@ -1145,8 +1145,17 @@ int launch_update_blocks(Ctx *c, hipStream_t s, const char *name, double fl, dou
     int64_t g = grid(Big::BM);
     const bool big = g >= 512 && u.NB % Big::BM == 0 && update_lds_ok<Big>(dT, u.NB, K);
     if (!big) g = grid(Small::BM);
-    const bool few = !big && g <= TINY_BLOCKS;
-    const bool tiny = few && update_lds_ok<Tiny>(dT, u.NB, K), small = !tiny && update_lds_ok<Small>(dT, u.NB, K);
+    // Tiles of 65 .. 127: most of a tile is ragged blocks of 64, the slow ones
+    // through LDS, so through registers, in blocks of 32 where those pad less
+    // (up to 96), but for few blocks of a tile that 32 divides (step-0 update of
+    // N = 16000, us, LDS blocks of 64 / this: FP64 NB = 80 1690 / 1099, 96 1370 /
+    // 982, 112 1072 / 1064; FP32 770 / 787, 608 / 600, 522 / 537.  dpotrf, ms:
+    // 113.4 / 74.6, 73.3 / 52.0, 55.6 / 50.7; spotrf 52.4 / 52.1, 36.3 / 34.7,
+    // 28.7 / 28.5).
+    const bool ragged = u.NB > 64 && u.NB < 128;
+    const bool few = !big && (g <= TINY_BLOCKS || (ragged && u.NB <= 96));
+    const bool tiny = few && g <= TINY_BLOCKS && (!ragged || u.NB % 32 == 0) && update_lds_ok<Tiny>(dT, u.NB, K);
+    const bool small = !tiny && !ragged && update_lds_ok<Small>(dT, u.NB, K);
     if (tiny || (few && !small)) g = grid(32);
     if (g > 0x7fffffff) { set_error("update grid too large"); return -3; }
     if (g <= 0) return 0;

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
-@pytest.mark.parametrize("N,NB,block", [(600, 160, 32), (250, 64, 32), (1100, 96, 64), (1800, 192, 64), (1700, 320, 64),
+@pytest.mark.parametrize("N,NB,block", [(600, 160, 32), (250, 64, 32), (1500, 128, 64), (1800, 192, 64), (1700, 320, 64),
                                         (5000, 512, 128), (4500, 384, 128)])
 def test_update_blocks(dev, N, NB, block, dtype):
     print(f"update N={N} NB={NB} blocks of {block} {dtype.__name__}", flush=True)
