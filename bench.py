@@ -14,11 +14,11 @@ for kappa in {1e2, 1e5, 1e8} against the FP64 GPU dpotrf + dpotrs of the same
 system (time, refinement steps, backward error, error vs the FP64 answer),
 the adjoint of the factorization (df/dA from a given df/dL) at the same
 size, the batched uneven Cholesky + solve (4096 matrices of orders 32..1024,
-FP64 and FP32, one hipGraph-replayed persistent launch against a launch per
-matrix), the differentiated Gaussian-process likelihood (N = 8192, FP64 and
-FP32, plus 64 GPs of 1024 points), the roofline of the dominant kernel (the
-trailing update, timed with HIP events on its own stream in a separate
-profiled step) and the CPU baseline:
+FP64 and FP32, one persistent launch per size class, the largest class
+replayed from a hipGraph, against a launch per matrix), the differentiated
+Gaussian-process likelihood (N = 8192, FP64 and FP32, plus 64 GPs of 1024
+points), the roofline of the dominant kernel (the trailing update, timed with
+HIP events on its own stream in a separate profiled step) and the CPU baseline:
 the oracle's tile-DAG executor (a restatement of src/zpotrf_L.jdf with
 OpenBLAS tile kernels) on the host cores, on a bounded sample.  When that
 sample is the full N = 32768 workload, its factor is compared element by
@@ -417,10 +417,10 @@ def batched_leg(dp, count=4096, lo=32, hi=1024, seed=11):
     """Batched uneven Cholesky + solve: `count` SPD matrices with orders
     uniform in [lo, hi] (splitmix64, seed 11), A_i = G_i^T G_i / n_i + I with
     G_i Gaussian, b uniform in [-0.5, 0.5], NRHS = 1.  FP64 and FP32 (the FP64
-    batch rounded), each as one persistent launch replayed from a hipGraph
-    with the tile shape the autotuner picked, against the same kernel
-    launched once per matrix (FP64).  Flops: LAWN-41 dpotrf + dpotrs counts
-    summed over the batch.  Backward errors of 8 matrices checked on the host."""
+    batch rounded), each as one persistent launch per size class (the largest
+    replayed from a hipGraph) in the shape the autotuner picked, against the
+    same kernel launched once per matrix (FP64).  Flops: LAWN-41 dpotrf +
+    dpotrs counts summed over the batch.  Backward errors of 8 matrices checked on the host."""
     import ctypes
     import numpy as np
     mi, _ = dp.libs()

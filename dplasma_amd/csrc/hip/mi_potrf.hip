@@ -279,8 +279,8 @@ __device__ inline void decode_block(int L, int nsub, int n_begin, int m_off, int
 // loaded with the first of them and waits in registers.  PAIR: even NB and
 // aligned pairs of rows, two a load.
 // dpotrf N = 378, NB = 93: 13.2 us a launch with masked loads one stage ahead
-// and C loaded at the end, 9.5 us now; N = 3900, NB = 367 2.09 -> 1.81 ms in
-// FP64, 1.66 -> 1.31 ms in FP32.
+// and C loaded at the end, 9.5 us with this (6.4 in blocks of 32); N = 3900, NB =
+// 367 2.09 -> 1.83 ms in FP64, 1.66 -> 1.33 ms in FP32.
 //
 // The products add up from zero and meet C once: as the MFMAs' start, C would
 // round at its own size every four columns (factor of N = 513, NB = 130 with a
@@ -514,8 +514,8 @@ template <> struct UpdShapes<float> {
 //     al bh + ah bl + ah bh            (the al bl term, ~2^-16 relative, dropped)
 // so the update carries about 16 significant bits per operand instead of 8,
 // at three BF16 MFMAs per product.  Used by the mixed-precision solve, whose
-// FP64 refinement recovers the rest.  Work decomposition, XCD grouping,
-// SYRK masking and C as the MFMAs' start as k_update_mfma; K in chunks of
+// FP64 refinement recovers the rest.  Work decomposition, XCD grouping
+// and SYRK masking as k_update_mfma, C as the MFMAs' start; K in chunks of
 // 32, split once per workgroup while staged into LDS as [row][k] bf16 rows
 // (row pitch 40 bf16 = 80 B: 16-byte aligned fragment reads, spread banks).
 // MFMA operand layout: A(i, k) and B(k, j) for lane l in i (resp. j) = l % 16,
